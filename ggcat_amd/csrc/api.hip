@@ -59,7 +59,7 @@ struct ggcat_gpu_ctx {
         unit_dcount, unit_dregion, unit_skmers;  // per unit after deduplication
     // merge buffers
     DevBuf items, n_items, work, parts, redo, redo_count, out_key, out_val, out_sub, chunk_cursor, chunk_fill_dev,
-        fix_key, fix_val, fix_sub, fix_cursor, out_colors, fix_colors;
+        chunk_off, fix_key, fix_val, fix_sub, fix_cursor, out_colors, fix_colors;
     // state
     ggcat_gpu_params P{};
     bool have_records = false, have_solid = false;
@@ -70,10 +70,8 @@ struct ggcat_gpu_ctx {
     uint32_t dd_max = 0;  // the compaction deduplicated the units of up to this many records
     bool resplit_done = false;  // the arena holds resplit buckets (ggcat_gpu_resplit_outliers)
     uint64_t n_spill = 0;  // records of the last bucketing past their unit's region
-    uint32_t n_chunks_used = 0;  // output chunks of the last merge
     uint32_t n_passes = 0;  // kernel passes of the last merge
-    std::vector<uint32_t> chunk_fill;  // host copy of their fill counts
-    uint64_t n_tail = 0;  // entries appended after the chunks (combined fixups)
+    DevBuf copy_mult, copy_flags;  // multiplicities and flags on their way to the host
     bool colored = false;
     uint32_t color_words = 0;  // bitmap words per solid entry of a colored build
     double ms[9] = {0};
@@ -114,7 +112,7 @@ struct ggcat_gpu_ctx {
     // color subsets of the solid table: ids for the color map and the colored
     // FASTA headers (assigned on first use after a merge)
     bool have_subsets = false;
-    std::vector<uint32_t> pos_subset;  // per table position, ~0u for an empty position
+    std::vector<uint32_t> pos_subset;  // per table position
     std::vector<std::vector<uint32_t>> subsets;
 };
 
@@ -455,7 +453,7 @@ void ggcat_gpu_destroy(ggcat_gpu_ctx* ctx) {
                       &ctx->unit_dcount, &ctx->unit_dregion, &ctx->unit_skmers,
                       &ctx->slot_color, &ctx->color_starts, &ctx->colors, &ctx->error_flag, &ctx->items,
                       &ctx->n_items, &ctx->work, &ctx->parts, &ctx->redo, &ctx->redo_count, &ctx->out_key,
-                      &ctx->out_val, &ctx->out_sub, &ctx->chunk_cursor, &ctx->chunk_fill_dev, &ctx->fix_key,
+                      &ctx->out_val, &ctx->out_sub, &ctx->chunk_cursor, &ctx->chunk_fill_dev, &ctx->chunk_off, &ctx->fix_key,
                       &ctx->fix_val, &ctx->fix_sub, &ctx->fix_cursor, &ctx->out_colors, &ctx->fix_colors,
                       &ctx->idx_key, &ctx->idx_pos, &ctx->idx_boff, &ctx->idx_bcount, &ctx->idx_bcursor,
                       &ctx->q_seq, &ctx->q_off, &ctx->q_matched, &ctx->q_counts, &ctx->q_work,
@@ -464,7 +462,8 @@ void ggcat_gpu_destroy(ggcat_gpu_ctx* ctx) {
                       &ctx->u_rest_n, &ctx->u_rep, &ctx->u_tab, &ctx->u_path, &ctx->stage_slots, &ctx->stage_unit,
                       &ctx->stage_rank, &ctx->stage_color, &ctx->stage_cursor, &ctx->defer, &ctx->defer_count,
                       &ctx->kmer_total, &ctx->spill_slots, &ctx->spill_color, &ctx->raw, &ctx->p_stats,
-                      &ctx->p_carry, &ctx->p_keep, &ctx->p_keep_off, &ctx->p_flags, &ctx->p_bits, &ctx->rk_pos};
+                      &ctx->p_carry, &ctx->p_keep, &ctx->p_keep_off, &ctx->p_flags, &ctx->p_bits, &ctx->rk_pos,
+                      &ctx->copy_mult, &ctx->copy_flags};
     if (ctx->pin_ring) (void)hipHostFree(ctx->pin_ring);
     if (ctx->server) (void)ggcat_gpu_serve_close(ctx);
     if (ctx->graph_a) (void)hipGraphExecDestroy(ctx->graph_a);
@@ -1590,14 +1589,21 @@ int ggcat_gpu_kmers_merge(ggcat_gpu_ctx* ctx) {
             fix_cap = std::max(fix_cap, n_fix + 1024);
             continue;
         }
-        ctx->chunk_fill.resize(used_chunks);
-        if (used_chunks)
-            HIPCHK(hipMemcpy(ctx->chunk_fill.data(), ctx->chunk_fill_dev.p, (size_t)used_chunks * 4, hipMemcpyDeviceToHost));
-        uint64_t n_out = 0;
-        for (uint32_t f : ctx->chunk_fill) n_out += f;
-        // combined fixups are appended after the last used chunk
-        const uint64_t tail0 = (uint64_t)used_chunks * OUT_CHUNK;
-        uint64_t n_add = 0;
+        // the partly filled chunks' entries close up; combined fixups are
+        // appended behind the dense table
+        uint64_t tail0 = 0;
+        if (used_chunks) {
+            ENSURE(ctx->chunk_off, ((size_t)used_chunks + 1) * 8);
+            const int rs = device_scan(ctx, P_<uint32_t>(ctx->chunk_fill_dev), P_<uint64_t>(ctx->chunk_off), used_chunks);
+            if (rs != GGCAT_GPU_OK) return rs;
+            HIPCHK(hipMemcpyAsync(&tail0, P_<uint64_t>(ctx->chunk_off) + used_chunks, 8, hipMemcpyDeviceToHost, ctx->stream));
+            hipLaunchKernelGGL(out_close_holes_kernel, dim3(used_chunks), dim3(256), 0, ctx->stream,
+                               P_<uint64_t>(ctx->chunk_off), used_chunks, M.out_key, key_words, M.out_val, M.out_sub,
+                               M.out_colors, W);
+            HIPCHK(hipGetLastError());
+            HIPCHK(hipStreamSynchronize(ctx->stream));
+        }
+        uint64_t n_out = tail0, n_add = 0;
         // combine the two halves of cross-unit boundary k-mers
         if (n_fix) {
             const uint32_t kw = key_words;
@@ -1644,8 +1650,6 @@ int ggcat_gpu_kmers_merge(ggcat_gpu_ctx* ctx) {
                 HIPCHK(hipMemcpy(P_<uint32_t>(ctx->out_colors) + tail0 * W, oc.data(), n_add * 4 * W,
                                  hipMemcpyHostToDevice));
         }
-        ctx->n_chunks_used = used_chunks;
-        ctx->n_tail = n_add;
         n_out += n_add;
         ctx->n_fix = n_fix;
         ctx->n_solid = n_out;
@@ -1672,28 +1676,27 @@ int ggcat_gpu_solid_copy(ggcat_gpu_ctx* ctx, uint64_t* keys, uint32_t* multiplic
     if (!ctx->have_solid) return fail(ctx, GGCAT_GPU_ESTATE, "no merge result");
     HIPCHK(hipSetDevice(ctx->device));
     const uint32_t kw = ctx->key_words;
-    // the output is the valid prefix of every used chunk, then the tail of
-    // combined cross-unit entries
-    std::vector<std::pair<uint64_t, uint64_t>> runs;  // (first entry, count)
-    for (uint32_t c = 0; c < ctx->n_chunks_used; c++)
-        if (ctx->chunk_fill[c]) runs.emplace_back((uint64_t)c * OUT_CHUNK, ctx->chunk_fill[c]);
-    if (ctx->n_tail) runs.emplace_back((uint64_t)ctx->n_chunks_used * OUT_CHUNK, ctx->n_tail);
-    std::vector<uint32_t> v;
-    uint64_t o = 0;
-    for (auto& r : runs) {
-        if (keys)
-            HIPCHK(hipMemcpy(keys + o * kw, P_<uint64_t>(ctx->out_key) + r.first * kw, r.second * 8 * kw,
-                             hipMemcpyDeviceToHost));
-        if (sub) HIPCHK(hipMemcpy(sub + o, P_<uint32_t>(ctx->out_sub) + r.first, r.second * 4, hipMemcpyDeviceToHost));
-        if (multiplicity || flags) {
-            v.resize(r.second);
-            HIPCHK(hipMemcpy(v.data(), P_<uint32_t>(ctx->out_val) + r.first, r.second * 4, hipMemcpyDeviceToHost));
-            for (uint64_t i = 0; i < r.second; i++) {
-                if (multiplicity) multiplicity[o + i] = v[i] & 0x3FFFFFFFu;
-                if (flags) flags[o + i] = (uint8_t)(v[i] >> 30);
-            }
+    const uint64_t n = ctx->n_solid;
+    // a graph read from files has keys only
+    if (((multiplicity || flags) && ctx->out_val.cap < n * 4) || (sub && ctx->out_sub.cap < n * 4))
+        return fail(ctx, GGCAT_GPU_EHIP, "the table holds keys only");
+    if (n && keys) HIPCHK(hipMemcpy(keys, ctx->out_key.p, n * 8 * kw, hipMemcpyDeviceToHost));
+    if (n && sub) HIPCHK(hipMemcpy(sub, ctx->out_sub.p, n * 4, hipMemcpyDeviceToHost));
+    if (multiplicity || flags) {
+        // split on the device, a slice at a time
+        const uint64_t slice = std::min<uint64_t>(n, 1ull << 26);
+        ENSURE(ctx->copy_mult, slice * 4);
+        ENSURE(ctx->copy_flags, slice);
+        for (uint64_t o = 0; o < n; o += slice) {
+            const uint64_t c = std::min(slice, n - o);
+            const uint32_t grid = (uint32_t)std::min<uint64_t>((c + 255) / 256, (uint64_t)ctx->n_cu * 16);
+            hipLaunchKernelGGL(out_split_kernel, dim3(grid), dim3(256), 0, ctx->stream, P_<uint32_t>(ctx->out_val) + o, c,
+                               P_<uint32_t>(ctx->copy_mult), P_<uint8_t>(ctx->copy_flags));
+            HIPCHK(hipGetLastError());
+            HIPCHK(hipStreamSynchronize(ctx->stream));
+            if (multiplicity) HIPCHK(hipMemcpy(multiplicity + o, ctx->copy_mult.p, c * 4, hipMemcpyDeviceToHost));
+            if (flags) HIPCHK(hipMemcpy(flags + o, ctx->copy_flags.p, c, hipMemcpyDeviceToHost));
         }
-        o += r.second;
     }
     return GGCAT_GPU_OK;
 }
@@ -1706,17 +1709,7 @@ int ggcat_gpu_solid_colors(ggcat_gpu_ctx* ctx, uint32_t* color_words, uint32_t* 
     if (color_words) *color_words = W;
     if (!bitmaps) return GGCAT_GPU_OK;
     HIPCHK(hipSetDevice(ctx->device));
-    uint64_t o = 0;
-    auto copy = [&](uint64_t first, uint64_t count) -> int {
-        HIPCHK(hipMemcpy(bitmaps + o * W, P_<uint32_t>(ctx->out_colors) + first * W, count * 4 * W,
-                         hipMemcpyDeviceToHost));
-        o += count;
-        return GGCAT_GPU_OK;
-    };
-    for (uint32_t c = 0; c < ctx->n_chunks_used; c++)
-        if (ctx->chunk_fill[c] && copy((uint64_t)c * OUT_CHUNK, ctx->chunk_fill[c]) != GGCAT_GPU_OK) return GGCAT_GPU_EHIP;
-    if (ctx->n_tail && copy((uint64_t)ctx->n_chunks_used * OUT_CHUNK, ctx->n_tail) != GGCAT_GPU_OK)
-        return GGCAT_GPU_EHIP;
+    if (ctx->n_solid) HIPCHK(hipMemcpy(bitmaps, ctx->out_colors.p, ctx->n_solid * 4 * W, hipMemcpyDeviceToHost));
     return GGCAT_GPU_OK;
 }
 
@@ -2145,17 +2138,8 @@ int ggcat_gpu_index_build(ggcat_gpu_ctx* ctx) {
     ENSURE(ctx->idx_boff, ((size_t)nb + 1) * 8);
     ENSURE(ctx->idx_key, n * 8 * kw + 8);
     ENSURE(ctx->idx_pos, n * 4 + 4);
-    if (ctx->n_chunks_used) {
-        ENSURE(ctx->chunk_fill_dev, (size_t)ctx->n_chunks_used * 4);
-        HIPCHK(hipMemcpy(ctx->chunk_fill_dev.p, ctx->chunk_fill.data(), (size_t)ctx->n_chunks_used * 4,
-                         hipMemcpyHostToDevice));
-    }
     IndexArgs I{};
     I.out_key = P_<uint64_t>(ctx->out_key);
-    I.chunk_fill = P_<uint32_t>(ctx->chunk_fill_dev);
-    I.n_chunks = ctx->n_chunks_used;
-    I.n_tail = ctx->n_tail;
-    I.chunk = OUT_CHUNK;
     I.key_words = kw;
     I.log_buckets = L;
     I.bcount = P_<uint32_t>(ctx->idx_bcount);
@@ -2163,7 +2147,7 @@ int ggcat_gpu_index_build(ggcat_gpu_ctx* ctx) {
     I.bcursor = P_<uint32_t>(ctx->idx_bcursor);
     I.idx_key = P_<uint64_t>(ctx->idx_key);
     I.idx_pos = P_<uint32_t>(ctx->idx_pos);
-    const uint64_t n_pos = (uint64_t)ctx->n_chunks_used * OUT_CHUNK + ctx->n_tail;
+    const uint64_t n_pos = n;
     if (n_pos >= 0x7FFFFFFFull) return fail(ctx, GGCAT_GPU_EINVAL, "solid table too large for the query index");
     HIPCHK(hipMemsetAsync(ctx->idx_bcount.p, 0, (size_t)nb * 4, ctx->stream));
     HIPCHK(hipMemsetAsync(ctx->idx_bcursor.p, 0, (size_t)nb * 4, ctx->stream));
@@ -2382,7 +2366,7 @@ static int build_unitigs(ggcat_gpu_ctx* ctx, bool joined, uint64_t* n_unitigs, u
     if (ctx->P.hash_kind != GGCAT_GPU_HASH_SEQ)
         return fail(ctx, GGCAT_GPU_EINVAL, "unitig extension needs seq-hash keys (the k-mer is the key)");
     HIPCHK(hipSetDevice(ctx->device));
-    const uint64_t n_pos = (uint64_t)ctx->n_chunks_used * OUT_CHUNK + ctx->n_tail;
+    const uint64_t n_pos = ctx->n_solid;
     const uint64_t ne = 2 * n_pos;
     if (ne >= (uint64_t)NO_LINK) return fail(ctx, GGCAT_GPU_EINVAL, "solid table too large for unitig links");
     ENSURE(ctx->u_nb, ne * 4 + 8);
@@ -2403,10 +2387,6 @@ static int build_unitigs(ggcat_gpu_ctx* ctx, bool joined, uint64_t* n_unitigs, u
     U.out_key = P_<uint64_t>(ctx->out_key);
     U.out_val = P_<uint32_t>(ctx->out_val);
     U.out_sub = P_<uint32_t>(ctx->out_sub);
-    U.chunk_fill = P_<uint32_t>(ctx->chunk_fill_dev);
-    U.n_chunks = ctx->n_chunks_used;
-    U.n_tail = ctx->n_tail;
-    U.chunk = OUT_CHUNK;
     U.key_words = ctx->key_words;
     U.k = ctx->P.k;
     U.tab = P_<uint64_t>(ctx->u_tab);
@@ -2447,11 +2427,7 @@ static int build_unitigs(ggcat_gpu_ctx* ctx, bool joined, uint64_t* n_unitigs, u
     HIPCHK(hipStreamSynchronize(ctx->stream));
     // Paths cover every node unless there are cycles: only then are the path
     // nodes marked, so that the remaining ones can be collected.
-    uint64_t n_nodes = counts[1];
-    if (!joined) {
-        n_nodes = ctx->n_tail;
-        for (uint32_t c = 0; c < ctx->n_chunks_used; c++) n_nodes += ctx->chunk_fill[c];
-    }
+    const uint64_t n_nodes = joined ? counts[1] : n_pos;
     const bool cycles = tot_bytes - (uint64_t)ctx->P.k * tot_n != n_nodes;
     U.mark_visited = cycles ? 1u : 0u;
     ENSURE(ctx->u_seq, tot_bytes + 8);
@@ -2574,21 +2550,15 @@ static int ensure_subsets(ggcat_gpu_ctx* ctx) {
     if (!ctx->colored) return fail(ctx, GGCAT_GPU_ESTATE, "the last build was not colored");
     HIPCHK(hipSetDevice(ctx->device));
     const uint32_t W = ctx->color_words;
-    const uint64_t n_pos = (uint64_t)ctx->n_chunks_used * OUT_CHUNK + ctx->n_tail;
+    const uint64_t n_pos = ctx->n_solid;
     std::vector<uint32_t> bm(n_pos * W);
     if (n_pos) HIPCHK(hipMemcpy(bm.data(), ctx->out_colors.p, n_pos * W * 4, hipMemcpyDeviceToHost));
-    auto filled = [&](uint64_t p) {
-        const uint64_t c = p / OUT_CHUNK;
-        return c < ctx->n_chunks_used ? (p - c * OUT_CHUNK) < ctx->chunk_fill[c]
-                                      : p - (uint64_t)ctx->n_chunks_used * OUT_CHUNK < ctx->n_tail;
-    };
     auto less = [&](uint64_t a, uint64_t b) {
         return std::lexicographical_compare(&bm[a * W], &bm[a * W] + W, &bm[b * W], &bm[b * W] + W);
     };
     std::vector<std::pair<uint64_t, uint32_t>> hp;  // (hash of the bitmap, position)
     hp.reserve(n_pos);
     for (uint64_t p = 0; p < n_pos; p++) {
-        if (!filled(p)) continue;
         uint64_t h = 0x9E3779B97F4A7C15ULL;
         for (uint32_t w = 0; w < W; w++) h = (h ^ bm[p * W + w]) * 0xbf58476d1ce4e5b9ULL;
         hp.emplace_back(h ^ (h >> 31), (uint32_t)p);
@@ -2632,11 +2602,7 @@ int ggcat_gpu_color_subsets(ggcat_gpu_ctx* ctx, uint64_t* n_subsets, uint32_t* s
     const int r = ensure_subsets(ctx);
     if (r != GGCAT_GPU_OK) return r;
     if (n_subsets) *n_subsets = ctx->subsets.size();
-    if (subset_of_entry) {
-        uint64_t o = 0;
-        for (uint64_t p = 0; p < ctx->pos_subset.size(); p++)
-            if (ctx->pos_subset[p] != ~0u) subset_of_entry[o++] = ctx->pos_subset[p];
-    }
+    if (subset_of_entry) std::copy(ctx->pos_subset.begin(), ctx->pos_subset.end(), subset_of_entry);
     return GGCAT_GPU_OK;
 }
 
@@ -2898,16 +2864,7 @@ int ggcat_gpu_extension_copy(ggcat_gpu_ctx* ctx, uint8_t* ext) {
     if (!ctx || !ext) return GGCAT_GPU_EINVAL;
     if (!ctx->have_unitigs) return fail(ctx, GGCAT_GPU_ESTATE, "no unitig result");
     HIPCHK(hipSetDevice(ctx->device));
-    uint64_t o = 0;
-    for (uint32_t c = 0; c < ctx->n_chunks_used; c++) {
-        if (!ctx->chunk_fill[c]) continue;
-        HIPCHK(hipMemcpy(ext + o, P_<uint8_t>(ctx->u_ext) + (uint64_t)c * OUT_CHUNK, ctx->chunk_fill[c],
-                         hipMemcpyDeviceToHost));
-        o += ctx->chunk_fill[c];
-    }
-    if (ctx->n_tail)
-        HIPCHK(hipMemcpy(ext + o, P_<uint8_t>(ctx->u_ext) + (uint64_t)ctx->n_chunks_used * OUT_CHUNK, ctx->n_tail,
-                         hipMemcpyDeviceToHost));
+    if (ctx->u_npos) HIPCHK(hipMemcpy(ext, ctx->u_ext.p, ctx->u_npos, hipMemcpyDeviceToHost));
     return GGCAT_GPU_OK;
 }
 

@@ -29,10 +29,6 @@ GG_DEV uint64_t index_hash(uint64_t lo, uint64_t hi) { return mix64(lo ^ mix64(h
 
 struct IndexArgs {
     const uint64_t* out_key;  // solid keys, key_words per position
-    const uint32_t* chunk_fill;  // valid entries of each output chunk
-    uint32_t n_chunks;  // chunks before the tail
-    uint64_t n_tail;  // entries after the chunks
-    uint32_t chunk;  // entries per chunk
     uint32_t key_words;
     uint32_t log_buckets;
     uint32_t* bcount;
@@ -42,12 +38,6 @@ struct IndexArgs {
     uint32_t* idx_pos;
 };
 
-GG_DEV bool solid_valid(const IndexArgs& A, uint64_t p) {
-    const uint64_t c = p / A.chunk;
-    if (c < A.n_chunks) return (p - c * A.chunk) < A.chunk_fill[c];
-    return p - (uint64_t)A.n_chunks * A.chunk < A.n_tail;
-}
-
 GG_DEV uint32_t index_bucket(const IndexArgs& A, uint64_t p) {
     const uint64_t lo = A.out_key[p * A.key_words];
     const uint64_t hi = A.key_words == 2 ? A.out_key[p * 2 + 1] : 0;
@@ -56,12 +46,11 @@ GG_DEV uint32_t index_bucket(const IndexArgs& A, uint64_t p) {
 
 __global__ void index_count_kernel(IndexArgs A, uint64_t n_pos) {
     for (uint64_t p = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; p < n_pos; p += (uint64_t)gridDim.x * blockDim.x)
-        if (solid_valid(A, p)) atomicAdd(&A.bcount[index_bucket(A, p)], 1u);
+        atomicAdd(&A.bcount[index_bucket(A, p)], 1u);
 }
 
 __global__ void index_fill_kernel(IndexArgs A, uint64_t n_pos) {
     for (uint64_t p = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; p < n_pos; p += (uint64_t)gridDim.x * blockDim.x) {
-        if (!solid_valid(A, p)) continue;
         const uint32_t b = index_bucket(A, p);
         const uint64_t slot = A.boff[b] + atomicAdd(&A.bcursor[b], 1u);
         for (uint32_t q = 0; q < A.key_words; q++) A.idx_key[slot * A.key_words + q] = A.out_key[p * A.key_words + q];

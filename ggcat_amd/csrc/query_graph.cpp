@@ -317,17 +317,14 @@ extern "C" int ggcat_gpu_query_graph(ggcat_gpu_ctx* ctx, const char* input_graph
         }
     }
     const uint64_t n = keys.size() / kw;
-    // the graph k-mers become the context's table (every entry in the tail
-    // part; no chunks), then the device index and query path take over
+    // the graph k-mers become the context's table (keys and colors only), then
+    // the device index and query path take over
     HIPCHK(hipSetDevice(ctx->device));
     ENSURE(ctx->out_key, n * 8 * kw + 16);
     ENSURE(ctx->out_colors, (uint64_t)n * 4 * std::max<uint32_t>(W, 1) + 16);
     if (n) HIPCHK(hipMemcpy(ctx->out_key.p, keys.data(), n * 8 * kw, hipMemcpyHostToDevice));
     if (n && W) HIPCHK(hipMemcpy(ctx->out_colors.p, bitmaps.data(), (uint64_t)n * 4 * W, hipMemcpyHostToDevice));
     ctx->have_records = ctx->have_unitigs = ctx->have_subsets = ctx->have_index = false;
-    ctx->n_chunks_used = 0;
-    ctx->chunk_fill.clear();
-    ctx->n_tail = n;
     ctx->n_solid = n;
     ctx->key_words = kw;
     ctx->colored = colors != 0;

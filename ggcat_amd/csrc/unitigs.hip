@@ -36,10 +36,6 @@ struct UnitigArgs {
     const uint64_t* out_key;
     const uint32_t* out_val;
     const uint32_t* out_sub;
-    const uint32_t* chunk_fill;
-    uint32_t n_chunks;
-    uint64_t n_tail;
-    uint32_t chunk;
     uint32_t key_words;
     uint32_t k;
     uint64_t* tab;  // [tab_mask + 1] open addressing: hash bits 32-63 << 32 | (position + 1); 0 = empty
@@ -63,17 +59,8 @@ struct UnitigArgs {
                          // written order (unitig i's k-mers start at head_off - i * k)
 };
 
-// Position p holds a solid entry (chunks are filled from their start).
-GG_DEV bool slot_filled(const UnitigArgs& A, uint64_t p) {
-    const uint64_t c = p / A.chunk;
-    if (c < A.n_chunks) return (p - c * A.chunk) < A.chunk_fill[c];
-    return p - (uint64_t)A.n_chunks * A.chunk < A.n_tail;
-}
-
 // Position p is a node of the graph being compacted.
-GG_DEV bool unitig_valid(const UnitigArgs& A, uint64_t p) {
-    return slot_filled(A, p) && (!A.global || A.rep[p]);
-}
+GG_DEV bool unitig_valid(const UnitigArgs& A, uint64_t p) { return !A.global || A.rep[p]; }
 
 GG_DEV u128_t key_at(const UnitigArgs& A, uint64_t p) {
     const uint64_t lo = A.out_key[p * A.key_words];
@@ -100,12 +87,11 @@ GG_DEV bool side_flagged(const UnitigArgs& A, uint64_t p, uint32_t s) {
     return (fl == 1 && s == 0) || (fl == 2 && s == 1);
 }
 
-// Every filled position goes into the lookup table (linear probing; the
+// Every position goes into the lookup table (linear probing; the
 // table has at least twice as many slots as positions, so probing ends).
 __global__ void utab_insert_kernel(UnitigArgs A, uint64_t n_pos) {
     for (uint64_t p = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; p < n_pos;
          p += (uint64_t)gridDim.x * blockDim.x) {
-        if (!slot_filled(A, p)) continue;
         const u128_t c = key_at(A, p);
         const uint64_t h = index_hash((uint64_t)c, (uint64_t)(c >> 64));
         const uint64_t v = (h & 0xFFFFFFFF00000000ULL) | (p + 1);
@@ -135,13 +121,13 @@ GG_DEV uint32_t lookup_in_sub(const UnitigArgs& A, u128_t c, uint32_t sub) {
     return best;
 }
 
-// Joined mode: marks each filled position that is its key's smallest one.
+// Joined mode: marks each position that is its key's smallest one.
 // Counts them into *n_nodes (blocks of 256 threads: one atomic per block).
 __global__ __launch_bounds__(256) void rep_kernel(UnitigArgs A, uint64_t n_pos) {
     __shared__ unsigned int part[4];
     unsigned int cnt = 0;
     for (uint64_t p = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; p < n_pos; p += (uint64_t)gridDim.x * blockDim.x) {
-        const bool r = slot_filled(A, p) && lookup_in_sub(A, key_at(A, p), 0) == (uint32_t)p;
+        const bool r = lookup_in_sub(A, key_at(A, p), 0) == (uint32_t)p;
         A.rep[p] = r;
         cnt += r ? 1u : 0u;
     }
