@@ -190,7 +190,6 @@ void nthash_tables(uint32_t m, uint64_t* gtab) {
 
 u128_t mk128(uint64_t hi, uint64_t lo) { return ((u128_t)hi << 64) | lo; }
 
-const uint32_t TILE_T = 1024;
 // Colored merges keep one bit per color in each table entry.
 const uint32_t MAX_COLORS = 1024;
 
@@ -555,12 +554,20 @@ int ggcat_gpu_bucketing(ggcat_gpu_ctx* ctx, const uint8_t* data, uint64_t n_byte
         }
         if (!chunked) HIPCHK(hipMemcpy(ctx->input.p, data, n_bytes, hipMemcpyHostToDevice));
     }
-    // w == 16 forms window minima in registers; its tile of 960 windows (plus
-    // the w + 1 halo) is exactly 62 blocks of 16, one per lane.  It keeps the
-    // low 32 bits of each window minimum, which must name the unique bit,
-    // bucket, second bucket and unit.
-    const bool regs16 = (w == 16 && p.k <= 47 && 1 + p.buckets_log + p.second_buckets_log + xb <= 32);
-    const uint32_t T = regs16 ? 960 : TILE_T;
+    // The staging pass keeps the low 32 bits of each window minimum: they name
+    // the unique bit, bucket, second bucket and unit (1 + 13 + 8 + 10 bits at
+    // most).  w == 16 with windows of at most 47 bases has a variant of its
+    // own, whose tile of 960 windows (plus the w + 1 halo) is 62 blocks of 16,
+    // one per lane; every other w takes the block size tile_block(w).
+    const bool regs16 = tile_w16(w, p.k);
+    const uint32_t T = regs16 ? 960 : tile_windows(w);
+    void (*stage_kernel)(BucketArgs) = bucket_stage_kernel<2>;
+    switch (regs16 ? 0 : tile_block(w)) {
+        case 0: stage_kernel = bucket_stage_kernel<0>; break;
+        case 4: stage_kernel = bucket_stage_kernel<4>; break;
+        case 8: stage_kernel = bucket_stage_kernel<8>; break;
+        case 16: stage_kernel = bucket_stage_kernel<16>; break;
+    }
     const uint64_t n_tiles = (n_bytes + T - 1) / T;
     const uint64_t seg_words = n_tiles * T / 32 + 2;
     ENSURE(ctx->seg_bits, seg_words * 4);
@@ -608,7 +615,7 @@ int ggcat_gpu_bucketing(ggcat_gpu_ctx* ctx, const uint8_t* data, uint64_t n_byte
     A.n_colors = n_colors;
     A.error_flag = P_<uint32_t>(ctx->error_flag);
     nthash_tables(p.m, A.gtab);
-    const TileGeom G = tile_geom(T, w, p.k, p.m, regs16);
+    const TileGeom G = tile_geom(T, w, p.k, p.m);
     ENSURE(ctx->stage_cursor, 8);
     ENSURE(ctx->defer_count, 8);
     ENSURE(ctx->kmer_total, 16);  // k-mer occurrences, records
@@ -641,10 +648,7 @@ int ggcat_gpu_bucketing(ggcat_gpu_ctx* ctx, const uint8_t* data, uint64_t n_byte
         hipLaunchKernelGGL(fill32_kernel, dim3(256), dim3(256), 0, ctx->stream, A.seg_bits, 0u, (uint64_t)seg_words);
         hipLaunchKernelGGL(bucket_reset_kernel, dim3(1), dim3(64), 0, ctx->stream, A);
         if (n_tiles) {
-            if (regs16)
-                hipLaunchKernelGGL(bucket_stage_kernel<16>, dim3((uint32_t)n_tiles), dim3(64), G.bytes, ctx->stream, A);
-            else
-                hipLaunchKernelGGL(bucket_stage_kernel<0>, dim3((uint32_t)n_tiles), dim3(64), G.bytes, ctx->stream, A);
+            hipLaunchKernelGGL(stage_kernel, dim3((uint32_t)n_tiles), dim3(64), G.bytes, ctx->stream, A);
             hipLaunchKernelGGL(bucket_defer_kernel, dim3(small_grid), dim3(256), 0, ctx->stream, A);
         }
         hipLaunchKernelGGL(unit_split_kernel, dim3(std::min<uint32_t>((n_units + 255) / 256, 4096)), dim3(256), 0,
@@ -696,10 +700,7 @@ int ggcat_gpu_bucketing(ggcat_gpu_ctx* ctx, const uint8_t* data, uint64_t n_byte
             if (safe > tiles_done) {
                 A.tile0 = tiles_done;
                 const dim3 grid((uint32_t)(safe - tiles_done));
-                if (regs16)
-                    hipLaunchKernelGGL(bucket_stage_kernel<16>, grid, dim3(64), G.bytes, ctx->stream, A);
-                else
-                    hipLaunchKernelGGL(bucket_stage_kernel<0>, grid, dim3(64), G.bytes, ctx->stream, A);
+                hipLaunchKernelGGL(stage_kernel, grid, dim3(64), G.bytes, ctx->stream, A);
                 HIPCHK(hipGetLastError());
                 tiles_done = safe;
             }

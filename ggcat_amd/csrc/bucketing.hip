@@ -46,7 +46,7 @@ struct BucketArgs {
     uint32_t k, m, w;
     uint32_t b, sb, xb;
     uint32_t canonical;
-    uint32_t T;  // windows per tile (multiple of 64)
+    uint32_t T;  // windows per tile (multiple of 32)
     uint64_t n_tiles;
     uint64_t tile0;  // index of the launch's first tile (launches over part of the tiles)
     uint32_t* seg_bits;  // [ceil(n/32)+2] group-start bitmap (written by pass 1)
@@ -90,52 +90,61 @@ struct BucketArgs {
     uint64_t gtab[40];  // interleaved (fw, rc) rolling tables, index out*4+in
 };
 
+// m-mers of one tile: 16 per lane of its wavefront.
+constexpr uint32_t TILE_MMERS = 1024;
+
+// Windows computed before a tile's own ones: at least w (a unique minimizer's
+// group spans at most w windows), a multiple of the lanes' 16.
+__host__ __device__ inline uint32_t tile_halo(uint32_t w) { return (w + 15) / 16 * 16; }
+
+// Windows per tile: the tile's windows, its halo and the window behind them
+// take m-mers 0 .. halo + T + w - 1; whole 32-bit words of the bitmap.
+__host__ __device__ inline uint32_t tile_windows(uint32_t w) { return (TILE_MMERS - tile_halo(w) - w) / 32 * 32; }
+
+// Block of the window minima (see tile_minima): the largest power of two that
+// is at most min(w, 16).
+__host__ __device__ inline uint32_t tile_block(uint32_t w) { return w >= 16 ? 16 : w >= 8 ? 8 : w >= 4 ? 4 : 2; }
+
+// The w == 16 variant: its invalid-base slice of 64 bits covers the windows of
+// a lane for k <= 47.
+__host__ __device__ inline bool tile_w16(uint32_t w, uint32_t k) { return w == 16 && k <= 47; }
+
 // LDS layout of one tile (host and device agree through this struct).
 struct TileGeom {
-    uint32_t NW, NWB, NM, NB;
-    uint32_t off_mm, off_wv, off_wp, off_pk, off_inv, off_fwd, off_seg, off_ok, off_last, off_g;
+    uint32_t NW, NB;
+    uint32_t off_px, off_pn, off_wv, off_wp, off_pk, off_inv, off_fwd, off_seg, off_ok, off_last, off_g;
     uint32_t bytes;
 };
 
-// With `regs` the window minima are formed in registers and the per-m-mer
-// hash array is not needed.
-__host__ __device__ inline TileGeom tile_geom(uint32_t T, uint32_t w, uint32_t k, uint32_t m, bool regs) {
+// Per window the low 32 bits of its minimum (all a record needs: unique bit,
+// bucket, second bucket and unit bits) and the minimizer's offset in the
+// window as a byte, per m-mer its strand as a bit; each lane's 16 entries are
+// padded by one word so that lanes' accesses hit distinct LDS banks.  Other
+// than tile_w16 also passes prefix minima through LDS (64-bit values, 4-bit
+// positions), before the window minima are written over them.
+__host__ __device__ inline TileGeom tile_geom(uint32_t T, uint32_t w, uint32_t k, uint32_t m) {
     TileGeom g;
-    g.NW = T + w + 1;
-    g.NWB = (g.NW + w - 1) / w;
-    g.NM = (g.NWB + 1) * w;
+    g.NW = T + tile_halo(w) + 1;
     // bases relative to borg: d0 in [1,16]; the furthest read is the word
-    // after the one holding relative base d0 + max(NM+m-2, NW+k-2)
-    uint32_t need = 48 + (g.NM + m > g.NW + k ? g.NM + m : g.NW + k);
+    // after the one holding relative base d0 + max(TILE_MMERS+m-2, NW+k-2)
+    uint32_t need = 48 + (TILE_MMERS + m > g.NW + k ? TILE_MMERS + m : g.NW + k);
     g.NB = (need + 31) / 32 * 32;
     uint32_t o = 0;
     g.off_g = o; o += 40 * 8;
-    g.off_mm = o; o += regs ? 0 : g.NM * 8;
-    if (regs) {
-        // register path (w == 16): per window the low 32 bits of its minimum
-        // (all the record needs: unique bit, bucket, second bucket and unit
-        // bits) and the minimizer's offset in the window as a byte, per m-mer
-        // its strand as a bit; each lane's 16 windows padded by one word so
-        // that lanes' stores hit distinct LDS banks
-        g.off_wv = o; o += (g.NWB * 17 + 1) * 4;
-        o = (o + 7) / 8 * 8;
-    } else {
-        // wv / wp / fwd are padded after every 16 entries (Tile::WV, WP, FWD)
-        // so that lanes writing 16-window blocks hit distinct LDS banks
-        g.off_wv = o; o += (g.NWB * w + g.NWB * w / 16 + 1) * 8;
-    }
+    g.off_px = o;
+    g.off_wv = o;
+    g.off_wp = (o + 64 * 17 * 4 + 7) / 8 * 8;
+    const bool lds_prefixes = !tile_w16(w, k);
+    const uint32_t minima = g.off_wp + 64 * 20 + 4, prefixes = o + (lds_prefixes ? 64 * 17 * 8 : 0);
+    o = ((minima > prefixes ? minima : prefixes) + 7) / 8 * 8;
+    g.off_pn = o; o += lds_prefixes ? 64 * 8 : 0;
     g.off_pk = o; o += g.NB / 16 * 4;
-    g.off_inv = o; o += g.NB / 32 * 4;
+    g.off_inv = o; o += (g.NB / 32 + 4) * 4;
+    o = (o + 7) / 8 * 8;
     g.off_seg = o; o += (g.NW / 64 + 2) * 8;
     g.off_ok = o; o += (g.NW / 64 + 2) * 8;
     g.off_last = o; o += (g.NW / 64 + 2) * 8;
-    if (regs) {
-        g.off_wp = o; o += g.NWB * 20 + 4;
-        g.off_fwd = o; o += (g.NWB + 2) * 2;
-    } else {
-        g.off_wp = o; o += (g.NWB * w + 2 * (g.NWB * w / 16) + 2) * 2;
-        g.off_fwd = o; o += g.NM + 4 * (g.NM / 16) + 4;
-    }
+    g.off_fwd = o; o += 66 * 2;
     g.bytes = (o + 15) / 16 * 16;
     return g;
 }
@@ -150,50 +159,26 @@ struct Tile {
     TileGeom G;
     int64_t t0, wlo, borg;
     uint32_t d0;  // wlo - borg
-    uint8_t* lds;
-    uint64_t* mm;
-    uint64_t* wv;
-    uint16_t* wp;
     uint32_t* pk;
     uint32_t* inv;
-    uint8_t* fwd;
     uint32_t* seg;
     uint32_t* ok;
     uint32_t* last;
     uint64_t* gt;
-    bool regs;  // the w == 16 layout: wv32 / wp8 / fwd16
+    uint64_t* px;  // prefix minima, entry i of lane q at 17 q + i (not tile_w16)
+    uint64_t* pn;  // their positions in the lane's 16 m-mers, 4 bits each
     uint32_t* wv32;
     uint8_t* wp8;
     uint16_t* fwd16;
 
     GG_DEV uint32_t code_rel(int64_t r) const { return (pk[r >> 4] >> ((r & 15) * 2)) & 3; }
     GG_DEV bool inv_rel(int64_t r) const { return (inv[r >> 5] >> (r & 31)) & 1; }
-    // true when any base in [r, r+len) (relative) is not ACGT
-    GG_DEV bool any_inv(int64_t r, uint32_t len) const {
-        int64_t e = r + len;  // exclusive
-        int64_t wi = r >> 5;
-        int64_t we = (e - 1) >> 5;
-        uint32_t lo_mask = ~0u << (r & 31);
-        if (wi == we) {
-            uint32_t hi_mask = ((e & 31) == 0) ? ~0u : ((1u << (e & 31)) - 1);
-            return (inv[wi] & lo_mask & hi_mask) != 0;
-        }
-        if (inv[wi] & lo_mask) return true;
-        for (int64_t q = wi + 1; q < we; q++)
-            if (inv[q]) return true;
-        uint32_t hi_mask = ((e & 31) == 0) ? ~0u : ((1u << (e & 31)) - 1);
-        return (inv[we] & hi_mask) != 0;
-    }
     GG_DEV bool bit(const uint32_t* a, uint32_t x) const { return (a[x >> 5] >> (x & 31)) & 1; }
-    // window minimum, its m-mer position, and forward-strand flag per m-mer
-    GG_DEV uint64_t& WV(uint32_t x) const { return wv[x + (x >> 4)]; }
-    GG_DEV uint16_t& WP(uint32_t x) const { return wp[x + 2 * (x >> 4)]; }
-    GG_DEV uint8_t& FWD(uint32_t x) const { return fwd[x + 4 * (x >> 4)]; }
-    // either layout: window minimum (the w == 16 path keeps its low 32 bits),
-    // its m-mer position, and the strand flag of m-mer p
-    GG_DEV uint64_t wval(uint32_t x) const { return regs ? (uint64_t)wv32[x + (x >> 4)] : WV(x); }
-    GG_DEV uint32_t wpos(uint32_t x) const { return regs ? x + wp8[x + 4 * (x >> 4)] : WP(x); }
-    GG_DEV bool fwd_at(uint32_t p) const { return regs ? ((fwd16[p >> 4] >> (p & 15)) & 1u) != 0 : FWD(p) != 0; }
+    // window minimum (its low 32 bits), its m-mer position, and the strand
+    // flag of m-mer p
+    GG_DEV uint64_t wval(uint32_t x) const { return wv32[x + (x >> 4)]; }
+    GG_DEV uint32_t wpos(uint32_t x) const { return x + wp8[x + 4 * (x >> 4)]; }
+    GG_DEV bool fwd_at(uint32_t p) const { return ((fwd16[p >> 4] >> (p & 15)) & 1u) != 0; }
 };
 
 // 16 codes of relative positions [r, r+16) packed (position r at bits 0..1);
@@ -216,13 +201,14 @@ GG_DEV uint32_t rev_comp16(uint32_t x) {
     return y ^ 0xAAAAAAAAu;
 }
 
-GG_DEV void tile_minima_lds(Tile& t);
+template <int B>
+GG_DEV void tile_minima(Tile& t);
 GG_DEV void tile_minima_w16(Tile& t);
-GG_DEV void tile_flags(Tile& t);
 
-// Phases 0-3: load, hash, window minima, per-window flags.  WC == 16 selects
-// the register path for w == 16 (k = 31, m = 15 and other k - m == 16).
-template <int WC>
+// Phases 0-3: load, hash, window minima, per-window flags.  B == 0 selects
+// the path of w == 16 (k = 31, m = 15 and other k - m == 16), whose neighbour
+// values all come from the next lane; otherwise B is tile_block(w).
+template <int B>
 GG_DEV void tile_compute(Tile& t) {
     const BucketArgs& A = *t.A;
     const TileGeom& G = t.G;
@@ -261,81 +247,10 @@ GG_DEV void tile_compute(Tile& t) {
     }
     __syncthreads();
 
-    if (WC == 16) {
-        tile_minima_w16(t);  // also writes the flag bitmaps
-    } else {
-        tile_minima_lds(t);
-        __syncthreads();
-        tile_flags(t);
-    }
-}
-
-// Phase 1 + 2, any w: every m-mer hash goes to LDS, then van Herk blocks.
-GG_DEV void tile_minima_lds(Tile& t) {
-    const BucketArgs& A = *t.A;
-    const TileGeom& G = t.G;
-    const uint32_t lane = threadIdx.x;
-    const uint32_t m = A.m, w = A.w;
-
-    // ---- phase 1: canonical ntHash of every m-mer (rolling strips) -------
-    // fw_i = rotl1(fw_{i-1}) ^ rotl(h(s_{i-1}), m) ^ h(s_{i+m-1})
-    // rc_i = rotr1(rc_{i-1}) ^ rotr1(rc(s_{i-1})) ^ rotl(rc(s_{i+m-1}), m-1)
-    // with the "out" term dropped while the first m bases are fed.
-    {
-        const uint32_t S = (G.NM + 63) / 64;
-        uint32_t p0 = lane * S, p1 = p0 + S;
-        if (p1 > G.NM) p1 = G.NM;
-        if (p0 < p1) {
-            uint64_t fw = 0, rc = 0;
-            const int64_t rb = (int64_t)t.d0;  // relative base of m-mer 0
-            for (uint32_t j = 0; j + 1 < m; j++) {
-                uint32_t e = 16 + t.code_rel(rb + p0 + j);
-                fw = rotl1_64(fw) ^ t.gt[2 * e];
-                rc = rotr1_64(rc) ^ t.gt[2 * e + 1];
-            }
-            for (uint32_t p = p0; p < p1; p++) {
-                uint32_t in = t.code_rel(rb + p + m - 1);
-                uint32_t out = (p == p0) ? 4u : t.code_rel(rb + p - 1);
-                uint32_t e = out * 4 + in;
-                fw = rotl1_64(fw) ^ t.gt[2 * e];
-                rc = rotr1_64(rc) ^ t.gt[2 * e + 1];
-                uint64_t mn = fw < rc ? fw : rc;
-                t.mm[p] = (mn << 1) | (fw != rc ? 1ULL : 0ULL);
-                t.FWD(p) = fw < rc ? 1 : 0;
-            }
-        }
-    }
-    __syncthreads();
-
-    // ---- phase 2: window minima, van Herk / Gil-Werman blocks of w -------
-    for (uint32_t q = lane; q < G.NWB; q += 64) {
-        const uint32_t base = q * w;
-        uint64_t sv = t.mm[base + w - 1];
-        uint32_t sp = base + w - 1;
-        t.WV(base + w - 1) = sv;
-        t.WP(base + w - 1) = (uint16_t)sp;
-        for (int i = (int)w - 2; i >= 0; i--) {
-            mm_combine(t.mm[base + i], base + i, sv, sp, sv, sp);
-            t.WV(base + i) = sv;
-            t.WP(base + i) = (uint16_t)sp;
-        }
-        uint64_t pv = 0;
-        uint32_t pp = 0;
-        const uint32_t nb = base + w;
-        for (uint32_t i = 1; i < w; i++) {
-            if (i == 1) {
-                pv = t.mm[nb];
-                pp = nb;
-            } else {
-                mm_combine(pv, pp, t.mm[nb + i - 1], nb + i - 1, pv, pp);
-            }
-            uint64_t rv;
-            uint32_t rp;
-            mm_combine(t.WV(base + i), t.WP(base + i), pv, pp, rv, rp);
-            t.WV(base + i) = rv;
-            t.WP(base + i) = (uint16_t)rp;
-        }
-    }
+    if constexpr (B == 0)
+        tile_minima_w16(t);
+    else
+        tile_minima<B>(t);
 }
 
 // 64 bits of a bit array starting at bit `r` (r >= 0).
@@ -346,8 +261,8 @@ GG_DEV uint64_t bits64(const uint32_t* a, int64_t r) {
     return (lo >> sh) | ((uint64_t)a[wi + 2] << (64 - sh));
 }
 
-// Phases 1-3 for w == 16 (k <= 47), one window block of 16 per lane (the
-// tile geometry makes NWB <= 64).  The lane owning window block q hashes
+// Phases 1-3 for w == 16 and k <= 47, one window block of 16 per lane (NWB <=
+// 62 blocks of windows).  The lane owning window block q hashes
 // m-mer blocks q and q+1 (rolling update, tables in LDS), takes suffix minima
 // of block q and running prefix minima of block q+1; window q*16+i is the
 // combination of the two (van Herk / Gil-Werman in registers).  The window
@@ -359,8 +274,8 @@ GG_DEV void tile_minima_w16(Tile& t) {
     const uint32_t m = t.A->m, k = t.A->k;
     const int64_t rb = (int64_t)t.d0;  // relative base of m-mer 0 (and of window 0)
     const ulonglong2* gt2 = reinterpret_cast<const ulonglong2*>(t.gt);
-    const uint32_t q = lane;
-    const bool have = q < G.NWB;
+    const uint32_t q = lane, NWB = (G.NW + 15) / 16;
+    const bool have = q < NWB;
     const uint32_t p0 = q * 16;
     uint32_t segm = 0, okm = 0, lastm = 0;
     bool need_prev = false;
@@ -372,7 +287,7 @@ GG_DEV void tile_minima_w16(Tile& t) {
     uint64_t sv[16], nv[16];
     uint32_t sp[16];
     uint32_t fbits = 0;
-    if (q <= G.NWB) {
+    if (q <= NWB) {
         uint64_t fw = 0, rc = 0;
         for (uint32_t j = 0; j + 1 < m; j++) {
             const ulonglong2 g = gt2[16 + t.code_rel(rb + p0 + j)];
@@ -479,42 +394,179 @@ GG_DEV void tile_minima_w16(Tile& t) {
     __syncthreads();
 }
 
-// Phase 3: per-window flags.
-GG_DEV void tile_flags(Tile& t) {
-    const BucketArgs& A = *t.A;
-    const TileGeom& G = t.G;
-    const uint32_t lane = threadIdx.x;
-    const uint32_t k = A.k;
-    const uint32_t nwords64 = (G.NW + 63) / 64;
-    for (uint32_t c = 0; c < nwords64; c++) {
-        uint32_t x = c * 64 + lane;
-        bool okf = false, lastf = false, segf = false;
-        if (x >= 1 && x < G.NW) {
-            int64_t r = (int64_t)t.d0 + x;  // relative base of window start
-            bool valid = !t.any_inv(r, k - 1);
-            bool first = t.inv_rel(r - 1);
-            bool lst = t.inv_rel(r + k - 1);
-            okf = valid && !(first && lst);
-            lastf = okf && lst;
-            if (okf) {
-                uint64_t v0 = t.WV(x - 1), v1 = t.WV(x);
-                bool differs = (v0 != v1) || ((v1 & 1) && t.WP(x) != t.WP(x - 1));
-                segf = first || differs;
-            }
-        }
-        uint64_t bs = __ballot(segf), bo = __ballot(okf), bl = __ballot(lastf);
-        if (lane == 0) {
-            reinterpret_cast<uint64_t*>(t.seg)[c] = bs;
-            reinterpret_cast<uint64_t*>(t.ok)[c] = bo;
-            reinterpret_cast<uint64_t*>(t.last)[c] = bl;
+// Canonical ntHashes of the lane's m-mers p0 .. p0 + 15 (rolling update, tables
+// in LDS) as v = hash << 1 | !symmetric; returns their strand bits.
+//   fw_i = rotl1(fw_{i-1}) ^ rotl(h(s_{i-1}), m) ^ h(s_{i+m-1})
+//   rc_i = rotr1(rc_{i-1}) ^ rotr1(rc(s_{i-1})) ^ rotl(rc(s_{i+m-1}), m-1)
+// with the "out" term dropped while the first m bases are fed.
+GG_DEV uint32_t hash_block16(const Tile& t, uint32_t p0, uint64_t* v) {
+    const ulonglong2* gt2 = reinterpret_cast<const ulonglong2*>(t.gt);
+    const int64_t rb = (int64_t)t.d0 + p0;
+    const uint32_t m = t.A->m;
+    uint64_t fw = 0, rc = 0;
+    for (uint32_t j0 = 0; j0 + 1 < m; j0 += 16) {
+        const uint32_t c = extract16(t, rb + j0), n = m - 1 - j0 < 16 ? m - 1 - j0 : 16;
+        for (uint32_t j = 0; j < n; j++) {
+            const ulonglong2 g = gt2[16 + ((c >> (2 * j)) & 3u)];
+            fw = rotl1_64(fw) ^ g.x;
+            rc = rotr1_64(rc) ^ g.y;
         }
     }
-    __syncthreads();
+    const uint32_t inw = extract16(t, rb + m - 1);
+    const uint32_t outw = extract16(t, rb - 1);
+    uint32_t fbits = 0;
+#pragma unroll
+    for (int i = 0; i < 16; i++) {
+        const uint32_t in = (inw >> (2 * i)) & 3u, out = (outw >> (2 * i)) & 3u;
+        const ulonglong2 g = gt2[(i == 0 ? 16u : out * 4u) + in];
+        fw = rotl1_64(fw) ^ g.x;
+        rc = rotr1_64(rc) ^ g.y;
+        const uint64_t mn = fw < rc ? fw : rc;
+        v[i] = (mn << 1) | (fw != rc ? 1ULL : 0ULL);
+        fbits |= (fw < rc ? 1u : 0u) << i;
+    }
+    return fbits;
 }
 
-GG_DEV bool tile_is_end(const Tile& t, uint32_t x) {
-    if (!t.bit(t.ok, x)) return false;
-    return t.bit(t.last, x) || t.bit(t.seg, x + 1);
+// Flags of the lane's 16 windows x = p0 + i from the invalid-base bits alone,
+// one bit per window: `ok` when the window (bases x .. x + k - 2) is all ACGT
+// and not an isolated one of its run, `first` / `last` when the base before /
+// behind it ends the run.  Bit j of im = base p0 - 1 + j is invalid; a window
+// is bad when any of bits i + 1 .. i + k - 1 is set: an OR over k - 1 shifts,
+// doubled, for the 16 windows at once.
+GG_DEV void window_flags16(const Tile& t, uint32_t p0, uint32_t* ok, uint32_t* first, uint32_t* last) {
+    const uint32_t k = t.A->k;
+    const int64_t r = (int64_t)t.d0 + p0 - 1;
+    const u128_t im = (u128_t)bits64(t.inv, r) | ((u128_t)bits64(t.inv, r + 64) << 64);
+    u128_t bad = im >> 1;
+    uint32_t len = 1;
+    while (2 * len <= k - 1) {
+        bad |= bad >> len;
+        len *= 2;
+    }
+    if (len < k - 1) bad |= bad >> (k - 1 - len);
+    const uint32_t f = (uint32_t)im & 0xFFFFu, l = (uint32_t)(im >> k) & 0xFFFFu;
+    // windows 1 .. NW - 1 of the tile
+    uint32_t in = p0 + 16 <= t.G.NW ? 0xFFFFu : p0 >= t.G.NW ? 0u : (1u << (t.G.NW - p0)) - 1u;
+    if (p0 == 0) in &= ~1u;
+    *ok = ~(uint32_t)bad & ~(f & l) & in;
+    *first = f;
+    *last = l;
+}
+
+// Bitmaps of the tile's windows from the lanes' 16-bit pieces; words past the
+// last window are zero.
+GG_DEV void write_bitmaps16(Tile& t, uint32_t segm, uint32_t okm, uint32_t lastm) {
+    const uint32_t lane = threadIdx.x;
+    const uint32_t npieces = (t.G.NW / 64 + 2) * 4;
+    for (uint32_t pc = lane; pc < npieces; pc += 64) {
+        const bool mine = pc == lane;
+        reinterpret_cast<uint16_t*>(t.seg)[pc] = mine ? (uint16_t)segm : 0;
+        reinterpret_cast<uint16_t*>(t.ok)[pc] = mine ? (uint16_t)okm : 0;
+        reinterpret_cast<uint16_t*>(t.last)[pc] = mine ? (uint16_t)lastm : 0;
+    }
+}
+
+// Phases 1-3 for any w >= B: lane q hashes m-mers 16q .. 16q + 15 and keeps
+// the suffix minima of their blocks of B in registers; the blocks' prefix
+// minima go to LDS.  Window x = 16q + i covers the suffix of its block from
+// i, the blocks between (none for w < 2B except one where the window crosses
+// two block ends, at most three for B = 16; a block's last prefix minimum is
+// its minimum) and the prefix up to m-mer x + w - 1 (van Herk / Gil-Werman
+// with a block that need not be w).  All index arithmetic on i is uniform, so
+// each window costs one 64-bit LDS read and two or three combinations, on all
+// 64 lanes; LDS arrays of every m-mer and one lane per block of w before.
+// Bound by VALU issue (64-bit hashing and compares).  Staging pass of 0.9
+// Gbases at w = 42: 22.1 -> 5.4 ms; of 0.24 Gbases at w = 33: 5.5 -> 1.4 ms.
+template <int B>
+GG_DEV void tile_minima(Tile& t) {
+    const uint32_t q = threadIdx.x, p0 = 16 * q, w = t.A->w;
+    uint64_t sv[16];
+    uint32_t sp[16];
+    t.fwd16[q] = (uint16_t)hash_block16(t, p0, sv);
+    uint32_t okm, firstm, lastm;
+    window_flags16(t, p0, &okm, &firstm, &lastm);
+    lastm &= okm;
+    {
+        uint64_t pv = 0, nib = 0;
+        uint32_t pp = 0;
+#pragma unroll
+        for (int i = 0; i < 16; i++) {
+            sp[i] = i;
+            if (i % B == 0) {
+                pv = sv[i];
+                pp = i;
+            } else {
+                mm_combine(pv, pp, sv[i], i, pv, pp);
+            }
+            t.px[17 * q + i] = pv;
+            nib |= (uint64_t)pp << (4 * i);
+        }
+        t.pn[q] = nib;
+#pragma unroll
+        for (int i = 14; i >= 0; i--)
+            if (i % B != B - 1) mm_combine(sv[i], sp[i], sv[i + 1], sp[i + 1], sv[i], sp[i]);
+    }
+    __syncthreads();
+    // window minima: low words, offsets, and where a window's minimum differs
+    // from the window before
+    uint32_t rv32[16], offs[4] = {0u, 0u, 0u, 0u}, diffm = 0;
+    uint64_t first_v = 0, last_v = 0, mv = 0;
+    uint32_t first_p = 0, last_p = 0, mp = 0, n_mid = 0;
+#pragma unroll
+    for (int i = 0; i < 16; i++) {
+        uint64_t rv = sv[i];
+        uint32_t rp = p0 + sp[i];
+        const uint32_t e = i + w - 1;  // last m-mer of the window, relative to p0
+        const uint32_t d = e / B - i / B;  // blocks from the window's first m-mer to its last
+        if (B == 16) {
+            // the blocks between only grow with i
+            while (n_mid + 1 < d) {
+                n_mid++;
+                const uint32_t qb = q + n_mid < 64 ? q + n_mid : 63u;  // windows past the tile's are not used
+                const uint64_t bv = t.px[17 * qb + 15];
+                const uint32_t bp = 16 * qb + (uint32_t)(t.pn[qb] >> 60);
+                if (n_mid == 1) {
+                    mv = bv;
+                    mp = bp;
+                } else {
+                    mm_combine(mv, mp, bv, bp, mv, mp);
+                }
+            }
+            if (n_mid) mm_combine(rv, rp, mv, mp, rv, rp);
+        } else if (d == 2) {
+            const uint32_t z = (i / B + 1) * B + B - 1;
+            const uint32_t qb = q + (z >> 4) < 64 ? q + (z >> 4) : 63u;
+            mm_combine(rv, rp, t.px[17 * qb + (z & 15)], 16 * qb + (uint32_t)((t.pn[qb] >> (4 * (z & 15))) & 15), rv, rp);
+        }
+        if (d) {
+            const uint32_t qe = q + (e >> 4) < 64 ? q + (e >> 4) : 63u;
+            mm_combine(rv, rp, t.px[17 * qe + (e & 15)], 16 * qe + (uint32_t)((t.pn[qe] >> (4 * (e & 15))) & 15), rv, rp);
+        }
+        rv32[i] = (uint32_t)rv;
+        offs[i >> 2] |= (rp - (p0 + i)) << (8 * (i & 3));
+        if (i == 0) {
+            first_v = rv;
+            first_p = rp;
+        } else if (rv != last_v || ((rv & 1) && rp != last_p)) {
+            diffm |= 1u << i;
+        }
+        last_v = rv;
+        last_p = rp;
+    }
+    // window p0 against the previous lane's last window
+    const uint64_t prev_v = lane_prev64(last_v);
+    const uint32_t prev_p = lane_prev32(last_p);
+    if (prev_v != first_v || ((first_v & 1) && first_p != prev_p)) diffm |= 1u;
+    const uint32_t segm = okm & (firstm | diffm);
+    __syncthreads();  // the prefix minima were read: their LDS is reused
+#pragma unroll
+    for (int i = 0; i < 16; i++) t.wv32[17 * q + i] = rv32[i];
+    uint32_t* o4 = reinterpret_cast<uint32_t*>(t.wp8 + 20 * q);
+#pragma unroll
+    for (int j = 0; j < 4; j++) o4[j] = offs[j];
+    write_bitmaps16(t, segm, okm, lastm);
+    __syncthreads();
 }
 
 // Sub-bucket of a window minimum: bucket = (h >> 1) mod 2^b for a unique
@@ -534,23 +586,19 @@ GG_DEV uint32_t unit_of(uint64_t v, uint32_t b, uint32_t sb, uint32_t xb) {
     return (sub_of(v, b, sb) << xb) | extra;
 }
 
-GG_DEV void tile_init(Tile& t, const BucketArgs* A, uint64_t tile, uint8_t* lds, bool regs) {
+GG_DEV void tile_init(Tile& t, const BucketArgs* A, uint64_t tile, uint8_t* lds) {
     t.A = A;
-    t.G = tile_geom(A->T, A->w, A->k, A->m, regs);
+    t.G = tile_geom(A->T, A->w, A->k, A->m);
     t.t0 = (int64_t)tile * A->T;
-    t.wlo = t.t0 - A->w;
+    t.wlo = t.t0 - tile_halo(A->w);
     int64_t bo = t.wlo - 1;
     t.borg = (bo >= 0) ? (bo / 16) * 16 : -(((-bo) + 15) / 16) * 16;
     t.d0 = (uint32_t)(t.wlo - t.borg);
-    t.lds = lds;
     t.gt = reinterpret_cast<uint64_t*>(lds + t.G.off_g);
-    t.mm = reinterpret_cast<uint64_t*>(lds + t.G.off_mm);
-    t.wv = reinterpret_cast<uint64_t*>(lds + t.G.off_wv);
-    t.wp = reinterpret_cast<uint16_t*>(lds + t.G.off_wp);
+    t.px = reinterpret_cast<uint64_t*>(lds + t.G.off_px);
+    t.pn = reinterpret_cast<uint64_t*>(lds + t.G.off_pn);
     t.pk = reinterpret_cast<uint32_t*>(lds + t.G.off_pk);
     t.inv = reinterpret_cast<uint32_t*>(lds + t.G.off_inv);
-    t.fwd = lds + t.G.off_fwd;
-    t.regs = regs;
     t.wv32 = reinterpret_cast<uint32_t*>(lds + t.G.off_wv);
     t.wp8 = lds + t.G.off_wp;
     t.fwd16 = reinterpret_cast<uint16_t*>(lds + t.G.off_fwd);
@@ -559,15 +607,15 @@ GG_DEV void tile_init(Tile& t, const BucketArgs* A, uint64_t tile, uint8_t* lds,
     t.last = reinterpret_cast<uint32_t*>(lds + t.G.off_last);
 }
 
-// w == 16 path: group ends among the 16 windows of the lane's block that the
-// tile owns (windows w .. w+T-1, absolute index below n).  Returns the mask
-// and sets *x0 / *j0 (first window, relative and absolute) and *segm.
+// Group ends among the 16 windows of the lane's block that the tile owns
+// (windows halo .. halo+T-1, absolute index below n).  Returns the mask and
+// sets *x0 / *j0 (first window, relative and absolute) and *segm.
 GG_DEV uint32_t lane_end_mask16(const Tile& t, uint32_t* x0, int64_t* j0, uint32_t* segm) {
-    const uint32_t q = threadIdx.x;
+    const uint32_t q = threadIdx.x, q0 = tile_halo(t.A->w) / 16;
     *x0 = q * 16;
-    *j0 = t.t0 + (int64_t)q * 16 - 16;
+    *j0 = t.wlo + (int64_t)q * 16;
     *segm = 0;
-    if (q < 1 || q > t.A->T / 16) return 0;
+    if (q < q0 || q >= q0 + t.A->T / 16) return 0;
     const uint32_t sg = reinterpret_cast<const uint16_t*>(t.seg)[q];
     const uint32_t okm = reinterpret_cast<const uint16_t*>(t.ok)[q];
     const uint32_t lastm = reinterpret_cast<const uint16_t*>(t.last)[q];
@@ -657,10 +705,10 @@ struct RecInfo {
 
 GG_DEV RecInfo rec_info(const Tile& t, uint32_t x) {
     const BucketArgs& A = *t.A;
-    const uint32_t w = A.w, k = A.k, m = A.m;
+    const uint32_t k = A.k, m = A.m;
     RecInfo r;
     r.ok = false;
-    const int64_t bwin = t.t0 + (int64_t)x - w;
+    const int64_t bwin = t.wlo + (int64_t)x;
     // group start: latest group-start bit at or before x inside the tile
     int64_t a = -1;
     {
@@ -816,22 +864,21 @@ constexpr uint32_t STAGE_R = 2;
 // (which gives its rank there), built and staged at the tile's positions; the
 // first record of a tile whose group starts further back is deferred to
 // bucket_defer_kernel, which runs once the group-start bitmap is complete.
-template <int WC>
+template <int B>
 __global__ __launch_bounds__(64) void bucket_stage_kernel(BucketArgs A) {
     extern __shared__ __align__(16) uint8_t lds[];
     Tile t;
-    tile_init(t, &A, A.tile0 + blockIdx.x, lds, WC != 0);
-    tile_compute<WC>(t);
+    tile_init(t, &A, A.tile0 + blockIdx.x, lds);
+    tile_compute<B>(t);
     const uint32_t lane = threadIdx.x;
-    const uint32_t w = A.w;
     const uint32_t SW = A.slot_words;
     __shared__ uint16_t ends[1024];
     __shared__ uint32_t n_ends;
-    if (WC == 16) {
+    {
         uint32_t x0, segm;
         int64_t j0;
         uint32_t endm = lane_end_mask16(t, &x0, &j0, &segm);
-        if (lane >= 1 && lane <= A.T / 16) reinterpret_cast<uint16_t*>(A.seg_bits)[j0 >> 4] = (uint16_t)segm;
+        if (j0 >= t.t0 && j0 < t.t0 + A.T) reinterpret_cast<uint16_t*>(A.seg_bits)[j0 >> 4] = (uint16_t)segm;
         const uint32_t cnt = __popc(endm);
         uint32_t inc = cnt;
         for (uint32_t d = 1; d < 64; d <<= 1) {
@@ -846,26 +893,6 @@ __global__ __launch_bounds__(64) void bucket_stage_kernel(BucketArgs A) {
         }
         if (lane == 63) n_ends = inc;
         __syncthreads();
-    } else {
-        if (lane == 0) n_ends = 0;
-        __syncthreads();
-        for (uint32_t c = 0; c < A.T; c += 64) {
-            const uint32_t x = w + c + lane;
-            const int64_t j = t.t0 + c + lane;
-            const bool sg = t.bit(t.seg, x) && j < (int64_t)A.n;
-            const uint64_t bs = __ballot(sg);
-            if (lane == 0) {
-                const uint64_t wi = (uint64_t)(t.t0 + c) >> 5;
-                A.seg_bits[wi] = (uint32_t)bs;
-                A.seg_bits[wi + 1] = (uint32_t)(bs >> 32);
-            }
-            const bool e = j < (int64_t)A.n && tile_is_end(t, x);
-            const uint64_t be = __ballot(e);
-            if (e) ends[n_ends + __popcll(be & ((1ULL << lane) - 1))] = (uint16_t)x;
-            __syncthreads();
-            if (lane == 0) n_ends += (uint32_t)__popcll(be);
-            __syncthreads();
-        }
     }
     const uint32_t n_end = n_ends;
     for (uint32_t e0 = 0; e0 < n_end; e0 += 64 * STAGE_R) {
@@ -885,7 +912,7 @@ __global__ __launch_bounds__(64) void bucket_stage_kernel(BucketArgs A) {
                 // group starts before the halo (non-unique minimizer): defer
                 const uint32_t d = atomicAdd(A.defer_count, 1u);
                 if (d < A.n_tiles) {
-                    A.defer[3 * (uint64_t)d] = (uint64_t)(t.t0 + (int64_t)x - w);
+                    A.defer[3 * (uint64_t)d] = (uint64_t)(t.wlo + (int64_t)x);
                     A.defer[3 * (uint64_t)d + 1] = t.wval(x);
                     A.defer[3 * (uint64_t)d + 2] = t.bit(t.last, x) ? 1 : 0;
                 } else {
