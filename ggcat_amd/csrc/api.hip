@@ -789,7 +789,7 @@ int ggcat_gpu_bucketing(ggcat_gpu_ctx* ctx, const uint8_t* data, uint64_t n_byte
         // (the two take disjoint units); both persistent grids are as large
         // as the CUs hold at once
         const bool wide = unit_cap > DEDUP_SMALL && DEDUP_WIDE * slot_words / 4 <= 8 * 256;
-        ctx->dd_max = wide ? DEDUP_WIDE : DEDUP_SMALL;
+        ctx->dd_max = wide ? DEDUP_WIDE : std::min(DEDUP_SMALL, 8 * 64 * 4 / slot_words);
         const size_t lds_small = dedup_lds_bytes(DEDUP_SMALL, slot_words, n_colors != 0);
         const size_t lds_wide = dedup_lds_bytes(DEDUP_WIDE, slot_words, n_colors != 0);
         int occ = 0;

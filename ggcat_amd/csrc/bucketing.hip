@@ -1082,8 +1082,7 @@ __host__ __device__ inline uint32_t dedup_lds_bytes(uint32_t max_rec, uint32_t s
 
 // NT threads per workgroup, units of LO < records <= HI (and, with PASS, the
 // other units kept as they are, except those of (DEDUP_SMALL, DEDUP_WIDE]
-// when the wide launch takes them).  At most 8 16-byte pieces per thread:
-// HI * slot_words / 4 <= 8 * NT.
+// when the wide launch takes them).  At most 8 16-byte pieces per thread.
 template <uint32_t NT, uint32_t LO, uint32_t HI, bool PASS>
 GG_DEV void unit_dedup_body(const BucketArgs& A, uint32_t n_units, bool wide) {
     extern __shared__ __align__(16) uint8_t lds[];
@@ -1095,7 +1094,9 @@ GG_DEV void unit_dedup_body(const BucketArgs& A, uint32_t n_units, bool wide) {
     const uint32_t SW = A.slot_words, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     uint32_t* rec = reinterpret_cast<uint32_t*>(lds);  // slot words
     uint32_t* col = rec + HI * SW;  // colored builds only
-    auto mine = [&](uint32_t n) { return n > LO && n <= HI; };
+    // a region must also fit the registers that stage it: with 16-word slots
+    // units of up to 128 records do
+    auto mine = [&](uint32_t n) { return n > LO && n <= HI && n * (SW / 4) <= 8 * NT; };
     // a unit's region is loaded into registers while the previous unit is
     // processed
     uint4 p0 = {}, p1 = {}, p2 = {}, p3 = {}, p4 = {}, p5 = {}, p6 = {}, p7 = {};
