@@ -99,7 +99,7 @@ struct ggcat_gpu_ctx {
     std::vector<uint8_t> cyc_seq, cyc_flags;
     std::vector<uint32_t> cyc_sub;
     DevBuf u_path;  // colored builds: table position of every unitig k-mer, in written order
-    DevBuf rk_pos;  // rabin-karp128 per-position start terms of the merge's rolling hash
+    DevBuf rk_pos, rk_tri;  // rabin-karp128 terms per position of the merge (rolling start state, whole k-mer)
     uint32_t rk_pos_k = 0;  // k they were computed for (0: none)
     // input files read straight into HBM: raw bytes, parse state per chunk,
     // and a pinned two-buffer staging ring for the uploads
@@ -461,7 +461,7 @@ void ggcat_gpu_destroy(ggcat_gpu_ctx* ctx) {
                       &ctx->u_rest_n, &ctx->u_rep, &ctx->u_tab, &ctx->u_path, &ctx->stage_slots, &ctx->stage_unit,
                       &ctx->stage_rank, &ctx->stage_color, &ctx->stage_cursor, &ctx->defer, &ctx->defer_count,
                       &ctx->kmer_total, &ctx->spill_slots, &ctx->spill_color, &ctx->raw, &ctx->p_stats,
-                      &ctx->p_carry, &ctx->p_keep, &ctx->p_keep_off, &ctx->p_flags, &ctx->p_bits, &ctx->rk_pos,
+                      &ctx->p_carry, &ctx->p_keep, &ctx->p_keep_off, &ctx->p_flags, &ctx->p_bits, &ctx->rk_pos, &ctx->rk_tri,
                       &ctx->copy_mult, &ctx->copy_flags};
     if (ctx->pin_ring) (void)hipHostFree(ctx->pin_ring);
     if (ctx->server) (void)ggcat_gpu_serve_close(ctx);
@@ -1389,8 +1389,20 @@ int ggcat_gpu_kmers_merge(ggcat_gpu_ctx* ctx) {
     M.kind = p.hash_kind;
     M.key_words = key_words;
     const uint32_t W = ctx->colored ? ctx->color_words : 0;
-    const size_t entry_bytes = 12 * key_words + 4 * W + 2;  // + claimed-slot list entry
-    M.lds_cap = key_words == 1 ? 2048 : 1024;
+    // identical records counted once (inline slots)
+    M.dedup = (ctx->slot_words <= 8 && ctx->tune.no_dedup != 1) ? 1 : 0;
+    // the merge's variant (see Mode in merge.hip): 0 takes what the others do
+    // not, among it the schedules without spread k-mers
+    const bool rk = p.hash_kind == GGCAT_GPU_HASH_RK128;
+    int mode = 0;
+    if (M.dedup && ctx->tune.no_dedup != 2 && p.k < 64 && !(rk && W))
+        mode = W    ? (p.k <= 32 ? 6 : 7)
+               : rk ? (p.k <= 32 ? 3 : 5)
+                    : (p.k > 32 ? 4 : ctx->slot_words == 4 ? 1 : 2);
+    const uint32_t table_words = mode == 0 ? key_words : p.k <= 32 ? 1 : 2;  // key words of a table entry
+    // table entry with its place in the claimed-slot list (mode 0: a state word beside a 128-bit key)
+    const size_t entry_bytes = 8 * table_words + 4 + (mode == 0 && key_words == 2 ? 4 : 0) + 4 * W + 2;
+    M.lds_cap = table_words == 1 ? 2048 : 1024;
     if (ctx->tune.lds_table_log) M.lds_cap = 1u << std::min<uint32_t>(std::max<uint32_t>(ctx->tune.lds_table_log, 8), 13);
     while (M.lds_cap > 256 && M.lds_cap * entry_bytes > 48 * 1024) M.lds_cap >>= 1;
     M.table_pct = ctx->tune.table_pct ? ctx->tune.table_pct : 200;
@@ -1398,29 +1410,37 @@ int ggcat_gpu_kmers_merge(ggcat_gpu_ctx* ctx) {
     M.slot_color = W ? P_<uint32_t>(ctx->slot_color) : nullptr;
     M.lds_try = ctx->tune.lds_max_occ ? ctx->tune.lds_max_occ : M.lds_cap * 16;
     const uint32_t item_occ = ctx->tune.item_occ ? ctx->tune.item_occ : M.lds_cap / 2;
-    // identical records counted once (seq-hash keys up to k = 32, inline slots)
-    M.dedup = (ctx->slot_words <= 8 && ctx->tune.no_dedup != 1) ? 1 : 0;
-    M.tag_kmers = (p.hash_kind == GGCAT_GPU_HASH_SEQ && p.k <= 32 && ctx->tune.no_dedup != 2) ? 1 : 0;
     // work items whose units the compaction deduplicated skip the record hashing
     M.rec_direct = ctx->tune.no_dedup != 3 ? 1 : 0;
     // workgroup size of the merge (128 or 256 threads); a chunk of records
     // (rec_cap / 2) has at most one record per thread
     const uint32_t merge_threads = ctx->tune.merge_threads == 128 ? 128u : 256u;
-    M.rec_cap = std::min<uint32_t>(ctx->tune.rec_cap ? ctx->tune.rec_cap : REC_CAP_DEFAULT, 2 * merge_threads);
+    M.rec_cap =
+        std::min<uint32_t>(ctx->tune.rec_cap ? ctx->tune.rec_cap : rec_cap_default(ctx->slot_words), 2 * merge_threads);
     M.rec_lds_off = (uint32_t)(((size_t)M.lds_cap * entry_bytes + 64 + 15) / 16 * 16);
-    // the uncolored rabin-karp128 variant spreads the distinct records' k-mers
-    // over the workgroup in segments (tags in the record table's LDS)
-    const bool rk_seg = M.dedup && key_words == 2 && W == 0 && !M.tag_kmers && ctx->slot_words == 8 &&
-                        p.hash_kind == GGCAT_GPU_HASH_RK128;
     const size_t lds_bytes =
-        M.dedup ? M.rec_lds_off + rec_table_bytes(ctx->slot_words, (M.tag_kmers || rk_seg) ? p.k : 0xFFFFu, M.rec_cap, rk_seg)
+        M.dedup ? M.rec_lds_off + rec_table_bytes(ctx->slot_words, p.k, M.rec_cap, mode == 0 ? 0 : mode == 1 ? 1 : 4, W != 0,
+                                                  mode == 3 || mode == 5 ? M.lds_cap : 0)
                 : (size_t)M.lds_cap * entry_bytes + 64;
     M.pool_words = ctx->pool_words;
     set_rk_constants(M, p.k);
     if (p.hash_kind == GGCAT_GPU_HASH_RK128) {
         // start terms of the rolling hash per base position and base
         if (ctx->rk_pos_k != p.k) {
-            std::vector<u128_t> tab((size_t)8 * (p.k - 1));
+            std::vector<u128_t> tab((size_t)8 * (p.k - 1)), tri((size_t)128 * ((p.k + 2) / 3));
+            std::vector<u128_t> pw(p.k);  // M^i
+            pw[0] = 1;
+            for (uint32_t i = 1; i < p.k; i++) pw[i] = pw[i - 1] * M.rk_mult;
+            for (uint32_t e = 0; e < tri.size() / 2; e++) {
+                u128_t f = 0, b = 0;
+                for (uint32_t j = 0, i = 3 * (e / 64); j < 3 && i < p.k; j++, i++) {
+                    const uint32_t c = (e >> (2 * j)) & 3;
+                    f += M.rk_fwd[c] * pw[p.k - 1 - i];
+                    b += M.rk_bkw[c] * pw[i];
+                }
+                tri[2 * e] = f;
+                tri[2 * e + 1] = b;
+            }
             for (uint32_t i = 0; i + 1 < p.k; i++) {
                 u128_t pf = 1, pb = M.rk_mult;  // M^(k-2-i), M^(i+1)
                 for (uint32_t e = 0; e + 2 + i < p.k; e++) pf *= M.rk_mult;
@@ -1431,11 +1451,14 @@ int ggcat_gpu_kmers_merge(ggcat_gpu_ctx* ctx) {
                 }
             }
             ctx->rk_pos_k = 0;
+            ENSURE(ctx->rk_tri, tri.size() * sizeof(u128_t));
+            HIPCHK(hipMemcpy(ctx->rk_tri.p, tri.data(), tri.size() * sizeof(u128_t), hipMemcpyHostToDevice));
             ENSURE(ctx->rk_pos, tab.size() * sizeof(u128_t));
             HIPCHK(hipMemcpy(ctx->rk_pos.p, tab.data(), tab.size() * sizeof(u128_t), hipMemcpyHostToDevice));
             ctx->rk_pos_k = p.k;
         }
         M.rk_pos = P_<u128_t>(ctx->rk_pos);
+        M.rk_tri = P_<u128_t>(ctx->rk_tri);
     }
 
     // work items: runs of units of one sub-bucket
@@ -1460,13 +1483,11 @@ int ggcat_gpu_kmers_merge(ggcat_gpu_ctx* ctx) {
 
     // resident workgroups per CU: what the 160 KiB LDS holds with the
     // kernel's static LDS, at most 8 (32 waves of 64)
-    // the seq-hash k <= 32 dedup path runs a variant with its switches compiled in,
-    const bool mode1 = key_words == 1 && W == 0 && M.dedup && M.tag_kmers && ctx->slot_words == 4;
-    // and the uncolored rabin-karp128 path another
-    const bool mode2 = key_words == 2 && W == 0 && !M.tag_kmers && ctx->slot_words == 8 &&
-                       p.hash_kind == GGCAT_GPU_HASH_RK128;
-    void (*merge_kernel)(MergeArgs) =
-        mode1 ? merge_lds_seq64_kernel : mode2 ? merge_lds_rk128_kernel : merge_lds_kernel;
+    static void (*const variants[])(MergeArgs) = {merge_lds_kernel,        merge_lds_seq64_kernel, merge_lds_seq64w_kernel,
+                                                  merge_lds_rk64_kernel,   merge_lds_seq128_kernel,
+                                                  merge_lds_rk128_kernel,  merge_lds_col64_kernel,
+                                                  merge_lds_col128_kernel};
+    void (*merge_kernel)(MergeArgs) = variants[mode];
     hipFuncAttributes fa{};
     HIPCHK(hipFuncGetAttributes(&fa, reinterpret_cast<const void*>(merge_kernel)));
     const size_t wg_lds = (lds_bytes + fa.sharedSizeBytes + 511) / 512 * 512;  // allocation granule

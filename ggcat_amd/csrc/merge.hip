@@ -60,8 +60,6 @@ struct MergeArgs {
     uint32_t lds_try;  // first pass: items with more occurrences go straight to partitioned passes
     uint32_t table_pct;  // table slots per 100 occurrences of a whole-item pass (power-of-two rounded)
     uint32_t dedup;  // identical records of an entry are inserted once with their count
-    uint32_t tag_kmers;  // dedup: every k-mer position of the distinct records is a thread's work item
-                         // (seq-hash, k <= 32); otherwise each distinct record's k-mers are rolled by one thread
     uint32_t rec_lds_off;  // byte offset of the record table in dynamic LDS
     uint32_t rec_cap;  // record table slots
     uint32_t rec_direct;  // items without dup: records placed in the record table by position, not hashed
@@ -98,28 +96,50 @@ struct MergeArgs {
     // per base position i < k - 1 of a k-mer and base c: entry 2(4i + c) is
     // rk_fwd[c] * rk_mult^(k-2-i), entry 2(4i + c) + 1 is rk_bkw[c] * rk_mult^(i+1)
     const u128_t* rk_pos;
+    // sums of three bases' terms of a whole k-mer's two hashes: entry
+    // 2(64g + c) is sum of rk_fwd[c_j] * rk_mult^(k-1-i) over the bases i =
+    // 3g + j (j < 3, i < k, c_j the j-th 2-bit code of c), entry
+    // 2(64g + c) + 1 the sum of rk_bkw[c_j] * rk_mult^i
+    const u128_t* rk_tri;
 };
 
 GG_DEV uint32_t hash128(uint64_t lo, uint64_t hi) { return tab_hash64(lo ^ (hi * 0x9E3779B97F4A7C15ULL)); }
 
-// Kernel variants: MODE 0 reads every switch from the arguments; MODE 1 is
-// the seq-hash k <= 32 path (64-bit keys, 4-word slots, record dedup with one
-// k-mer position per thread, no colors) and MODE 2 the uncolored
-// rabin-karp128 path (128-bit keys, 8-word slots, record dedup with each
-// distinct record rolled by one thread), with those switches compiled in,
-// which keeps the other paths' code out of their register allocation.
+// Kernel variants.  MODE 0 reads every switch from the arguments: the paths
+// without spread k-mers (no_dedup), k = 64, slots of 16 words and colored
+// rabin-karp128.  The others have their key width, hash and colors compiled
+// in, which keeps the other paths' code out of their register allocation:
+//   1 seq-hash k <= 32, 4-word slots      2 seq-hash k <= 32
+//   3 rabin-karp128 k <= 32               4 seq-hash 32 < k < 64
+//   5 rabin-karp128 32 < k < 64           6, 7 as 2 and 4 with colors
+// All of them count the canonical 2-bit k-mers, which name the same entries as
+// their rabin-karp128 hashes (up to hash collisions, 2^-128 per pair of
+// k-mers); an entry's hash is formed when it is emitted (rk_of_kmer), so that
+// the 128-bit multiplies of the rolling hash are not paid per occurrence.
 template <int MODE>
 struct Mode {
-    static constexpr bool S64 = MODE == 1;  // seq-hash k <= 32, 4-word slots, uncolored
-    static GG_DEV uint32_t key_words(const MergeArgs& A) { return S64 ? 1u : MODE == 2 ? 2u : A.key_words; }
-    static GG_DEV uint32_t color_words(const MergeArgs& A) { return MODE != 0 ? 0u : A.color_words; }
-    static GG_DEV bool seq64(const MergeArgs& A) { return S64 || (MODE == 0 && A.kind == 0 && A.k <= 32); }
-    static GG_DEV bool seq128(const MergeArgs& A) { return MODE == 0 && A.kind == 0; }
-    static GG_DEV bool dedup(const MergeArgs& A) { return S64 || A.dedup; }
-    static GG_DEV bool tag_kmers(const MergeArgs& A) { return S64 || (MODE == 0 && A.tag_kmers); }
-    static GG_DEV uint32_t slot_words(const MergeArgs& A) { return S64 ? 4u : MODE == 2 ? 8u : A.slot_words; }
-    static constexpr uint32_t MAX_SW = S64 ? 4u : 8u;  // register copies of a slot
+    static constexpr bool FAST = MODE != 0;
+    static constexpr uint32_t TKW = (MODE == 4 || MODE == 5 || MODE == 7) ? 2u : 1u;  // table key words (MODE != 0)
+    static constexpr bool RK = MODE == 3 || MODE == 5;
+    static constexpr bool COL = MODE == 6 || MODE == 7;
+    // k-mers of a distinct record that one thread takes: one where the tags of
+    // every k-mer position fit beside the other LDS tables (4-word slots: 18
+    // per record at most), else runs of four, rolled
+    static constexpr uint32_t SEG = MODE == 1 ? 1u : 4u;
+    static GG_DEV uint32_t key_words(const MergeArgs& A) { return RK || TKW == 2 ? 2u : FAST ? 1u : A.key_words; }
+    static GG_DEV uint32_t color_words(const MergeArgs& A) { return FAST && !COL ? 0u : A.color_words; }
+    static GG_DEV bool dedup(const MergeArgs& A) { return FAST || A.dedup; }
+    static GG_DEV uint32_t slot_words(const MergeArgs& A) { return MODE == 1 ? 4u : A.slot_words; }
+    static constexpr uint32_t MAX_SW = MODE == 1 ? 4u : 8u;  // register copies of a slot
 };
+
+// Table keys of 32 < k < 64: the low 63 bits of the 2-bit k-mer and the rest,
+// so that neither word is EMPTY64.
+GG_DEV void pair_of(uint64_t lo, uint64_t hi, uint64_t& a, uint64_t& b) {
+    a = lo & ~(1ULL << 63);
+    b = (lo >> 63) | (hi << 1);
+}
+GG_DEV uint32_t pair_hash(uint64_t a, uint64_t b) { return tab_hash64(a ^ (b * 0x9E3779B97F4A7C15ULL)); }
 
 // Insert one occurrence.  Returns 1 when this call claimed a new slot, 0 when
 // the key was present, 2 when no slot was found within min(mask+1,
@@ -146,6 +166,41 @@ GG_DEV uint32_t tab_insert64(KP keys, VP vals, uint32_t mask, uint64_t key, uint
     }
     atomicAdd((uint32_t*)&vals[i], bits & CNT_MASK);
     if (bits & ~CNT_MASK) atomicOr((uint32_t*)&vals[i], bits & ~CNT_MASK);
+    slot = i;
+    return claimed;
+}
+
+// Two-word keys, interleaved: a slot belongs to the first key whose first word
+// claims word 0 and whose second word then claims word 1.  Words only ever
+// change from EMPTY64 to their value, so a key that loses either claim moves
+// on and no lane waits for another; a slot costs one 16-byte read and, when
+// free, two compare-and-swaps.
+GG_DEV uint32_t tab_insert_pair(uint64_t* keys, uint32_t* vals, uint32_t mask, uint32_t h, uint64_t a, uint64_t b,
+                                uint32_t bits, uint32_t probe_limit, uint32_t& slot) {
+    uint32_t i = h & mask;
+    uint32_t claimed = 0;
+    for (uint32_t probes = 0;; probes++) {
+        if (probes > mask || probes >= probe_limit) return 2;
+        ulonglong2 cur = *reinterpret_cast<const ulonglong2*>(keys + 2 * i);
+        if (cur.x == EMPTY64) {
+            cur.x = atomicCAS((unsigned long long*)&keys[2 * i], (unsigned long long)EMPTY64, (unsigned long long)a);
+            if (cur.x == EMPTY64) cur.x = a;
+        }
+        if (cur.x == a) {
+            if (cur.y == EMPTY64) {
+                cur.y = atomicCAS((unsigned long long*)&keys[2 * i + 1], (unsigned long long)EMPTY64,
+                                  (unsigned long long)b);
+                if (cur.y == EMPTY64) {
+                    claimed = 1;
+                    break;
+                }
+            }
+            if (cur.y == b) break;
+        }
+        i = (i + 1) & mask;
+    }
+    atomicAdd(&vals[i], bits & CNT_MASK);
+    if (bits & ~CNT_MASK) atomicOr(&vals[i], bits & ~CNT_MASK);
     slot = i;
     return claimed;
 }
@@ -218,9 +273,21 @@ GG_DEV void rk_segment(const MergeArgs& A, const uint32_t* bw, uint32_t i0, uint
     }
 }
 
-// k-mers per segment when the k-mers of rabin-karp128 records are spread
-// over the threads of a workgroup (each segment starts from the table)
-constexpr uint32_t RK_SEG = 16;
+// Rabin-karp128 key of a k-mer from its 2-bit form (lo, hi): the sums of its
+// bases' terms, three bases per table entry (43 KB at k = 63: lines of one
+// group are shared by the lanes), and the smaller of the two; *swap when that
+// is the hash of the reverse complement.
+GG_DEV u128_t rk_of_kmer(const MergeArgs& A, uint64_t lo, uint64_t hi, bool* swap) {
+    u128_t x = ((u128_t)hi << 64) | lo, f = 0, b = 0;
+    for (uint32_t g = 0; 3 * g < A.k; g++) {
+        const u128_t* e = A.rk_tri + 2 * (64 * g + ((uint32_t)x & 63u));
+        f += e[0];
+        b += e[1];
+        x >>= 6;
+    }
+    *swap = f > b;
+    return f < b ? f : b;
+}
 
 // Iterate the k-mers of one slot; cb(lo, hi, is_forward, idx, last_idx).
 template <int MODE, class CB>
@@ -247,7 +314,7 @@ GG_DEV void for_each_kmer(const MergeArgs& A, const uint32_t* slot, CB&& cb) {
     const uint32_t k = A.k;
     if (len < k) return;
     const uint32_t last = len - k;
-    if (Mode<MODE>::seq64(A)) {
+    if (Mode<MODE>::FAST ? Mode<MODE>::TKW == 1 : A.kind == 0 && k <= 32) {
         const uint64_t mask = (k == 32) ? ~0ULL : ((1ULL << (2 * k)) - 1);
         uint64_t fw = 0, rc = 0;
         uint32_t word = 0;
@@ -258,7 +325,7 @@ GG_DEV void for_each_kmer(const MergeArgs& A, const uint32_t* slot, CB&& cb) {
             rc = ((rc << 2) | (c ^ 2)) & mask;
             if (i + 1 >= k) cb(fw < rc ? fw : rc, 0ULL, fw < rc, i + 1 - k, last);
         }
-    } else if (Mode<MODE>::seq128(A)) {
+    } else if (Mode<MODE>::FAST || A.kind == 0) {
         const u128_t mask = (k == 64) ? ~(u128_t)0 : (((u128_t)1 << (2 * k)) - 1);
         u128_t fw = 0, rc = 0;
         uint32_t word = 0;
@@ -308,12 +375,12 @@ GG_DEV void close_chunk(const MergeArgs& A, EmitState& es) {
     es.fill = 0;
 }
 
-// Emit solid entries among the table slots claimed by the entry (`claimed`,
-// n of them); cross-marked entries holding only one flag bit go to the
-// fixup list.  Wavefronts take 64 claimed slots at a time.
-template <int MODE, class KP, class SP, class VP>
-GG_DEV void emit_solid(const MergeArgs& A, uint32_t sub, KP klo, KP khi, SP st, VP vals, const uint32_t* cbits,
-                       const uint16_t* claimed, uint32_t n, EmitState& es) {
+// Emit solid entries among the table slots listed in `claimed` (n of them);
+// cross-marked entries holding only one flag bit go to the fixup list.
+// Wavefronts take 64 listed slots at a time.
+template <int MODE>
+GG_DEV void emit_solid(const MergeArgs& A, uint32_t sub, const uint64_t* klo, const uint64_t* khi, const uint32_t* st,
+                       const uint32_t* vals, const uint32_t* cbits, const uint16_t* claimed, uint32_t n, EmitState& es) {
     const uint32_t W = Mode<MODE>::color_words(A), KW = Mode<MODE>::key_words(A);
     const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const uint64_t below = (1ULL << lane) - 1;
@@ -323,7 +390,7 @@ GG_DEV void emit_solid(const MergeArgs& A, uint32_t sub, KP klo, KP khi, SP st, 
         bool solid = false, fix = false;
         uint32_t outv = 0;
         if (j < n) {
-            bool occupied = (KW == 1) ? (klo[i] != EMPTY64) : (st[i] == 2);
+            bool occupied = Mode<MODE>::FAST || ((KW == 1) ? (klo[i] != EMPTY64) : (st[i] == 2));
             if (occupied) {
                 uint32_t v = vals[i];
                 uint32_t cnt = v & CNT_MASK, fl = v >> 30;
@@ -331,6 +398,25 @@ GG_DEV void emit_solid(const MergeArgs& A, uint32_t sub, KP klo, KP khi, SP st, 
                 solid = mult >= A.min_mult;
                 fix = solid && (v & VAL_CROSS) && (fl == 1 || fl == 2);
                 outv = mult | (fl << 30);
+            }
+        }
+        uint64_t lo = 0, hi = 0;
+        if (solid) {
+            if (Mode<MODE>::FAST && Mode<MODE>::TKW == 2) {
+                const uint64_t a = klo[2 * i], b = klo[2 * i + 1];
+                lo = a | (b << 63);
+                hi = b >> 1;
+            } else {
+                lo = klo[i];
+                if (!Mode<MODE>::FAST && KW == 2) hi = khi[i];
+            }
+            if (Mode<MODE>::RK) {
+                bool swap;
+                const u128_t key = rk_of_kmer(A, lo, hi, &swap);
+                lo = (uint64_t)key;
+                hi = (uint64_t)(key >> 64);
+                // the flags face the hash's strand
+                if (swap) outv = (outv & 0x3FFFFFFFu) | ((outv >> 31) << 30) | ((outv & (1u << 30)) << 1);
             }
         }
         const bool main = solid && !fix;
@@ -346,10 +432,10 @@ GG_DEV void emit_solid(const MergeArgs& A, uint32_t sub, KP klo, KP khi, SP st, 
             if (main && es.chunk < A.n_chunks) {
                 const uint64_t pos = (uint64_t)es.chunk * OUT_CHUNK + es.fill + __popcll(bal & below);
                 if (KW == 1) {
-                    A.out_key[pos] = klo[i];
+                    A.out_key[pos] = lo;
                 } else {
-                    A.out_key[2 * pos] = klo[i];
-                    A.out_key[2 * pos + 1] = khi[i];
+                    A.out_key[2 * pos] = lo;
+                    A.out_key[2 * pos + 1] = hi;
                 }
                 A.out_val[pos] = outv;
                 A.out_sub[pos] = sub;
@@ -365,10 +451,10 @@ GG_DEV void emit_solid(const MergeArgs& A, uint32_t sub, KP klo, KP khi, SP st, 
                 uint64_t pos = basef + __popcll(balf & below);
                 if (pos < A.fix_cap) {
                     if (KW == 1) {
-                        A.fix_key[pos] = klo[i];
+                        A.fix_key[pos] = lo;
                     } else {
-                        A.fix_key[2 * pos] = klo[i];
-                        A.fix_key[2 * pos + 1] = khi[i];
+                        A.fix_key[2 * pos] = lo;
+                        A.fix_key[2 * pos + 1] = hi;
                     }
                     A.fix_val[pos] = outv;
                     A.fix_sub[pos] = sub;
@@ -379,15 +465,39 @@ GG_DEV void emit_solid(const MergeArgs& A, uint32_t sub, KP klo, KP khi, SP st, 
     }
 }
 
+// rabin-karp128 variants: the slots of `claimed` holding solid entries, listed
+// in `solid` (at most n), so that the hashes are formed by full wavefronts.
+// Returns how many.
+GG_DEV uint32_t list_solid(const MergeArgs& A, const uint32_t* vals, const uint16_t* claimed, uint32_t n,
+                           uint16_t* solid, uint32_t* n_solid) {
+    const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    for (uint32_t i0 = wave * 64; i0 < n; i0 += blockDim.x) {
+        const uint32_t j = i0 + lane;
+        const uint32_t i = j < n ? claimed[j] : 0u;
+        bool is = false;
+        if (j < n) {
+            const uint32_t v = vals[i];
+            is = ((v & CNT_MASK) >> ((v >> 30) == 3 ? 1 : 0)) >= A.min_mult;
+        }
+        const uint64_t bal = __ballot(is);
+        if (!bal) continue;
+        uint32_t base = 0;
+        if (lane == 0) base = atomicAdd(n_solid, (uint32_t)__popcll(bal));
+        base = __shfl(base, 0);
+        if (is) solid[base + (uint32_t)__popcll(bal & ((1ULL << lane) - 1))] = (uint16_t)i;
+    }
+    __syncthreads();
+    return *n_solid;
+}
+
 // Inserts every occurrence of the item's records whose k-mer lies in the
 // work entry's partition (bits 16.. of the table hash; the slot index uses
 // the low bits).  An insert that needs more than `probe_limit` probes sets
 // *overflow and insertion stops (the entry is then redone as finer parts).
-template <int MODE, class KP, class SP, class VP>
-GG_DEV void insert_item(const MergeArgs& A, uint64_t r0, uint64_t r1, const PartWork& w, KP klo, KP khi, SP st,
-                        VP vals, uint32_t* cbits, uint32_t mask, uint32_t probe_limit, uint32_t* overflow,
+GG_DEV void insert_item(const MergeArgs& A, uint64_t r0, uint64_t r1, const PartWork& w, uint64_t* klo, uint64_t* khi,
+                        uint32_t* st, uint32_t* vals, uint32_t* cbits, uint32_t mask, uint32_t probe_limit, uint32_t* overflow,
                         uint16_t* claimed, uint32_t* n_claimed) {
-    const uint32_t W = Mode<MODE>::color_words(A), KW = Mode<MODE>::key_words(A);
+    const uint32_t W = A.color_words, KW = A.key_words;
     const uint32_t SW = A.slot_words;
     const uint32_t part_mask = (1u << w.log_parts) - 1;
     for (uint64_t r = r0 + threadIdx.x; r < r1; r += blockDim.x) {
@@ -395,7 +505,7 @@ GG_DEV void insert_item(const MergeArgs& A, uint64_t r0, uint64_t r1, const Part
         const uint32_t meta = slot[0];
         const uint32_t color = W ? A.slot_color[r] : 0u;
         const uint32_t extra = meta_mult(meta) - 1;  // identical copies stored once
-        for_each_kmer<MODE>(A, slot, [&](uint64_t lo, uint64_t hi, bool is_fwd, uint32_t idx, uint32_t last) {
+        for_each_kmer<0>(A, slot, [&](uint64_t lo, uint64_t hi, bool is_fwd, uint32_t idx, uint32_t last) {
             if (*(volatile uint32_t*)overflow) return;
             if (part_mask) {
                 const uint32_t h = (KW == 1) ? tab_hash64(lo) : hash128(lo, hi);
@@ -415,18 +525,19 @@ GG_DEV void insert_item(const MergeArgs& A, uint64_t r0, uint64_t r1, const Part
     }
 }
 
-// ---- identical-record path (seq-hash keys, k <= 32) -----------------------
+// ---- identical-record path -------------------------------------------------
 // The reference merges identical super-k-mers of a bucket before counting
 // (crates/minimizer_bucketing/src/compactor.rs:128-196, multiplicities
 // summed, :159-163); counting each distinct record once with its multiplicity
 // gives the same MapEntries.  Records are keyed by their whole slot (meta
 // word with length, flags, minimizer position and cross marks, then the
 // packed bases) plus their color; a record the table cannot take is counted
-// on its own.  After deduplication every thread takes k-mer positions of the
-// distinct records, so the k-mer work is spread evenly over the workgroup.
+// on its own.  After deduplication every thread takes k-mers of the distinct
+// records (MODE != 0), so the k-mer work is spread evenly over the workgroup.
 // Record table slots (a power of two, 16..512); chunks of rec_cap / 2
-// records are deduplicated at a time.
-constexpr uint32_t REC_CAP_DEFAULT = 512;
+// records are deduplicated at a time.  Slots of 8 words take 256: 512 would
+// cost the 128-bit variants one of the four workgroups a CU's LDS holds.
+__host__ __device__ inline uint32_t rec_cap_default(uint32_t slot_words) { return slot_words <= 4 ? 512 : 256; }
 
 struct RecTable {
     uint32_t* key;  // rec_cap * SW
@@ -434,7 +545,7 @@ struct RecTable {
     uint32_t* state;  // 0 free, 1 being written, 2 ready
     uint32_t* col;
     uint32_t* n;  // [1]: k-mers of the chunk, [2..5]: wave totals of the scan
-    uint16_t* rec_of;  // each k-mer position of the chunk: record slot << 7 | k-mer index in the record
+    uint16_t* rec_of;  // each segment of SEG k-mers of the chunk: record slot << 7 | index of the segment in the record
 };
 
 // k-mers of one inline record at most.
@@ -451,23 +562,21 @@ GG_DEV RecTable rec_table(const MergeArgs& A, uint8_t* lds) {
     b += A.rec_cap;
     R.state = b;
     b += A.rec_cap;
-    R.col = b;
-    b += A.rec_cap;
+    R.col = b;  // colored builds only
+    if (A.color_words) b += A.rec_cap;
     R.n = b;
     b += 6;
     R.rec_of = reinterpret_cast<uint16_t*>(b);
     return R;
 }
 
-// Bytes of dynamic LDS the record table needs (k = 0xFFFF: no per-k-mer tags,
-// the rolling mode of 128-bit keys).
-// With rk_seg the tags are per segment of RK_SEG k-mers, for up to rec_cap
-// records (the uncolored rabin-karp128 variant).
-__host__ __device__ inline uint32_t rec_table_bytes(uint32_t slot_words, uint32_t k, uint32_t rec_cap,
-                                                    bool rk_seg = false) {
-    const uint32_t tags = rk_seg ? rec_cap * ((rec_max_kmers(slot_words, k) + RK_SEG - 1) / RK_SEG)
-                                 : (rec_cap / 2) * rec_max_kmers(slot_words, k);
-    return (rec_cap * slot_words + 3 * rec_cap + 6) * 4 + tags * 2 + 4;
+// Bytes of dynamic LDS the record table needs; seg = 0: no tags (MODE 0).
+// The tags' place also takes the list of the entry's solid slots (list_solid),
+// at most `solid` of them.
+__host__ __device__ inline uint32_t rec_table_bytes(uint32_t slot_words, uint32_t k, uint32_t rec_cap, uint32_t seg,
+                                                    bool colors, uint32_t solid) {
+    const uint32_t tags = seg ? (rec_cap / 2) * ((rec_max_kmers(slot_words, k) + seg - 1) / seg) : 0;
+    return (rec_cap * slot_words + (colors ? 3 : 2) * rec_cap + 6) * 4 + (tags > solid ? tags : solid) * 2 + 4;
 }
 
 GG_DEV uint32_t rec_hash(const uint32_t* w, uint32_t sw, uint32_t color) {
@@ -475,6 +584,15 @@ GG_DEV uint32_t rec_hash(const uint32_t* w, uint32_t sw, uint32_t color) {
     for (uint32_t i = 0; i < sw; i++) h = (h ^ w[i]) * 0xbf58476d1ce4e5b9ULL;
     h ^= h >> 31;
     return (uint32_t)h;
+}
+
+// Reverse complement of a 2-bit k-mer (k <= 32): complement every base,
+// reverse the 2-bit groups.
+GG_DEV uint64_t kmer_rc64(uint64_t fw, uint32_t k) {
+    uint64_t x = fw ^ 0xAAAAAAAAAAAAAAAAULL;
+    x = ((uint64_t)__brev((uint32_t)x) << 32) | __brev((uint32_t)(x >> 32));
+    x = ((x >> 1) & 0x5555555555555555ULL) | ((x & 0x5555555555555555ULL) << 1);
+    return x >> (64 - 2 * k);
 }
 
 // Canonical 2-bit k-mer (k <= 32) at base offset i of packed words (16 bases
@@ -486,39 +604,72 @@ GG_DEV uint64_t kmer_at(const uint32_t* bw, uint32_t i, uint32_t k, bool* fwd) {
     uint64_t fw = sh ? (lo >> sh) | ((uint64_t)bw[wi + 2] << (64 - sh)) : lo;
     const uint64_t mask = (k == 32) ? ~0ULL : ((1ULL << (2 * k)) - 1);
     fw &= mask;
-    // reverse complement: complement every base, reverse the 2-bit groups
-    uint64_t x = fw ^ 0xAAAAAAAAAAAAAAAAULL;
-    x = ((uint64_t)__brev((uint32_t)x) << 32) | __brev((uint32_t)(x >> 32));
-    x = ((x >> 1) & 0x5555555555555555ULL) | ((x & 0x5555555555555555ULL) << 1);
-    const uint64_t rc = x >> (64 - 2 * k);
+    const uint64_t rc = kmer_rc64(fw, k);
     *fwd = fw < rc;
     return fw < rc ? fw : rc;
 }
 
-template <int MODE, class KP, class SP, class VP>
-GG_DEV void insert_item_dedup(const MergeArgs& A, uint64_t r0, uint64_t r1, const PartWork& w, KP klo, KP khi, SP st,
-                              VP vals, uint32_t* cbits, uint32_t mask, uint32_t probe_limit, uint32_t* overflow,
+// Both strands of the k-mer (32 < k < 64) at base offset i of packed words, as
+// their 2-bit forms.
+GG_DEV void kmer_pair_at(const uint32_t* bw, uint32_t i, uint32_t k, u128_t* fw, u128_t* rc) {
+    const uint32_t wi = i >> 4, sh = (i & 15) * 2;
+    const u128_t w03 = (u128_t)((uint64_t)bw[wi] | ((uint64_t)bw[wi + 1] << 32)) |
+                       ((u128_t)((uint64_t)bw[wi + 2] | ((uint64_t)bw[wi + 3] << 32)) << 64);
+    const u128_t mask = ((u128_t)1 << (2 * k)) - 1;
+    u128_t x = w03 >> sh;
+    // the fifth word is only read when the k-mer reaches into it
+    if (sh + 2 * k > 128) x |= (u128_t)bw[wi + 4] << (128 - sh);
+    x &= mask;
+    *fw = x;
+    constexpr uint64_t AA = 0xAAAAAAAAAAAAAAAAULL, M5 = 0x5555555555555555ULL;
+    const uint64_t xl = (uint64_t)x ^ AA, xh = (uint64_t)(x >> 64) ^ AA;
+    uint64_t l = ((uint64_t)__brev((uint32_t)xh) << 32) | __brev((uint32_t)(xh >> 32));
+    uint64_t h = ((uint64_t)__brev((uint32_t)xl) << 32) | __brev((uint32_t)(xl >> 32));
+    l = ((l >> 1) & M5) | ((l & M5) << 1);
+    h = ((h >> 1) & M5) | ((h & M5) << 1);
+    *rc = (((u128_t)h << 64) | l) >> (128 - 2 * k);
+}
+
+template <int MODE>
+GG_DEV void insert_item_dedup(const MergeArgs& A, uint64_t r0, uint64_t r1, const PartWork& w, uint64_t* klo,
+                              uint64_t* khi, uint32_t* st, uint32_t* vals, uint32_t* cbits, uint32_t mask, uint32_t probe_limit, uint32_t* overflow,
                               uint16_t* claimed, uint32_t* n_claimed, const RecTable& R, const uint32_t* pre,
                               uint32_t pre_color, bool hashed) {
+    constexpr bool FAST = Mode<MODE>::FAST;
+    constexpr uint32_t SEG = Mode<MODE>::SEG;
     const uint32_t W = Mode<MODE>::color_words(A), KW = Mode<MODE>::key_words(A);
     const uint32_t SW = Mode<MODE>::slot_words(A), k = A.k, RC = A.rec_cap;
     const uint32_t part_mask = (1u << w.log_parts) - 1;
     // one occurrence (or cnt identical ones) of a k-mer of either key width
-    auto insert_key = [&](uint64_t lo, uint64_t hi, uint32_t bits, uint32_t color) {
-        if (*(volatile uint32_t*)overflow) return;
-        if (part_mask) {
-            const uint32_t h = (KW == 1) ? tab_hash64(lo) : hash128(lo, hi);
-            if (((h >> 16) & part_mask) != w.part) return;
+    // returns whether it claimed table slot `at`
+    auto insert_one = [&](uint64_t lo, uint64_t hi, uint32_t bits, uint32_t color, uint32_t& at) -> bool {
+        uint32_t res;
+        if (FAST && Mode<MODE>::TKW == 2) {
+            uint64_t a, b;
+            pair_of(lo, hi, a, b);
+            const uint32_t h = pair_hash(a, b);
+            if (part_mask && ((h >> 16) & part_mask) != w.part) return false;
+            res = tab_insert_pair(klo, vals, mask, h, a, b, bits, probe_limit, at);
+        } else {
+            const bool one = FAST || KW == 1;
+            if (part_mask) {
+                const uint32_t h = one ? tab_hash64(lo) : hash128(lo, hi);
+                if (((h >> 16) & part_mask) != w.part) return false;
+            }
+            res = one ? tab_insert64(klo, vals, mask, lo, bits, probe_limit, at)
+                      : tab_insert128(klo, khi, st, vals, mask, lo, hi, bits, probe_limit, at);
         }
-        uint32_t at = 0;
-        const uint32_t res = (KW == 1) ? tab_insert64(klo, vals, mask, lo, bits, probe_limit, at)
-                                                : tab_insert128(klo, khi, st, vals, mask, lo, hi, bits, probe_limit, at);
         if (res == 2) {
             atomicOr(overflow, 1u);
-            return;
+            return false;
         }
-        if (res == 1) claimed[atomicAdd(n_claimed, 1u)] = (uint16_t)at;
         if (W) atomicOr(&cbits[at * W + (color >> 5)], 1u << (color & 31));
+        return res == 1;
+    };
+    auto insert_key = [&](uint64_t lo, uint64_t hi, uint32_t bits, uint32_t color) {
+        if (*(volatile uint32_t*)overflow) return;
+        uint32_t at = 0;
+        if (insert_one(lo, hi, bits, color, at)) claimed[atomicAdd(n_claimed, 1u)] = (uint16_t)at;
     };
     // the record table's states are all free here (cleared at kernel start
     // and by phase B of the previous chunk)
@@ -538,7 +689,7 @@ GG_DEV void insert_item_dedup(const MergeArgs& A, uint64_t r0, uint64_t r1, cons
             // <= min(rec_cap, blockDim); both powers of two)
             const uint32_t i = RC > blockDim.x ? threadIdx.x * (RC / blockDim.x) : threadIdx.x;
             for (uint32_t q = 0; q < SW; q++) R.key[i * SW + q] = pre[q];
-            R.col[i] = color;
+            if (W) R.col[i] = color;
             R.cnt[i] = meta_mult(meta);
             R.state[i] = 2;
         } else if (!direct) {
@@ -552,14 +703,14 @@ GG_DEV void insert_item_dedup(const MergeArgs& A, uint64_t r0, uint64_t r1, cons
                 if (sv == 0) {
                     if (atomicCAS(&R.state[i], 0u, 1u) == 0u) {
                         for (uint32_t q = 0; q < SW; q++) R.key[i * SW + q] = wv[q];
-                        R.col[i] = color;
+                        if (W) R.col[i] = color;
                         R.cnt[i] = meta_mult(meta);
                         __threadfence_block();
                         atomicExch(&R.state[i], 2u);
                         done = true;
                     }
                 } else if (sv == 2) {
-                    bool eq = R.col[i] == color;
+                    bool eq = !W || R.col[i] == color;
                     for (uint32_t q = 0; q < SW && eq; q++) eq = R.key[i * SW + q] == wv[q];
                     if (eq) {
                         atomicAdd(&R.cnt[i], meta_mult(meta));
@@ -585,9 +736,9 @@ GG_DEV void insert_item_dedup(const MergeArgs& A, uint64_t r0, uint64_t r1, cons
     }
 phase_a_done:
     __syncthreads();
-    if (!Mode<MODE>::tag_kmers(A) && MODE != 2) {
-        // 128-bit keys: each thread rolls the k-mers of the distinct records
-        // in its table slots (rec_cap / blockDim of them) and frees the slots
+    if (!FAST) {
+        // each thread rolls the k-mers of the distinct records in its table
+        // slots (rec_cap / blockDim of them) and frees the slots
         const uint32_t per = RC > blockDim.x ? RC / blockDim.x : 1u;
         const uint32_t s0 = threadIdx.x * per;
         for (uint32_t q = 0; q < per; q++) {
@@ -602,12 +753,11 @@ phase_a_done:
         }
         return;
     }
-    // phase B: one exclusive scan over the table slots of their k-mer counts
-    // places the distinct records' k-mers (each position tagged with its
-    // record's slot and k-mer index; the rabin-karp128 variant tags segments
-    // of RK_SEG k-mers with their index instead); each thread owns
-    // rec_cap / blockDim consecutive slots (at least one) and frees them for
-    // the next chunk once read.
+    // phase B: one exclusive scan over the table slots of their segment counts
+    // places the distinct records' segments of SEG k-mers (each tagged with its
+    // record's slot and its index there); each thread owns rec_cap / blockDim
+    // consecutive slots (at least one) and frees them for the next chunk once
+    // read.
     {
         const uint32_t per = RC > blockDim.x ? RC / blockDim.x : 1u;
         const uint32_t s0 = threadIdx.x * per;
@@ -619,7 +769,7 @@ phase_a_done:
             if (si < RC && R.state[si] == 2) {
                 const uint32_t len = meta_len(R.key[si * SW]);
                 const uint32_t nk = len >= k ? len - k + 1 : 0u;
-                pk[q] = MODE == 2 ? (nk + RK_SEG - 1) / RK_SEG : nk;
+                pk[q] = (nk + SEG - 1) / SEG;
                 R.state[si] = 0;
             }
             mine += pk[q];
@@ -649,54 +799,79 @@ phase_a_done:
         if (threadIdx.x == 0) R.n[1] = all;
         __syncthreads();
     }
-    // phase B2: every k-mer of the distinct records, one per thread (the
-    // rabin-karp128 variant: one segment of RK_SEG k-mers per thread)
+    // phase B2: every segment of SEG k-mers of the distinct records, one per
+    // thread; the first k-mer is extracted, the others rolled from it
     const uint32_t total = R.n[1];
     for (uint32_t j0 = 0; j0 < total; j0 += blockDim.x) {
         const uint32_t j = j0 + threadIdx.x;
-        if (MODE == 2) {
-            if (j < total) {
-                const uint32_t v = R.rec_of[j];
-                const uint32_t si = v >> 7, i0 = (v & 127u) * RK_SEG;
-                const uint32_t* rw = R.key + si * SW;
-                const uint32_t cnt = R.cnt[si], meta = rw[0], last = meta_len(meta) - k;
-                const uint32_t i1 = i0 + RK_SEG < last + 1 ? i0 + RK_SEG : last + 1;
-                rk_segment(A, rw + 1, i0, i1, [&](uint64_t lo, uint64_t hi, bool fwd, uint32_t x) {
-                    insert_key(lo, hi, occurrence_bits(meta, fwd, x, last) - 1u + cnt, 0u);
-                });
-            }
-            continue;
-        }
-        bool cl = false;
-        uint32_t at = 0;
+        uint32_t cnt = 0, color = 0, meta = 0, last = 0, i0 = 0, n = 0;
+        const uint32_t* bw = R.key + 1;
         if (j < total) {
             const uint32_t v = R.rec_of[j];
-            const uint32_t si = v >> 7, i = v & 127u;
-            const uint32_t* rw = R.key + si * SW;
-            const uint32_t cnt = R.cnt[si], color = W ? R.col[si] : 0u;
-            const uint32_t meta = rw[0];
-            const uint32_t len = meta_len(meta);
-            bool fwd;
-            const uint64_t key = kmer_at(rw + 1, i, k, &fwd);
-            const uint32_t bits = occurrence_bits(meta, fwd, i, len - k) - 1u + cnt;
-            if (!part_mask || ((tab_hash64(key) >> 16) & part_mask) == w.part) {
-                const uint32_t res = tab_insert64(klo, vals, mask, key, bits, probe_limit, at);
-                if (res == 2) {
-                    atomicOr(overflow, 1u);
+            const uint32_t si = v >> 7;
+            i0 = (v & 127u) * SEG;
+            bw = R.key + si * SW + 1;
+            cnt = R.cnt[si];
+            color = W ? R.col[si] : 0u;
+            meta = bw[-1];
+            last = meta_len(meta) - k;
+            n = last + 1 - i0 < SEG ? last + 1 - i0 : SEG;
+        }
+        u128_t fw2 = 0, rc2 = 0;
+        uint64_t fw1 = 0, rc1 = 0, next = 0;  // next: the segment's bases behind its first k-mer, 2 bits each
+        if (SEG > 1 && n) {
+            if (Mode<MODE>::TKW == 2) {
+                kmer_pair_at(bw, i0, k, &fw2, &rc2);
+            } else {
+                bool fwd;
+                const uint64_t c = kmer_at(bw, i0, k, &fwd);
+                const uint64_t o = kmer_rc64(c, k);
+                fw1 = fwd ? c : o;
+                rc1 = fwd ? o : c;
+            }
+            const uint32_t nb = i0 + k;  // SEG - 1 <= 16 more bases: two words (the record's words end in the table)
+            next = ((uint64_t)bw[nb >> 4] | ((uint64_t)bw[(nb >> 4) + 1] << 32)) >> (2 * (nb & 15));
+        }
+#pragma unroll
+        for (uint32_t x = 0; x < SEG; x++) {
+            bool cl = false;
+            uint32_t at = 0;
+            if (x < n) {
+                uint64_t lo, hi = 0;
+                bool fwd;
+                if (Mode<MODE>::TKW == 2) {
+                    fwd = fw2 < rc2;
+                    const u128_t key = fwd ? fw2 : rc2;
+                    lo = (uint64_t)key;
+                    hi = (uint64_t)(key >> 64);
+                } else if (SEG > 1) {
+                    fwd = fw1 < rc1;
+                    lo = fwd ? fw1 : rc1;
                 } else {
-                    cl = res == 1;
-                    if (W) atomicOr(&cbits[at * W + (color >> 5)], 1u << (color & 31));
+                    lo = kmer_at(bw, i0, k, &fwd);
+                }
+                cl = insert_one(lo, hi, occurrence_bits(meta, fwd, i0 + x, last) - 1u + cnt, color, at);
+            }
+            if (SEG > 1) {
+                const uint64_t c = next & 3u;
+                next >>= 2;
+                if (Mode<MODE>::TKW == 2) {
+                    fw2 = (fw2 >> 2) | ((u128_t)c << (2 * (k - 1)));
+                    rc2 = ((rc2 << 2) | (c ^ 2)) & (((u128_t)1 << (2 * k)) - 1);
+                } else {
+                    fw1 = (fw1 >> 2) | (c << (2 * (k - 1)));
+                    rc1 = ((rc1 << 2) | (c ^ 2)) & (k == 32 ? ~0ULL : (1ULL << (2 * k)) - 1);
                 }
             }
-        }
-        // one LDS atomic per wavefront for the slots it claimed
-        const uint64_t bal = __ballot(cl);
-        if (bal) {
-            const uint32_t lane = threadIdx.x & 63, first = (uint32_t)__builtin_ctzll(bal);
-            uint32_t base = 0;
-            if (lane == first) base = atomicAdd(n_claimed, (uint32_t)__popcll(bal));
-            base = __shfl(base, (int)first);
-            if (cl) claimed[base + (uint32_t)__popcll(bal & ((1ULL << lane) - 1))] = (uint16_t)at;
+            // one LDS atomic per wavefront for the slots it claimed
+            const uint64_t bal = __ballot(cl);
+            if (bal) {
+                const uint32_t lane = threadIdx.x & 63, first = (uint32_t)__builtin_ctzll(bal);
+                uint32_t base = 0;
+                if (lane == first) base = atomicAdd(n_claimed, (uint32_t)__popcll(bal));
+                base = __shfl(base, (int)first);
+                if (cl) claimed[base + (uint32_t)__popcll(bal & ((1ULL << lane) - 1))] = (uint16_t)at;
+            }
         }
     }
 }
@@ -742,21 +917,26 @@ GG_DEV void merge_lds_body(const MergeArgs& A) {
     __shared__ Fetched s_cur;
     EmitState es{~0u, 0u};
     const uint32_t cap_max = A.lds_cap;  // the host allocates this many entries plus a margin
+    // key words per table entry, then the counters; MODE 0 keeps 128-bit keys
+    // in two arrays with a state word per slot behind the counters
+    constexpr bool FAST = Mode<MODE>::FAST;
+    const uint32_t KW = FAST ? Mode<MODE>::TKW : A.key_words;
     uint64_t* klo = reinterpret_cast<uint64_t*>(lds);
-    uint64_t* khi = klo + cap_max;  // only used for 128-bit keys
-    const uint32_t KW = Mode<MODE>::key_words(A);
+    uint64_t* khi = klo + cap_max;
     uint32_t* vals = reinterpret_cast<uint32_t*>(lds + (size_t)cap_max * 8 * KW);
-    uint32_t* st = vals + cap_max;  // only used for 128-bit keys
-    uint32_t* cbits = vals + (size_t)cap_max * KW;  // color_words per entry (colored builds)
+    uint32_t* st = vals + cap_max;
+    uint32_t* cbits = vals + (size_t)cap_max * (FAST ? 1 : KW);  // color_words per entry (colored builds)
     const uint32_t W = Mode<MODE>::color_words(A);
     uint16_t* claimed = reinterpret_cast<uint16_t*>(cbits + (size_t)cap_max * W);  // slots claimed by the entry
+    __shared__ uint32_t s_solid;
     __shared__ uint32_t s_claimed;
     const bool leader = threadIdx.x == 0;
     // the table starts empty; afterwards only claimed slots are reset
     for (uint32_t i = threadIdx.x; i < cap_max; i += blockDim.x) {
         klo[i] = EMPTY64;
+        if (FAST && KW == 2) klo[cap_max + i] = EMPTY64;
         vals[i] = 0;
-        if (KW == 2) st[i] = 0;
+        if (!FAST && KW == 2) st[i] = 0;
     }
     for (uint32_t i = threadIdx.x; i < cap_max * W; i += blockDim.x) cbits[i] = 0;
     if (Mode<MODE>::dedup(A)) {
@@ -771,14 +951,18 @@ GG_DEV void merge_lds_body(const MergeArgs& A) {
     auto load_rec = [&](uint64_t r, uint64_t r_end, uint32_t* wv, uint32_t& col) {
         if (threadIdx.x < chunk && r < r_end) {
             const uint32_t* sp = A.slots + r * SW;
-            if (SW == 4) {
-                const uint4 v = *reinterpret_cast<const uint4*>(sp);
-                wv[0] = v.x;
-                wv[1] = v.y;
-                wv[2] = v.z;
-                wv[3] = v.w;
-            } else {
-                for (uint32_t q = 0; q < SW; q++) wv[q] = sp[q];
+            // slots of 4 or 8 words, 16-byte aligned
+            const uint4 v = *reinterpret_cast<const uint4*>(sp);
+            wv[0] = v.x;
+            wv[1] = v.y;
+            wv[2] = v.z;
+            wv[3] = v.w;
+            if (MSW == 8 && SW == 8) {
+                const uint4 u = *reinterpret_cast<const uint4*>(sp + 4);
+                wv[4] = u.x;
+                wv[5] = u.y;
+                wv[6] = u.z;
+                wv[7] = u.w;
             }
             col = W ? A.slot_color[r] : 0u;
         }
@@ -787,6 +971,7 @@ GG_DEV void merge_lds_body(const MergeArgs& A) {
     Pipe pp{};
     if (leader) {
         s_claimed = 0;
+        s_solid = 0;
         pp.bat = pp.bat_end = 0;
         pp.n1.e = pipe_claim(A, pp);
         pipe_part(A, pp);
@@ -825,12 +1010,10 @@ GG_DEV void merge_lds_body(const MergeArgs& A) {
             // factor stays at most one half), one record per thread; identical
             // records of one chunk are counted once, the k-mer table
             // accumulates over the chunks.  Each thread's record of the next
-            // chunk is loaded while the current chunk is processed.  Records
-            // placed by position without per-k-mer tags (each distinct record
-            // rolled by one thread) fill the whole record table: one record
-            // per thread of the workgroup.
-            chunk = (hashed || Mode<MODE>::tag_kmers(A)) ? A.rec_cap / 2
-                                                         : (A.rec_cap < blockDim.x ? A.rec_cap : blockDim.x);
+            // chunk is loaded while the current chunk is processed.  Without
+            // segment tags (MODE 0) records placed by position fill the whole
+            // record table: one record per thread of the workgroup.
+            chunk = (hashed || FAST) ? A.rec_cap / 2 : (A.rec_cap < blockDim.x ? A.rec_cap : blockDim.x);
             load_rec(it.r0 + threadIdx.x, it.r1, cw, ccol);
             for (uint64_t c0 = it.r0; c0 < it.r1; c0 += chunk) {
                 const uint64_t c1 = c0 + chunk < it.r1 ? c0 + chunk : it.r1;
@@ -844,7 +1027,7 @@ GG_DEV void merge_lds_body(const MergeArgs& A) {
                 __syncthreads();  // the next chunk reuses the record table
             }
         } else {
-            insert_item<MODE>(A, it.r0, it.r1, w, klo, khi, st, vals, cbits, mask, 96u, &s_overflow, claimed, &s_claimed);
+            insert_item(A, it.r0, it.r1, w, klo, khi, st, vals, cbits, mask, 96u, &s_overflow, claimed, &s_claimed);
         }
         if (leader) pipe_item(A, pp);
         __syncthreads();
@@ -853,17 +1036,31 @@ GG_DEV void merge_lds_body(const MergeArgs& A) {
             // more distinct k-mers than the table holds: redone as finer parts
             if (leader) A.redo[atomicAdd(A.redo_count, 1u)] = PartWork{w.item, w.part, w.log_parts, it.occ};
         } else {
-            emit_solid<MODE>(A, it.sub, klo, khi, st, vals, cbits, claimed, n_cl, es);
+            if constexpr (Mode<MODE>::RK) {
+                uint16_t* solid = rec_table(A, lds).rec_of;
+                const uint32_t n = list_solid(A, vals, claimed, n_cl, solid, &s_solid);
+                emit_solid<MODE>(A, it.sub, klo, khi, st, vals, cbits, solid, n, es);
+            } else {
+                emit_solid<MODE>(A, it.sub, klo, khi, st, vals, cbits, claimed, n_cl, es);
+            }
         }
         __syncthreads();
         for (uint32_t j = threadIdx.x; j < n_cl; j += blockDim.x) {
             const uint32_t i = claimed[j];
-            klo[i] = EMPTY64;
+            if (FAST && KW == 2) {
+                klo[2 * i] = EMPTY64;
+                klo[2 * i + 1] = EMPTY64;
+            } else {
+                klo[i] = EMPTY64;
+            }
             vals[i] = 0;
-            if (KW == 2) st[i] = 0;
+            if (!FAST && KW == 2) st[i] = 0;
             for (uint32_t q = 0; q < W; q++) cbits[i * W + q] = 0;
         }
-        if (leader) s_claimed = 0;
+        if (leader) {
+            s_claimed = 0;
+            s_solid = 0;
+        }
         __syncthreads();
     }
     close_chunk(A, es);
@@ -875,7 +1072,14 @@ __global__ __launch_bounds__(256) void merge_lds_kernel(MergeArgs A) { merge_lds
 // the LDS tables allow that many workgroups.
 __global__ __launch_bounds__(256, 8) void merge_lds_seq64_kernel(MergeArgs A) { merge_lds_body<1>(A); }
 
-__global__ __launch_bounds__(256) void merge_lds_rk128_kernel(MergeArgs A) { merge_lds_body<2>(A); }
+// The other variants: up to 128 VGPRs, for the four workgroups that a CU's LDS
+// holds with their tables.
+__global__ __launch_bounds__(256, 4) void merge_lds_seq64w_kernel(MergeArgs A) { merge_lds_body<2>(A); }
+__global__ __launch_bounds__(256, 4) void merge_lds_rk64_kernel(MergeArgs A) { merge_lds_body<3>(A); }
+__global__ __launch_bounds__(256, 4) void merge_lds_seq128_kernel(MergeArgs A) { merge_lds_body<4>(A); }
+__global__ __launch_bounds__(256, 4) void merge_lds_rk128_kernel(MergeArgs A) { merge_lds_body<5>(A); }
+__global__ __launch_bounds__(256, 4) void merge_lds_col64_kernel(MergeArgs A) { merge_lds_body<6>(A); }
+__global__ __launch_bounds__(256, 4) void merge_lds_col128_kernel(MergeArgs A) { merge_lds_body<7>(A); }
 
 // Makes the solid table dense: with T = off[n_chunks] entries in all (off: the
 // exclusive scan of the chunks' fill counts), the entries at positions >= T
