@@ -503,13 +503,13 @@ int ggcat_gpu_bucketing(ggcat_gpu_ctx* ctx, const uint8_t* data, uint64_t n_byte
     ctx->P = p;
     const uint32_t w = p.k - p.m;
     const uint32_t n_sub = ((1u << p.buckets_log) + 1) << p.second_buckets_log;
-    // physical units: about `unit_bytes` input bytes per unit (default 2000,
-    // 1000 for colored builds),
+    // physical units: about `unit_bytes` input bytes per unit (default 2000),
     // at most 2^25 units (unit sizes then stay near unit_bytes up to ~30 GB
     // of input, so a schedule tuned on a sample holds at full size)
     uint32_t xb = 0;
-    // (colored builds have smaller LDS tables per workgroup: smaller units)
-    const uint64_t unit_bytes = ctx->tune.unit_bytes ? ctx->tune.unit_bytes : (n_colors ? 1000 : 2000);
+    // (colored builds with the same units, although their LDS tables are
+    // smaller: 64 colors of 41 MB 2.54 ms against 2.74 ms with units of 1000)
+    const uint64_t unit_bytes = ctx->tune.unit_bytes ? ctx->tune.unit_bytes : 2000;
     while (xb < 10 && (n_bytes >> xb) / n_sub > unit_bytes && ((uint64_t)n_sub << (xb + 1)) <= (1u << 25)) xb++;
     const uint32_t n_units = n_sub << xb;
     // slot: meta word + inline bases for the longest unique-minimizer record (2k - m)
@@ -1416,7 +1416,7 @@ int ggcat_gpu_kmers_merge(ggcat_gpu_ctx* ctx) {
     // (rec_cap / 2) has at most one record per thread
     const uint32_t merge_threads = ctx->tune.merge_threads == 128 ? 128u : 256u;
     M.rec_cap =
-        std::min<uint32_t>(ctx->tune.rec_cap ? ctx->tune.rec_cap : rec_cap_default(ctx->slot_words), 2 * merge_threads);
+        std::min<uint32_t>(ctx->tune.rec_cap ? ctx->tune.rec_cap : REC_CAP_DEFAULT, 2 * merge_threads);
     M.rec_lds_off = (uint32_t)(((size_t)M.lds_cap * entry_bytes + 64 + 15) / 16 * 16);
     const size_t lds_bytes =
         M.dedup ? M.rec_lds_off + rec_table_bytes(ctx->slot_words, p.k, M.rec_cap, mode == 0 ? 0 : mode == 1 ? 1 : 4, W != 0,

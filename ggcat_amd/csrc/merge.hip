@@ -535,9 +535,10 @@ GG_DEV void insert_item(const MergeArgs& A, uint64_t r0, uint64_t r1, const Part
 // on its own.  After deduplication every thread takes k-mers of the distinct
 // records (MODE != 0), so the k-mer work is spread evenly over the workgroup.
 // Record table slots (a power of two, 16..512); chunks of rec_cap / 2
-// records are deduplicated at a time.  Slots of 8 words take 256: 512 would
-// cost the 128-bit variants one of the four workgroups a CU's LDS holds.
-__host__ __device__ inline uint32_t rec_cap_default(uint32_t slot_words) { return slot_words <= 4 ? 512 : 256; }
+// records are deduplicated at a time.  512 would cost one of the four
+// workgroups that a CU's LDS holds: merge of 1.57 G occurrences (k = 31)
+// 11.0 ms against 8.6 ms with 256, of 551 M (k = 63) 14.3 against 11.4 ms.
+constexpr uint32_t REC_CAP_DEFAULT = 256;
 
 struct RecTable {
     uint32_t* key;  // rec_cap * SW

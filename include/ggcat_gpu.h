@@ -219,7 +219,7 @@ int ggcat_gpu_solid_colors(ggcat_gpu_ctx* ctx, uint32_t* color_words, uint32_t* 
  *                     which otherwise take their records by position
  *                     (no mode changes a result)
  *   unit_bytes        bucketing: input bytes per physical unit (sub-bucket
- *                     refinement); default 2000, 1000 for colored builds
+ *                     refinement); default 2000
  *   use_graphs        1: capture the bucketing staging pass (clears, stage
  *                     and deferred-record kernels) in a HIP graph per
  *                     argument set and replay it on later calls
@@ -228,7 +228,7 @@ int ggcat_gpu_solid_colors(ggcat_gpu_ctx* ctx, uint32_t* color_words, uint32_t* 
  *                     records expected per unit); records past it go to a
  *                     spill list; the result never depends on it
  *   rec_cap           merge: identical-record table slots (power of two in
- *                     [16, 512], default 512); records are deduplicated in
+ *                     [16, 512], default 256); records are deduplicated in
  *                     chunks of rec_cap / 2 (at most one record per thread)
  *   merge_threads     threads per merge workgroup: 128 or 256 (default)
  *   read_block        input files: the read block of the reference's line
