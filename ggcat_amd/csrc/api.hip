@@ -85,10 +85,10 @@ struct ggcat_gpu_ctx {
     } graph_a_key{};
     uint32_t n_color_ids = 0;  // largest color id + 1 of the colored build
     // query index over the solid table
-    DevBuf idx_key, idx_pos, idx_boff, idx_bcount, idx_bcursor;
+    DevBuf idx_slots, idx_count;
     bool have_index = false;
-    uint32_t idx_log_buckets = 0;
-    DevBuf q_seq, q_off, q_matched, q_counts, q_work;
+    gg::KmerTable idx{};
+    DevBuf q_seq, q_off, q_matched, q_counts;
     struct Server* server = nullptr;
     // unitig chains
     DevBuf u_nb, u_ext, u_link, u_hbytes, u_hcount, u_hoff, u_hidx, u_seq, u_sub, u_flags, u_visited, u_rest,
@@ -207,8 +207,7 @@ int device_scan(ggcat_gpu_ctx* ctx, const uint32_t* counts, uint64_t* off, uint3
 
 // rabin-karp128 constants (crates/hashes/src/cn_rkhash.rs:65-78) and
 // rmmult = MULT^(k-1) (crates/hashes/src/lib.rs:167-191).
-template <class Args>
-void set_rk_constants(Args& M, uint32_t k) {
+void set_rk_constants(MergeArgs& M, uint32_t k) {
     M.rk_mult = mk128(0x3eb9402f3e733993ULL, 0xadd64d3ca00e1b6bULL);
     M.rk_mult_inv = mk128(0x09cb6ff6f1b1a6d7ULL, 0x33e0952e899c3943ULL);
     const u128_t A_ = mk128(0x4751137d01d863c5ULL, 0xb8c36de2b7d399dfULL);
@@ -225,6 +224,68 @@ void set_rk_constants(Args& M, uint32_t k) {
         M.rk_fwd_rm[c] = M.rk_fwd[c] * r;
         M.rk_bkw_rm[c] = M.rk_bkw[c] * r;
     }
+}
+
+// Hash table over the n solid entries, on the context's stream.
+int table_build(ggcat_gpu_ctx* ctx, uint64_t n, DevBuf& slots, DevBuf& count, KmerTable* out) {
+    KmerTable T{};
+    T.nb = table_buckets(n);
+    T.key_words = ctx->key_words;
+    const uint64_t slot_words = (uint64_t)T.nb * TAB_BUCKET * T.key_words * 4;  // 32-bit
+    ENSURE(slots, slot_words * 4);
+    ENSURE(count, (size_t)T.nb * 4);
+    T.slots = P_<ulonglong2>(slots);
+    T.count = P_<uint32_t>(count);
+    const uint32_t wide = (uint32_t)ctx->n_cu * 16;
+    hipLaunchKernelGGL(fill32_kernel, dim3((uint32_t)std::min<uint64_t>((slot_words + 255) / 256, wide)), dim3(256), 0,
+                       ctx->stream, P_<uint32_t>(slots), 0xFFFFFFFFu, slot_words);
+    hipLaunchKernelGGL(fill32_kernel, dim3(std::min<uint32_t>((T.nb + 255) / 256, wide)), dim3(256), 0, ctx->stream,
+                       T.count, 0u, (uint64_t)T.nb);
+    if (n)
+        hipLaunchKernelGGL(table_insert_kernel, dim3((uint32_t)std::min<uint64_t>((n + 255) / 256, wide)), dim3(256), 0,
+                           ctx->stream, T, P_<uint64_t>(ctx->out_key), n);
+    HIPCHK(hipGetLastError());
+    *out = T;
+    return GGCAT_GPU_OK;
+}
+
+// Tables of the rabin-karp128 hash for k: start terms of the rolling hash per
+// base position and base (rk_pos), terms of three bases of a whole k-mer
+// (rk_tri); kept until another k is asked for.
+int rk_tables(ggcat_gpu_ctx* ctx, uint32_t k) {
+    if (ctx->rk_pos_k == k) return GGCAT_GPU_OK;
+    MergeArgs M{};
+    set_rk_constants(M, k);
+    std::vector<u128_t> tab((size_t)8 * (k - 1)), tri((size_t)128 * ((k + 2) / 3));
+    std::vector<u128_t> pw(k);  // M^i
+    pw[0] = 1;
+    for (uint32_t i = 1; i < k; i++) pw[i] = pw[i - 1] * M.rk_mult;
+    for (uint32_t e = 0; e < tri.size() / 2; e++) {
+        u128_t f = 0, b = 0;
+        for (uint32_t j = 0, i = 3 * (e / 64); j < 3 && i < k; j++, i++) {
+            const uint32_t c = (e >> (2 * j)) & 3;
+            f += M.rk_fwd[c] * pw[k - 1 - i];
+            b += M.rk_bkw[c] * pw[i];
+        }
+        tri[2 * e] = f;
+        tri[2 * e + 1] = b;
+    }
+    for (uint32_t i = 0; i + 1 < k; i++) {
+        u128_t pf = 1, pb = M.rk_mult;  // M^(k-2-i), M^(i+1)
+        for (uint32_t e = 0; e + 2 + i < k; e++) pf *= M.rk_mult;
+        for (uint32_t e = 0; e < i; e++) pb *= M.rk_mult;
+        for (uint32_t c = 0; c < 4; c++) {
+            tab[2 * (4 * i + c)] = M.rk_fwd[c] * pf;
+            tab[2 * (4 * i + c) + 1] = M.rk_bkw[c] * pb;
+        }
+    }
+    ctx->rk_pos_k = 0;
+    ENSURE(ctx->rk_tri, tri.size() * sizeof(u128_t));
+    HIPCHK(hipMemcpy(ctx->rk_tri.p, tri.data(), tri.size() * sizeof(u128_t), hipMemcpyHostToDevice));
+    ENSURE(ctx->rk_pos, tab.size() * sizeof(u128_t));
+    HIPCHK(hipMemcpy(ctx->rk_pos.p, tab.data(), tab.size() * sizeof(u128_t), hipMemcpyHostToDevice));
+    ctx->rk_pos_k = k;
+    return GGCAT_GPU_OK;
 }
 
 // Query records of a joined buffer: start offsets [n + 1] (entry q + 1 is one
@@ -255,17 +316,29 @@ void query_kmer_counts(const std::vector<uint64_t>& off, uint32_t k, uint64_t* o
 QueryArgs query_args(ggcat_gpu_ctx* ctx) {
     QueryArgs Q{};
     Q.k = ctx->P.k;
-    Q.kind = ctx->P.hash_kind;
-    Q.key_words = ctx->key_words;
-    Q.idx_key = P_<uint64_t>(ctx->idx_key);
-    Q.idx_pos = P_<uint32_t>(ctx->idx_pos);
-    Q.boff = P_<uint64_t>(ctx->idx_boff);
-    Q.log_buckets = ctx->idx_log_buckets;
+    Q.index = ctx->idx;
     Q.color_words = ctx->colored ? ctx->color_words : 0;
     Q.out_colors = ctx->colored ? P_<uint32_t>(ctx->out_colors) : nullptr;
     Q.n_colors = ctx->colored ? ctx->n_color_ids : 0;
-    set_rk_constants(Q, ctx->P.k);
+    Q.rk_tri = P_<u128_t>(ctx->rk_tri);
     return Q;
+}
+
+// Queries Q.seq[0, n_bytes) on a stream; the results are cleared already.
+// Positions per wavefront: the batch over 16 wavefronts per CU, at least 64
+// (short requests spread over the chip), at most QUERY_SPAN.
+void launch_query(const ggcat_gpu_ctx* ctx, QueryArgs& Q, uint64_t n_bytes, hipStream_t stream) {
+    Q.n = n_bytes;
+    const uint64_t want = n_bytes / ((uint64_t)ctx->n_cu * 16) / 64 * 64;
+    Q.span = (uint32_t)std::min<uint64_t>(QUERY_SPAN, std::max<uint64_t>(64, want));
+    const dim3 grid((uint32_t)((n_bytes + Q.span - 1) / Q.span));
+    const size_t lds = (size_t)Q.n_colors * 4 + 16;
+    if (ctx->P.hash_kind == GGCAT_GPU_HASH_RK128)
+        hipLaunchKernelGGL(query_kernel<2>, grid, dim3(64), lds, stream, Q);
+    else if (ctx->P.k > 32)
+        hipLaunchKernelGGL(query_kernel<1>, grid, dim3(64), lds, stream, Q);
+    else
+        hipLaunchKernelGGL(query_kernel<0>, grid, dim3(64), lds, stream, Q);
 }
 
 // First-fit allocator over one pre-allocated range (offsets 256-aligned).
@@ -315,7 +388,7 @@ struct ServeReq {
     int stream = -1;
     uint64_t dev_off = 0, pin_off = 0, bytes = 0;
     // layout inside both ranges
-    uint64_t o_seq = 0, o_off = 0, o_work = 0, o_matched = 0, o_counts = 0;
+    uint64_t o_seq = 0, o_off = 0, o_matched = 0, o_counts = 0;
     hipEvent_t ev = nullptr;
 };
 
@@ -338,7 +411,7 @@ struct Server {
 namespace {
 
 // Layout of one request inside its device / pinned range (same offsets in
-// both): query bytes, offsets, work counter, then the results.
+// both): query bytes, offsets, then the results.
 void serve_layout(const ggcat_gpu_ctx* ctx, ServeReq& r) {
     const uint32_t nq = r.n_queries, nc = ctx->colored ? ctx->n_color_ids : 0;
     uint64_t o = 0;
@@ -349,7 +422,6 @@ void serve_layout(const ggcat_gpu_ctx* ctx, ServeReq& r) {
     };
     r.o_seq = place(r.n_bytes + 16);
     r.o_off = place(((uint64_t)nq + 1) * 8);
-    r.o_work = place(8);
     r.o_matched = place((uint64_t)nq * 8);
     r.o_counts = place((uint64_t)nq * nc * 4 + 4);
     r.bytes = o;
@@ -362,7 +434,7 @@ int serve_admit(ggcat_gpu_ctx* ctx) {
     Server& S = *ctx->server;
     while (!S.waiting.empty()) {
         ServeReq& r = S.reqs[S.waiting.front()];
-        const uint32_t nq = r.n_queries, nc = ctx->colored ? ctx->n_color_ids : 0;
+        const uint32_t nq = r.n_queries;
         uint64_t doff, poff;
         if (!S.dalloc.alloc(r.bytes, &doff)) break;
         if (!S.palloc.alloc(r.bytes, &poff)) {
@@ -374,24 +446,24 @@ int serve_admit(ggcat_gpu_ctx* ctx) {
         uint8_t* hp = S.pin + poff;
         memcpy(hp + r.o_seq, r.src, r.n_bytes);
         memcpy(hp + r.o_off, r.off.data(), r.off.size() * 8);
-        memset(hp + r.o_work, 0, 8);
         int si = 0;
         for (int i = 1; i < (int)S.streams.size(); i++)
             if (S.load[i] < S.load[si]) si = i;
         r.stream = si;
         hipStream_t st = S.streams[si];
         uint8_t* dp = S.dev + doff;
-        HIPCHK(hipMemcpyAsync(dp, hp, r.o_matched, hipMemcpyHostToDevice, st));  // seq, offsets, work counter
+        HIPCHK(hipMemcpyAsync(dp, hp, r.o_matched, hipMemcpyHostToDevice, st));  // seq, offsets
         QueryArgs Q = query_args(ctx);
         Q.seq = dp + r.o_seq;
         Q.qoff = reinterpret_cast<const uint64_t*>(dp + r.o_off);
         Q.n_queries = nq;
         Q.matched = reinterpret_cast<uint64_t*>(dp + r.o_matched);
         Q.color_counts = reinterpret_cast<uint32_t*>(dp + r.o_counts);
-        Q.work = reinterpret_cast<unsigned int*>(dp + r.o_work);
         if (nq) {
-            const uint32_t grid = std::min<uint32_t>(nq, ctx->n_cu * 4);
-            hipLaunchKernelGGL(query_kernel, dim3(grid), dim3(256), (size_t)nc * 4 + 16, st, Q);
+            const uint64_t words = (r.bytes - r.o_matched) / 4;
+            hipLaunchKernelGGL(fill32_kernel, dim3((uint32_t)std::min<uint64_t>((words + 255) / 256, ctx->n_cu * 16)),
+                               dim3(256), 0, st, reinterpret_cast<uint32_t*>(dp + r.o_matched), 0u, words);
+            launch_query(ctx, Q, r.n_bytes, st);
             HIPCHK(hipGetLastError());
         }
         HIPCHK(hipMemcpyAsync(hp + r.o_matched, dp + r.o_matched, r.bytes - r.o_matched, hipMemcpyDeviceToHost, st));
@@ -454,8 +526,8 @@ void ggcat_gpu_destroy(ggcat_gpu_ctx* ctx) {
                       &ctx->n_items, &ctx->work, &ctx->parts, &ctx->redo, &ctx->redo_count, &ctx->out_key,
                       &ctx->out_val, &ctx->out_sub, &ctx->chunk_cursor, &ctx->chunk_fill_dev, &ctx->chunk_off, &ctx->fix_key,
                       &ctx->fix_val, &ctx->fix_sub, &ctx->fix_cursor, &ctx->out_colors, &ctx->fix_colors,
-                      &ctx->idx_key, &ctx->idx_pos, &ctx->idx_boff, &ctx->idx_bcount, &ctx->idx_bcursor,
-                      &ctx->q_seq, &ctx->q_off, &ctx->q_matched, &ctx->q_counts, &ctx->q_work,
+                      &ctx->idx_slots, &ctx->idx_count,
+                      &ctx->q_seq, &ctx->q_off, &ctx->q_matched, &ctx->q_counts,
                       &ctx->u_nb, &ctx->u_ext, &ctx->u_link, &ctx->u_hbytes, &ctx->u_hcount, &ctx->u_hoff,
                       &ctx->u_hidx, &ctx->u_seq, &ctx->u_sub, &ctx->u_flags, &ctx->u_visited, &ctx->u_rest,
                       &ctx->u_rest_n, &ctx->u_rep, &ctx->u_tab, &ctx->u_path, &ctx->stage_slots, &ctx->stage_unit,
@@ -1424,39 +1496,9 @@ int ggcat_gpu_kmers_merge(ggcat_gpu_ctx* ctx) {
                 : (size_t)M.lds_cap * entry_bytes + 64;
     M.pool_words = ctx->pool_words;
     set_rk_constants(M, p.k);
-    if (p.hash_kind == GGCAT_GPU_HASH_RK128) {
-        // start terms of the rolling hash per base position and base
-        if (ctx->rk_pos_k != p.k) {
-            std::vector<u128_t> tab((size_t)8 * (p.k - 1)), tri((size_t)128 * ((p.k + 2) / 3));
-            std::vector<u128_t> pw(p.k);  // M^i
-            pw[0] = 1;
-            for (uint32_t i = 1; i < p.k; i++) pw[i] = pw[i - 1] * M.rk_mult;
-            for (uint32_t e = 0; e < tri.size() / 2; e++) {
-                u128_t f = 0, b = 0;
-                for (uint32_t j = 0, i = 3 * (e / 64); j < 3 && i < p.k; j++, i++) {
-                    const uint32_t c = (e >> (2 * j)) & 3;
-                    f += M.rk_fwd[c] * pw[p.k - 1 - i];
-                    b += M.rk_bkw[c] * pw[i];
-                }
-                tri[2 * e] = f;
-                tri[2 * e + 1] = b;
-            }
-            for (uint32_t i = 0; i + 1 < p.k; i++) {
-                u128_t pf = 1, pb = M.rk_mult;  // M^(k-2-i), M^(i+1)
-                for (uint32_t e = 0; e + 2 + i < p.k; e++) pf *= M.rk_mult;
-                for (uint32_t e = 0; e < i; e++) pb *= M.rk_mult;
-                for (uint32_t c = 0; c < 4; c++) {
-                    tab[2 * (4 * i + c)] = M.rk_fwd[c] * pf;
-                    tab[2 * (4 * i + c) + 1] = M.rk_bkw[c] * pb;
-                }
-            }
-            ctx->rk_pos_k = 0;
-            ENSURE(ctx->rk_tri, tri.size() * sizeof(u128_t));
-            HIPCHK(hipMemcpy(ctx->rk_tri.p, tri.data(), tri.size() * sizeof(u128_t), hipMemcpyHostToDevice));
-            ENSURE(ctx->rk_pos, tab.size() * sizeof(u128_t));
-            HIPCHK(hipMemcpy(ctx->rk_pos.p, tab.data(), tab.size() * sizeof(u128_t), hipMemcpyHostToDevice));
-            ctx->rk_pos_k = p.k;
-        }
+    if (rk) {
+        const int r = rk_tables(ctx, p.k);
+        if (r != GGCAT_GPU_OK) return r;
         M.rk_pos = P_<u128_t>(ctx->rk_pos);
         M.rk_tri = P_<u128_t>(ctx->rk_tri);
     }
@@ -2150,43 +2192,12 @@ int ggcat_gpu_index_build(ggcat_gpu_ctx* ctx) {
     if (!ctx->have_solid) return fail(ctx, GGCAT_GPU_ESTATE, "no merge result");
     if (ctx->server) return fail(ctx, GGCAT_GPU_ESTATE, "close the query server before rebuilding the index");
     HIPCHK(hipSetDevice(ctx->device));
-    const uint32_t kw = ctx->key_words;
     const uint64_t n = ctx->n_solid;
-    uint32_t L = 0;
-    while (L < 30 && (1ull << (L + 2)) < n) L++;  // about 4 entries per bucket
-    const uint32_t nb = 1u << L;
-    ENSURE(ctx->idx_bcount, (size_t)nb * 4);
-    ENSURE(ctx->idx_bcursor, (size_t)nb * 4);
-    ENSURE(ctx->idx_boff, ((size_t)nb + 1) * 8);
-    ENSURE(ctx->idx_key, n * 8 * kw + 8);
-    ENSURE(ctx->idx_pos, n * 4 + 4);
-    IndexArgs I{};
-    I.out_key = P_<uint64_t>(ctx->out_key);
-    I.key_words = kw;
-    I.log_buckets = L;
-    I.bcount = P_<uint32_t>(ctx->idx_bcount);
-    I.boff = P_<uint64_t>(ctx->idx_boff);
-    I.bcursor = P_<uint32_t>(ctx->idx_bcursor);
-    I.idx_key = P_<uint64_t>(ctx->idx_key);
-    I.idx_pos = P_<uint32_t>(ctx->idx_pos);
-    const uint64_t n_pos = n;
-    if (n_pos >= 0x7FFFFFFFull) return fail(ctx, GGCAT_GPU_EINVAL, "solid table too large for the query index");
-    HIPCHK(hipMemsetAsync(ctx->idx_bcount.p, 0, (size_t)nb * 4, ctx->stream));
-    HIPCHK(hipMemsetAsync(ctx->idx_bcursor.p, 0, (size_t)nb * 4, ctx->stream));
-    const uint32_t grid = (uint32_t)std::min<uint64_t>((n_pos + 255) / 256 + 1, (uint64_t)ctx->n_cu * 16);
-    if (n_pos) hipLaunchKernelGGL(index_count_kernel, dim3(grid), dim3(256), 0, ctx->stream, I, n_pos);
-    HIPCHK(hipGetLastError());
-    {
-        int r = device_scan(ctx, I.bcount, P_<uint64_t>(ctx->idx_boff), nb);
-        if (r != GGCAT_GPU_OK) return r;
-    }
-    if (n_pos) hipLaunchKernelGGL(index_fill_kernel, dim3(grid), dim3(256), 0, ctx->stream, I, n_pos);
-    HIPCHK(hipGetLastError());
-    uint64_t total = 0;
-    HIPCHK(hipMemcpyAsync(&total, P_<uint64_t>(ctx->idx_boff) + nb, 8, hipMemcpyDeviceToHost, ctx->stream));
+    if (n >= 0x7FFFFFFFull) return fail(ctx, GGCAT_GPU_EINVAL, "solid table too large for the query index");
+    int r = ctx->P.hash_kind == GGCAT_GPU_HASH_RK128 ? rk_tables(ctx, ctx->P.k) : GGCAT_GPU_OK;
+    if (r == GGCAT_GPU_OK) r = table_build(ctx, n, ctx->idx_slots, ctx->idx_count, &ctx->idx);
+    if (r != GGCAT_GPU_OK) return r;
     HIPCHK(hipStreamSynchronize(ctx->stream));
-    if (total != n) return fail(ctx, GGCAT_GPU_EHIP, "query index holds a different number of entries than the solid table");
-    ctx->idx_log_buckets = L;
     ctx->have_index = true;
     return GGCAT_GPU_OK;
 }
@@ -2212,20 +2223,18 @@ int ggcat_gpu_query(ggcat_gpu_ctx* ctx, const uint8_t* queries, uint64_t n_bytes
     ENSURE(ctx->q_off, ((size_t)n_queries + 1) * 8);
     ENSURE(ctx->q_matched, (size_t)n_queries * 8 + 8);
     ENSURE(ctx->q_counts, (size_t)n_queries * nc * 4 + 4);
-    ENSURE(ctx->q_work, 8);
     if (n_bytes) HIPCHK(hipMemcpy(ctx->q_seq.p, queries, n_bytes, hipMemcpyHostToDevice));
     HIPCHK(hipMemcpy(ctx->q_off.p, off.data(), off.size() * 8, hipMemcpyHostToDevice));
-    HIPCHK(hipMemsetAsync(ctx->q_work.p, 0, 8, ctx->stream));
     QueryArgs Q = query_args(ctx);
     Q.seq = P_<uint8_t>(ctx->q_seq);
     Q.qoff = P_<uint64_t>(ctx->q_off);
     Q.n_queries = n_queries;
     Q.matched = P_<uint64_t>(ctx->q_matched);
     Q.color_counts = P_<uint32_t>(ctx->q_counts);
-    Q.work = P_<unsigned int>(ctx->q_work);
     if (n_queries) {
-        const uint32_t grid = std::min<uint32_t>(n_queries, ctx->n_cu * 4);
-        hipLaunchKernelGGL(query_kernel, dim3(grid), dim3(256), (size_t)nc * 4 + 16, ctx->stream, Q);
+        HIPCHK(hipMemsetAsync(ctx->q_matched.p, 0, (size_t)n_queries * 8, ctx->stream));
+        if (nc) HIPCHK(hipMemsetAsync(ctx->q_counts.p, 0, (size_t)n_queries * nc * 4, ctx->stream));
+        launch_query(ctx, Q, n_bytes, ctx->stream);
         HIPCHK(hipGetLastError());
     }
     HIPCHK(hipStreamSynchronize(ctx->stream));

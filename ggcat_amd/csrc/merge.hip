@@ -273,14 +273,14 @@ GG_DEV void rk_segment(const MergeArgs& A, const uint32_t* bw, uint32_t i0, uint
     }
 }
 
-// Rabin-karp128 key of a k-mer from its 2-bit form (lo, hi): the sums of its
-// bases' terms, three bases per table entry (43 KB at k = 63: lines of one
+// Rabin-karp128 key of a k-mer from its 2-bit form x: the sums of its bases'
+// terms, three bases per table entry (43 KB at k = 63: lines of one
 // group are shared by the lanes), and the smaller of the two; *swap when that
 // is the hash of the reverse complement.
-GG_DEV u128_t rk_of_kmer(const MergeArgs& A, uint64_t lo, uint64_t hi, bool* swap) {
-    u128_t x = ((u128_t)hi << 64) | lo, f = 0, b = 0;
-    for (uint32_t g = 0; 3 * g < A.k; g++) {
-        const u128_t* e = A.rk_tri + 2 * (64 * g + ((uint32_t)x & 63u));
+GG_DEV u128_t rk_of_kmer(const u128_t* tri, uint32_t k, u128_t x, bool* swap) {
+    u128_t f = 0, b = 0;
+    for (uint32_t g = 0; 3 * g < k; g++) {
+        const u128_t* e = tri + 2 * (64 * g + ((uint32_t)x & 63u));
         f += e[0];
         b += e[1];
         x >>= 6;
@@ -412,7 +412,7 @@ GG_DEV void emit_solid(const MergeArgs& A, uint32_t sub, const uint64_t* klo, co
             }
             if (Mode<MODE>::RK) {
                 bool swap;
-                const u128_t key = rk_of_kmer(A, lo, hi, &swap);
+                const u128_t key = rk_of_kmer(A.rk_tri, A.k, ((u128_t)hi << 64) | lo, &swap);
                 lo = (uint64_t)key;
                 hi = (uint64_t)(key >> 64);
                 // the flags face the hash's strand
@@ -610,13 +610,13 @@ GG_DEV uint64_t kmer_at(const uint32_t* bw, uint32_t i, uint32_t k, bool* fwd) {
     return fw < rc ? fw : rc;
 }
 
-// Both strands of the k-mer (32 < k < 64) at base offset i of packed words, as
-// their 2-bit forms.
+// Both strands of the k-mer (k <= 64) at base offset i of packed words, as
+// their 2-bit forms; reads the word of its first base and the three behind it.
 GG_DEV void kmer_pair_at(const uint32_t* bw, uint32_t i, uint32_t k, u128_t* fw, u128_t* rc) {
     const uint32_t wi = i >> 4, sh = (i & 15) * 2;
     const u128_t w03 = (u128_t)((uint64_t)bw[wi] | ((uint64_t)bw[wi + 1] << 32)) |
                        ((u128_t)((uint64_t)bw[wi + 2] | ((uint64_t)bw[wi + 3] << 32)) << 64);
-    const u128_t mask = ((u128_t)1 << (2 * k)) - 1;
+    const u128_t mask = ~(u128_t)0 >> (128 - 2 * k);
     u128_t x = w03 >> sh;
     // the fifth word is only read when the k-mer reaches into it
     if (sh + 2 * k > 128) x |= (u128_t)bw[wi + 4] << (128 - sh);

@@ -4,21 +4,21 @@
 // hipMalloc (tight serving loops, code that must not allocate): the queries
 // and every result live in caller-owned device memory, and the only device
 // memory beyond them is `scratch`, a fixed array of this library holding the
-// work cursor, the per-block newline counts and the query offsets.  Its
+// per-block newline counts and the query offsets.  Its
 // address is looked up once per device when a context is created
 // (noalloc_scratch_setup) and only that address is handed to kernels.
 //
 // Every call on a device shares that device's array: calls that overlap on
 // one GPU (two contexts or two threads) race and must be serialised by the
 // caller.  The array keeps the last call's contents; what must start at zero
-// (the work cursor, the error word) is cleared by a kernel at every call.
+// (the error word) is cleared by a kernel at every call.
 //
 // Included by api.hip (one translation unit).
 
 namespace {
 
 // Scratch layout (bytes):
-//   [0, 256)                    header: u32 work cursor, u32 error word, u32 newline total
+//   [0, 256)                    header: u32 unused, u32 error word, u32 newline total
 //   [256, 256 + 4 * NA_MAX_BLOCKS)  newline count of each 16 KiB block, scanned in place
 //   [NA_OFF_AT, ...)            (n_queries + 1) u64 query start offsets
 constexpr uint32_t NA_BLOCK_BYTES = 16384;  // bytes per counting block (256 threads x 64 bytes)
@@ -153,12 +153,17 @@ __global__ void na_check_kernel(const uint8_t* seq, uint64_t n, uint32_t n_queri
     if (header[2] != n_queries || (n && seq[n - 1] != '\n')) atomicOr(&header[1], 2u);
 }
 
-// query_kmers[q] = length - (k - 1), saturating (crates/querier/src/lib.rs:138-150).
-__global__ void na_qkmers_kernel(const uint64_t* off, uint32_t n_queries, uint32_t k, uint64_t* out) {
-    const uint32_t q = blockIdx.x * blockDim.x + threadIdx.x;
-    if (q >= n_queries) return;
-    const uint64_t len = off[q + 1] - off[q] - 1;
-    out[q] = len >= k ? len - (k - 1) : 0;
+// query_kmers[q] = length - (k - 1), saturating (crates/querier/src/lib.rs:138-150)
+// where wanted; the counters that the query adds to are cleared.
+__global__ void na_init_kernel(const uint64_t* off, uint32_t n_queries, uint32_t k, uint64_t* query_kmers,
+                               uint64_t* matched, uint32_t* color_counts, uint32_t n_colors) {
+    const uint64_t i0 = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x, step = (uint64_t)gridDim.x * blockDim.x;
+    for (uint64_t q = i0; q < n_queries; q += step) {
+        const uint64_t len = off[q + 1] - off[q] - 1;
+        if (query_kmers) query_kmers[q] = len >= k ? len - (k - 1) : 0;
+        matched[q] = 0;
+    }
+    for (uint64_t i = i0; i < (uint64_t)n_queries * n_colors; i += step) color_counts[i] = 0;
 }
 
 }  // namespace
@@ -196,18 +201,17 @@ extern "C" int ggcat_gpu_query_device_noalloc(ggcat_gpu_ctx* ctx, const uint8_t*
     HIPCHK(hipMemcpyAsync(&err, header + 1, 4, hipMemcpyDeviceToHost, ctx->stream));
     HIPCHK(hipStreamSynchronize(ctx->stream));
     if (err) return fail(ctx, GGCAT_GPU_EINVAL, "queries must be n_queries records, each ending with '\\n'");
-    if (d_query_kmers)
-        hipLaunchKernelGGL(na_qkmers_kernel, dim3((n_queries + 255) / 256), dim3(256), 0, ctx->stream, off, n_queries,
-                           ctx->P.k, d_query_kmers);
+    const uint32_t grid =
+        (uint32_t)std::min<uint64_t>(((uint64_t)n_queries * std::max(nc, 1u) + 255) / 256, (uint64_t)ctx->n_cu * 16);
+    hipLaunchKernelGGL(na_init_kernel, dim3(grid), dim3(256), 0, ctx->stream, off, n_queries, ctx->P.k, d_query_kmers,
+                       d_matched, d_color_counts, nc);
     QueryArgs Q = query_args(ctx);
     Q.seq = d_queries;
     Q.qoff = off;
     Q.n_queries = n_queries;
     Q.matched = d_matched;
     Q.color_counts = d_color_counts;
-    Q.work = header;  // header[0]: work cursor, zeroed above
-    const uint32_t grid = std::min<uint32_t>(n_queries, ctx->n_cu * 4);
-    hipLaunchKernelGGL(query_kernel, dim3(grid), dim3(256), (size_t)nc * 4 + 16, ctx->stream, Q);
+    launch_query(ctx, Q, n_bytes, ctx->stream);
     HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(ctx->stream));
     return GGCAT_GPU_OK;

@@ -8,10 +8,9 @@
 // and once for each color of that k-mer's color set.  The graph k-mer set is
 // the solid table of the build (the k-mers of its unitigs).
 //
-// Index: the solid entries hashed into 2^L buckets (about 4 entries each) and
-// stored bucket-major (key words + position of the entry in the solid
-// arrays), built with a count / scan / scatter like the bucketing.  A lookup
-// reads the bucket bounds and scans one short run of keys.
+// Index: a hash table of 4-entry buckets (KmerTable) over the solid entries;
+// an entry holds its key words and its position in the solid arrays, so a
+// lookup reads one line in most cases.
 #include "common.h"
 
 namespace gg {
@@ -27,92 +26,105 @@ GG_DEV uint64_t mix64(uint64_t x) {
 
 GG_DEV uint64_t index_hash(uint64_t lo, uint64_t hi) { return mix64(lo ^ mix64(hi + 0x9E3779B97F4A7C15ULL)); }
 
-struct IndexArgs {
-    const uint64_t* out_key;  // solid keys, key_words per position
+constexpr uint32_t NO_POS = 0xFFFFFFFFu;
+
+// Hash table of solid entries: nb buckets of 4 entries, a bucket's entries in
+// arrival order, the first free one empty (position NO_POS); an entry whose
+// bucket is full goes to the next bucket with room.  Entry words: 64-bit keys
+// {key, position}, 128-bit keys {low, high, position, 0}, so a bucket is 64 or
+// 128 bytes.  1.6 slots per entry: few buckets overflow (mean fill 2.5).
+// Bound by one random counter update and one random 16-byte store per entry
+// (the counters of 100 M entries fit the 256 MiB cache); building it takes one
+// pass over the keys where offsets of exactly sized buckets took a counting
+// pass, a scan and a placing pass with its own atomics, and a lookup reads the
+// bucket alone instead of offsets, keys and positions.  Index of 57.7 M
+// entries 8.3 -> 5.9 ms (0.4 of it clearing).
+struct KmerTable {
+    ulonglong2* slots;  // [nb * 4 * key_words]
+    uint32_t* count;  // [nb] entries that arrived (more than 4: the bucket overflowed)
+    uint32_t nb;
     uint32_t key_words;
-    uint32_t log_buckets;
-    uint32_t* bcount;
-    const uint64_t* boff;
-    uint32_t* bcursor;
-    uint64_t* idx_key;
-    uint32_t* idx_pos;
 };
 
-GG_DEV uint32_t index_bucket(const IndexArgs& A, uint64_t p) {
-    const uint64_t lo = A.out_key[p * A.key_words];
-    const uint64_t hi = A.key_words == 2 ? A.out_key[p * 2 + 1] : 0;
-    return A.log_buckets ? (uint32_t)(index_hash(lo, hi) >> (64 - A.log_buckets)) : 0u;
+constexpr uint32_t TAB_BUCKET = 4;
+__host__ __device__ inline uint32_t table_buckets(uint64_t n) { return (uint32_t)(n * 2 / 5 + 1); }
+
+GG_DEV uint32_t table_bucket(const KmerTable& T, uint64_t lo, uint64_t hi) {
+    return (uint32_t)(((index_hash(lo, hi) >> 32) * T.nb) >> 32);
 }
 
-__global__ void index_count_kernel(IndexArgs A, uint64_t n_pos) {
-    for (uint64_t p = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; p < n_pos; p += (uint64_t)gridDim.x * blockDim.x)
-        atomicAdd(&A.bcount[index_bucket(A, p)], 1u);
+// Entries [0, n) of the solid keys into the table (cleared: counts 0, slots ~0).
+__global__ void table_insert_kernel(KmerTable T, const uint64_t* key, uint64_t n) {
+    for (uint64_t p = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; p < n; p += (uint64_t)gridDim.x * blockDim.x) {
+        const uint64_t lo = key[p * T.key_words], hi = T.key_words == 2 ? key[p * 2 + 1] : 0;
+        uint32_t b = table_bucket(T, lo, hi), r;
+        // 4 nb > n: some bucket has room
+        while ((r = atomicAdd(&T.count[b], 1u)) >= TAB_BUCKET) b = b + 1 == T.nb ? 0 : b + 1;
+        ulonglong2* e = T.slots + ((uint64_t)b * TAB_BUCKET + r) * T.key_words;
+        ulonglong2 v;
+        v.x = lo;
+        v.y = T.key_words == 1 ? p : hi;
+        e[0] = v;
+        if (T.key_words == 2) {
+            v.x = p;
+            v.y = 0;
+            e[1] = v;
+        }
+    }
 }
 
-__global__ void index_fill_kernel(IndexArgs A, uint64_t n_pos) {
-    for (uint64_t p = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; p < n_pos; p += (uint64_t)gridDim.x * blockDim.x) {
-        const uint32_t b = index_bucket(A, p);
-        const uint64_t slot = A.boff[b] + atomicAdd(&A.bcursor[b], 1u);
-        for (uint32_t q = 0; q < A.key_words; q++) A.idx_key[slot * A.key_words + q] = A.out_key[p * A.key_words + q];
-        A.idx_pos[slot] = (uint32_t)p;
+// Calls found(position) for the entries of a key until it returns true.
+template <class F>
+GG_DEV void table_find(const KmerTable& T, uint64_t lo, uint64_t hi, F&& found) {
+    uint32_t b = table_bucket(T, lo, hi);
+    // at most nb buckets, of which at least one is not full
+    while (true) {
+        const ulonglong2* e = T.slots + (uint64_t)b * TAB_BUCKET * T.key_words;
+        if (T.key_words == 1) {
+            ulonglong2 v[TAB_BUCKET];
+#pragma unroll
+            for (uint32_t i = 0; i < TAB_BUCKET; i++) v[i] = e[i];
+#pragma unroll
+            for (uint32_t i = 0; i < TAB_BUCKET; i++) {
+                if ((uint32_t)v[i].y == NO_POS) return;
+                if (v[i].x == lo && found((uint32_t)v[i].y)) return;
+            }
+        } else {
+            for (uint32_t i = 0; i < TAB_BUCKET; i++) {
+                const ulonglong2 v = e[2 * i];
+                const uint32_t pos = (uint32_t)e[2 * i + 1].x;
+                if (pos == NO_POS) return;
+                if (v.x == lo && v.y == hi && found(pos)) return;
+            }
+        }
+        b = b + 1 == T.nb ? 0 : b + 1;
     }
 }
 
 struct QueryArgs {
     const uint8_t* seq;  // joined queries
+    uint64_t n;  // bytes in seq
     const uint64_t* qoff;  // [n_queries + 1] start of each query (query q ends at qoff[q+1] - 1, its '\n')
     uint32_t n_queries;
     uint32_t k;
-    uint32_t kind;  // 0 seq-hash, 1 rabin-karp128
-    uint32_t key_words;
-    const uint64_t* idx_key;
-    const uint32_t* idx_pos;
-    const uint64_t* boff;
-    uint32_t log_buckets;
+    uint32_t span;  // k-mer start positions per wavefront (a multiple of 64, at most QUERY_SPAN)
+    KmerTable index;
     const uint32_t* out_colors;  // color_words per solid position (colored)
     uint32_t color_words;  // 0: uncolored
     uint32_t n_colors;  // per-query color counters written (<= 32 * color_words)
-    uint64_t* matched;  // [n_queries]
-    uint32_t* color_counts;  // [n_queries * n_colors]
-    unsigned int* work;
-    u128_t rk_mult, rk_mult_inv, rk_rmmult;
-    u128_t rk_fwd[4], rk_bkw[4];
-    u128_t rk_fwd_rm[4], rk_bkw_rm[4];  // rk_fwd[c] * rk_rmmult, rk_bkw[c] * rk_rmmult
+    uint64_t* matched;  // [n_queries], cleared
+    uint32_t* color_counts;  // [n_queries * n_colors], cleared
+    const u128_t* rk_tri;  // rabin-karp128: terms of three bases per entry (see MergeArgs)
 };
-
-constexpr uint32_t NO_POS = 0xFFFFFFFFu;
+constexpr uint32_t QUERY_SPAN = 1024;
 
 GG_DEV uint32_t index_lookup(const QueryArgs& A, uint64_t lo, uint64_t hi) {
-    const uint32_t b = A.log_buckets ? (uint32_t)(index_hash(lo, hi) >> (64 - A.log_buckets)) : 0u;
-    const uint64_t e0 = A.boff[b], e1 = A.boff[b + 1];
-    for (uint64_t e = e0; e < e1; e++) {
-        if (A.key_words == 1) {
-            if (A.idx_key[e] == lo) return A.idx_pos[e];
-        } else if (A.idx_key[2 * e] == lo && A.idx_key[2 * e + 1] == hi) {
-            return A.idx_pos[e];
-        }
-    }
-    return NO_POS;
-}
-
-GG_DEV bool colors_equal(const QueryArgs& A, uint32_t p0, uint32_t p1) {
-    if (p0 == p1) return true;
-    for (uint32_t w = 0; w < A.color_words; w++)
-        if (A.out_colors[(uint64_t)p0 * A.color_words + w] != A.out_colors[(uint64_t)p1 * A.color_words + w])
-            return false;
-    return true;
-}
-
-GG_DEV void flush_run(const QueryArgs& A, uint32_t pos, uint32_t cnt, uint32_t* counts) {
-    if (pos == NO_POS || cnt == 0) return;
-    for (uint32_t w = 0; w < A.color_words; w++) {
-        uint32_t bits = A.out_colors[(uint64_t)pos * A.color_words + w];
-        while (bits) {
-            const uint32_t c = w * 32 + (__ffs(bits) - 1);
-            bits &= bits - 1;
-            if (c < A.n_colors) atomicAdd(&counts[c], cnt);
-        }
-    }
+    uint32_t pos = NO_POS;
+    table_find(A.index, lo, hi, [&](uint32_t p) {
+        pos = p;
+        return true;
+    });
+    return pos;
 }
 
 GG_DEV uint32_t ascii_code(uint8_t c) { return (c >> 1) & 3u; }
@@ -121,105 +133,139 @@ GG_DEV bool ascii_acgt(uint8_t c) {
     return u == 'A' || u == 'C' || u == 'G' || u == 'T';
 }
 
-// One workgroup per query (work-stealing over the batch).  Each thread takes
-// a contiguous range of k-mer start positions, rolls the canonical hash over
-// it and looks every all-ACGT k-mer up; runs of hits with the same color set
-// are added to the per-color LDS counters once per run.
-__global__ __launch_bounds__(256) void query_kernel(QueryArgs A) {
+// One wavefront per `span` consecutive byte positions of the batch, whatever
+// the queries' lengths: every position is the start of a k-mer, 64 at a time,
+// one per lane.  The bytes become 2-bit codes and invalid / newline bits in
+// LDS once; a k-mer is cut out of them (a newline is an invalid base, so none
+// crosses queries), its key looked up, and the hits of the 64 positions are
+// counted per query by ballots, one global atomic per query and wavefront.
+// Colors: a run of neighbouring hits with the same color set (its head found by
+// comparing with the lane before) is added to the wavefront's counters by all
+// lanes at once, lane c taking colors c, c + 64, ...
+// One workgroup per query gave a 150 bp read 120 of 256 lanes, each of which
+// loaded k bytes one by one, and rabin-karp128 2 k dependent 128-bit multiplies
+// per lane.  Bound by the lookups (one random line of the table each).
+// 100 K reads: of 250 bp, k = 31, 2.25 -> 0.81 ms; of 150 bp, k = 63
+// rabin-karp128, 3.99 -> 1.01 ms; 5000 colored queries of 100 - 10000 bp 0.64
+// -> 0.44 ms.
+// KIND 0: seq-hash k <= 32, 1: seq-hash k > 32, 2: rabin-karp128.
+template <int KIND>
+__global__ __launch_bounds__(64) void query_kernel(QueryArgs A) {
     extern __shared__ __align__(16) uint8_t lds[];
-    uint32_t* counts = reinterpret_cast<uint32_t*>(lds);
-    __shared__ uint32_t s_q;
-    __shared__ unsigned long long s_matched;
-    const uint32_t k = A.k;
-    while (true) {
-        if (threadIdx.x == 0) {
-            s_q = atomicAdd(A.work, 1u);
-            s_matched = 0;
-        }
-        __syncthreads();
-        const uint32_t q = s_q;
-        if (q >= A.n_queries) break;
-        for (uint32_t c = threadIdx.x; c < A.n_colors; c += blockDim.x) counts[c] = 0;
-        __syncthreads();
-        const uint8_t* s = A.seq + A.qoff[q];
-        const uint64_t len = A.qoff[q + 1] - A.qoff[q] - 1;
-        const uint64_t nk = len >= k ? len - k + 1 : 0;
-        const uint64_t per = (nk + blockDim.x - 1) / blockDim.x;
-        const uint64_t j0 = per * threadIdx.x, j1 = j0 + per < nk ? j0 + per : nk;
-        uint64_t hits = 0;
-        uint32_t run_pos = NO_POS, run_cnt = 0;
-        if (j0 < j1) {
-            int64_t last_bad = (int64_t)j0 - 1;  // last non-ACGT base seen
-            auto on_key = [&](uint64_t lo, uint64_t hi) {
-                const uint32_t pos = index_lookup(A, lo, hi);
-                if (pos == NO_POS) return;
-                hits++;
-                if (A.color_words) {
-                    if (run_pos != NO_POS && colors_equal(A, run_pos, pos)) {
-                        run_cnt++;
-                    } else {
-                        flush_run(A, run_pos, run_cnt, counts);
-                        run_pos = pos;
-                        run_cnt = 1;
-                    }
-                }
-            };
-            if (A.kind == 0 && k <= 32) {
-                const uint64_t mask = (k == 32) ? ~0ULL : ((1ULL << (2 * k)) - 1);
-                uint64_t fw = 0, rc = 0;
-                for (uint64_t i = j0; i < j1 + k - 1; i++) {
-                    const uint8_t ch = s[i];
-                    if (!ascii_acgt(ch)) last_bad = (int64_t)i;
-                    const uint64_t c = ascii_code(ch);
-                    fw = (fw >> 2) | (c << (2 * (k - 1)));
-                    rc = ((rc << 2) | (c ^ 2)) & mask;
-                    if (i + 1 >= j0 + k && last_bad < (int64_t)(i + 1 - k)) on_key(fw < rc ? fw : rc, 0);
-                }
-            } else if (A.kind == 0) {
-                const u128_t mask = (k == 64) ? ~(u128_t)0 : (((u128_t)1 << (2 * k)) - 1);
-                u128_t fw = 0, rc = 0;
-                for (uint64_t i = j0; i < j1 + k - 1; i++) {
-                    const uint8_t ch = s[i];
-                    if (!ascii_acgt(ch)) last_bad = (int64_t)i;
-                    const u128_t c = ascii_code(ch);
-                    fw = (fw >> 2) | (c << (2 * (k - 1)));
-                    rc = ((rc << 2) | (c ^ 2)) & mask;
-                    if (i + 1 >= j0 + k && last_bad < (int64_t)(i + 1 - k)) {
-                        const u128_t key = fw < rc ? fw : rc;
-                        on_key((uint64_t)key, (uint64_t)(key >> 64));
-                    }
-                }
-            } else {
-                // rabin-karp128 rolling (crates/hashes/src/base/cn_rkhash_base.rs:65-110)
-                u128_t fh = 0, bk = 0;
-                for (uint64_t i = j0; i + 1 < j0 + k; i++) {
-                    if (!ascii_acgt(s[i])) last_bad = (int64_t)i;
-                    fh = fh * A.rk_mult + A.rk_fwd[ascii_code(s[i])];
-                }
-                for (int64_t i = (int64_t)(j0 + k) - 2; i >= (int64_t)j0; i--) bk = bk * A.rk_mult + A.rk_bkw[ascii_code(s[i])];
-                bk = bk * A.rk_mult;
-                for (uint64_t idx = j0 + k - 1; idx < j1 + k - 1; idx++) {
-                    if (!ascii_acgt(s[idx])) last_bad = (int64_t)idx;
-                    const uint32_t in = ascii_code(s[idx]), out = ascii_code(s[idx - (k - 1)]);
-                    const u128_t cur_f = fh * A.rk_mult + A.rk_fwd[in];
-                    fh = cur_f - A.rk_fwd_rm[out];
-                    const u128_t cur_b = bk * A.rk_mult_inv + A.rk_bkw_rm[in];
-                    bk = cur_b - A.rk_bkw[out];
-                    if (last_bad < (int64_t)(idx + 1 - k)) {
-                        const u128_t key = cur_f < cur_b ? cur_f : cur_b;
-                        on_key((uint64_t)key, (uint64_t)(key >> 64));
-                    }
-                }
+    uint32_t* counts = reinterpret_cast<uint32_t*>(lds);  // [n_colors] of the current query
+    // 16 positions per chunk: the span, up to 15 bytes before it, k - 1 behind
+    // it, and chunks that the reads of whole words run into
+    constexpr uint32_t CHUNKS = (15 + QUERY_SPAN + 63 + 15) / 16 + 6;
+    __shared__ uint32_t pk[CHUNKS];
+    __shared__ uint32_t inv[CHUNKS / 2 + 1], nl[CHUNKS / 2 + 1];
+    const uint32_t k = A.k, lane = threadIdx.x;
+    const uint64_t p0 = (uint64_t)blockIdx.x * A.span;
+    const uint32_t n_pos = A.n - p0 < A.span ? (uint32_t)(A.n - p0) : A.span;
+    const uint32_t mis = (uint32_t)(reinterpret_cast<uintptr_t>(A.seq + p0) & 15);  // chunks are 16-byte aligned
+    const uint32_t n_chunks = (mis + n_pos + k - 1 + 15) / 16;
+    for (uint32_t c = lane; c < n_chunks + 6; c += 64) {
+        const int64_t a = (int64_t)p0 - mis + 16 * (int64_t)c;
+        uint32_t packed = 0, bad = 0, ends = 0;
+        if (c < n_chunks && a >= 0 && a + 16 <= (int64_t)A.n) {
+            const uint4 v = *reinterpret_cast<const uint4*>(A.seq + a);
+            const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+            for (uint32_t i = 0; i < 16; i++) {
+                const uint8_t ch = (uint8_t)(w[i >> 2] >> (8 * (i & 3)));
+                packed |= ascii_code(ch) << (2 * i);
+                bad |= (ascii_acgt(ch) ? 0u : 1u) << i;
+                ends |= (ch == '\n' ? 1u : 0u) << i;
             }
-            if (A.color_words) flush_run(A, run_pos, run_cnt, counts);
+        } else {
+            for (uint32_t i = 0; i < 16; i++) {
+                const uint8_t ch =
+                    c < n_chunks && a + i >= 0 && a + i < (int64_t)A.n ? A.seq[a + i] : (uint8_t)0;
+                packed |= ascii_code(ch) << (2 * i);
+                bad |= (ascii_acgt(ch) ? 0u : 1u) << i;
+                ends |= (ch == '\n' ? 1u : 0u) << i;
+            }
         }
-        if (hits) atomicAdd(&s_matched, (unsigned long long)hits);
-        __syncthreads();
-        if (threadIdx.x == 0) A.matched[q] = s_matched;
-        for (uint32_t c = threadIdx.x; c < A.n_colors; c += blockDim.x)
-            A.color_counts[(uint64_t)q * A.n_colors + c] = counts[c];
-        __syncthreads();
+        pk[c] = packed;
+        reinterpret_cast<uint16_t*>(inv)[c] = (uint16_t)bad;
+        reinterpret_cast<uint16_t*>(nl)[c] = (uint16_t)ends;
     }
+    for (uint32_t c = lane; c < A.n_colors; c += 64) counts[c] = 0;
+    // the query holding the first position: the last one starting at or before
+    // it, 64 candidates per step
+    uint32_t q = 0;
+    for (uint32_t hi = A.n_queries; hi - q > 1;) {
+        const uint32_t step = (hi - q + 63) / 64;
+        const uint64_t at = q + (uint64_t)(lane + 1) * step;
+        const uint32_t m = (uint32_t)__popcll(__ballot(at < hi && A.qoff[at] <= p0));
+        q += m * step;
+        hi = hi - q < step ? hi : q + step;
+    }
+    __syncthreads();
+    uint32_t cnt = 0;  // hits of query q so far
+    auto flush = [&]() {
+        if (!cnt) return;
+        if (lane == 0) atomicAdd(reinterpret_cast<unsigned long long*>(&A.matched[q]), (unsigned long long)cnt);
+        for (uint32_t c = lane; c < A.n_colors; c += 64) {
+            if (counts[c]) atomicAdd(&A.color_counts[(uint64_t)q * A.n_colors + c], counts[c]);
+            counts[c] = 0;
+        }
+        cnt = 0;
+    };
+    for (uint32_t i0 = 0; i0 < n_pos; i0 += 64) {
+        const uint32_t i = i0 + lane, r = mis + i;
+        uint32_t pos = NO_POS;
+        bool end = false;
+        if (i < n_pos) {
+            end = (nl[r >> 5] >> (r & 31)) & 1;
+            if ((bits64(inv, r) & (~0ULL >> (64 - k))) == 0) {
+                uint64_t lo, hi = 0;
+                bool fwd;
+                if (KIND == 0) {
+                    lo = kmer_at(pk, r, k, &fwd);
+                } else {
+                    u128_t fw, rc;
+                    kmer_pair_at(pk, r, k, &fw, &rc);
+                    const u128_t key = KIND == 2 ? rk_of_kmer(A.rk_tri, k, fw, &fwd) : fw < rc ? fw : rc;
+                    lo = (uint64_t)key;
+                    hi = (uint64_t)(key >> 64);
+                }
+                pos = index_lookup(A, lo, hi);
+            }
+        }
+        const uint64_t hits = __ballot(pos != NO_POS), ends = __ballot(end);
+        uint64_t heads = 0;
+        if (A.color_words) {
+            // a hit whose color set is that of the hit one position before
+            // continues its run
+            bool same = lane && pos != NO_POS && ((hits >> (lane - 1)) & 1);
+            for (uint32_t w = 0; w < A.color_words; w++) {
+                const uint32_t x = pos != NO_POS ? A.out_colors[(uint64_t)pos * A.color_words + w] : 0u;
+                if (lane_prev32(x) != x) same = false;
+            }
+            heads = __ballot(pos != NO_POS && !same);
+        }
+        // the 64 positions' queries in turn
+        uint64_t left = ~0ULL, e = ends;
+        while (true) {
+            const uint64_t upto = e ? e ^ (e - 1) : ~0ULL;  // positions up to the next newline
+            const uint64_t part = left & upto;
+            cnt += (uint32_t)__popcll(hits & part);
+            for (uint64_t h = heads & part; h; h &= h - 1) {
+                const uint32_t b = (uint32_t)__builtin_ctzll(h);
+                const uint64_t more = b == 63 ? 0 : (hits & ~heads) >> (b + 1);  // hits that continue the run
+                const uint32_t len = 1 + (uint32_t)__builtin_ctzll(~more);
+                const uint32_t hp = (uint32_t)__shfl((int)pos, (int)b);
+                for (uint32_t c = lane; c < A.n_colors; c += 64)
+                    counts[c] += ((A.out_colors[(uint64_t)hp * A.color_words + (c >> 5)] >> (c & 31)) & 1u) * len;
+            }
+            if (!e) break;
+            flush();
+            q++;
+            left = ~upto;
+            e &= e - 1;
+        }
+    }
+    flush();
 }
 
 }  // namespace gg
