@@ -91,8 +91,8 @@ struct ggcat_gpu_ctx {
     DevBuf q_seq, q_off, q_matched, q_counts;
     struct Server* server = nullptr;
     // unitig chains
-    DevBuf u_nb, u_ext, u_link, u_hbytes, u_hcount, u_hoff, u_hidx, u_seq, u_sub, u_flags, u_visited, u_rest,
-        u_rest_n, u_rep, u_tab;
+    DevBuf u_nb, u_ext, u_link, u_seg, u_head, u_uhead, u_ubytes, u_uoff, u_seq, u_sub, u_flags, u_visited, u_rest,
+        u_rest_n, u_totals, u_rep, u_tab;
     bool have_unitigs = false;
     bool u_joined = false;
     uint64_t u_n = 0, u_bytes = 0, u_npos = 0;
@@ -528,8 +528,8 @@ void ggcat_gpu_destroy(ggcat_gpu_ctx* ctx) {
                       &ctx->fix_val, &ctx->fix_sub, &ctx->fix_cursor, &ctx->out_colors, &ctx->fix_colors,
                       &ctx->idx_slots, &ctx->idx_count,
                       &ctx->q_seq, &ctx->q_off, &ctx->q_matched, &ctx->q_counts,
-                      &ctx->u_nb, &ctx->u_ext, &ctx->u_link, &ctx->u_hbytes, &ctx->u_hcount, &ctx->u_hoff,
-                      &ctx->u_hidx, &ctx->u_seq, &ctx->u_sub, &ctx->u_flags, &ctx->u_visited, &ctx->u_rest,
+                      &ctx->u_nb, &ctx->u_ext, &ctx->u_link, &ctx->u_seg, &ctx->u_head, &ctx->u_uhead,
+                      &ctx->u_ubytes, &ctx->u_uoff, &ctx->u_totals, &ctx->u_seq, &ctx->u_sub, &ctx->u_flags, &ctx->u_visited, &ctx->u_rest,
                       &ctx->u_rest_n, &ctx->u_rep, &ctx->u_tab, &ctx->u_path, &ctx->stage_slots, &ctx->stage_unit,
                       &ctx->stage_rank, &ctx->stage_color, &ctx->stage_cursor, &ctx->defer, &ctx->defer_count,
                       &ctx->kmer_total, &ctx->spill_slots, &ctx->spill_color, &ctx->raw, &ctx->p_stats,
@@ -2403,10 +2403,12 @@ static int build_unitigs(ggcat_gpu_ctx* ctx, bool joined, uint64_t* n_unitigs, u
     ENSURE(ctx->u_nb, ne * 4 + 8);
     ENSURE(ctx->u_link, ne * 4 + 8);
     ENSURE(ctx->u_ext, n_pos + 8);
-    ENSURE(ctx->u_hbytes, ne * 4 + 8);
-    ENSURE(ctx->u_hcount, ne * 4 + 8);
-    ENSURE(ctx->u_hoff, (ne + 1) * 8);
-    ENSURE(ctx->u_hidx, (ne + 1) * 8);
+    const uint64_t n_seg = 2 * ((n_pos + SPLIT - 1) / SPLIT);
+    ENSURE(ctx->u_seg, n_seg * 8 + 8);
+    ENSURE(ctx->u_head, ne * 8 + 8);
+    ENSURE(ctx->u_uhead, n_pos * 4 + 8);
+    ENSURE(ctx->u_ubytes, n_pos * 4 + 8);
+    ENSURE(ctx->u_totals, 24);
     ENSURE(ctx->u_visited, n_pos + 8);
     ENSURE(ctx->u_rest_n, 8);
     ENSURE(ctx->u_rep, n_pos + 8);
@@ -2425,40 +2427,48 @@ static int build_unitigs(ggcat_gpu_ctx* ctx, bool joined, uint64_t* n_unitigs, u
     U.nb = P_<uint32_t>(ctx->u_nb);
     U.ext = P_<uint8_t>(ctx->u_ext);
     U.link = P_<uint32_t>(ctx->u_link);
-    U.head_bytes = P_<uint32_t>(ctx->u_hbytes);
-    U.head_count = P_<uint32_t>(ctx->u_hcount);
-    U.head_off = P_<uint64_t>(ctx->u_hoff);
-    U.head_idx = P_<uint64_t>(ctx->u_hidx);
+    U.seg = P_<uint64_t>(ctx->u_seg);
+    U.head = P_<uint64_t>(ctx->u_head);
+    U.uni_of = U.nb;  // the neighbours are not read once the links are made
+    U.uni_head = P_<uint32_t>(ctx->u_uhead);
+    U.uni_bytes = P_<uint32_t>(ctx->u_ubytes);
+    U.totals = P_<unsigned long long>(ctx->u_totals);
     U.visited = P_<uint8_t>(ctx->u_visited);
     U.global = joined ? 1u : 0u;
     U.rep = P_<uint8_t>(ctx->u_rep);
-    U.n_nodes = P_<unsigned int>(ctx->u_rest_n) + 1;
     U.mark_visited = 0;
     const uint32_t grid = (uint32_t)std::min<uint64_t>((ne + 255) / 256 + 1, (uint64_t)ctx->n_cu * 16);
     HIPCHK(hipEventRecord(ctx->ev[11], ctx->stream));
-    HIPCHK(hipMemsetAsync(ctx->u_rest_n.p, 0, 8, ctx->stream));  // [0] cycle nodes, [1] graph nodes
+    HIPCHK(hipMemsetAsync(ctx->u_rest_n.p, 0, 8, ctx->stream));  // cycle nodes
+    HIPCHK(hipMemsetAsync(ctx->u_totals.p, 0, 24, ctx->stream));
     if (n_pos) {
         HIPCHK(hipMemsetAsync(ctx->u_tab.p, 0, tab_slots * 8, ctx->stream));
+        if (joined) HIPCHK(hipMemsetAsync(ctx->u_rep.p, 1, n_pos, ctx->stream));
         hipLaunchKernelGGL(utab_insert_kernel, dim3(grid), dim3(256), 0, ctx->stream, U, n_pos);
-        if (joined) hipLaunchKernelGGL(rep_kernel, dim3(grid), dim3(256), 0, ctx->stream, U, n_pos);
         hipLaunchKernelGGL(ext_kernel, dim3(grid), dim3(256), 0, ctx->stream, U, n_pos);
         hipLaunchKernelGGL(link_kernel, dim3(grid), dim3(256), 0, ctx->stream, U, n_pos);
-        hipLaunchKernelGGL(walk_kernel<false>, dim3(grid), dim3(256), 0, ctx->stream, U, n_pos);
+        hipLaunchKernelGGL(seg_walk_kernel, dim3(grid), dim3(256), 0, ctx->stream, U, n_pos);
+        // each round multiplies how far every splitter's pair leads by at
+        // least SEG_HOPS + 1, until the n_seg / 2 splitters of the longest
+        // path are behind it
+        const uint32_t jgrid = (uint32_t)std::min<uint64_t>((n_seg + 255) / 256, (uint64_t)ctx->n_cu * 16);
+        for (uint64_t reach = 1; reach < n_seg / 2 + 1; reach *= SEG_HOPS + 1)
+            hipLaunchKernelGGL(seg_jump_kernel, dim3(jgrid), dim3(256), 0, ctx->stream, U, n_pos);
+        const uint32_t hgrid = (uint32_t)std::min<uint64_t>((ne + 1023) / 1024, (uint64_t)ctx->n_cu * 8);
+        hipLaunchKernelGGL(head_kernel, dim3(hgrid), dim3(256), 0, ctx->stream, U, n_pos);
         HIPCHK(hipGetLastError());
     }
-    int r = device_scan(ctx, U.head_bytes, P_<uint64_t>(ctx->u_hoff), (uint32_t)ne);
-    if (r != GGCAT_GPU_OK) return r;
-    r = device_scan(ctx, U.head_count, P_<uint64_t>(ctx->u_hidx), (uint32_t)ne);
-    if (r != GGCAT_GPU_OK) return r;
-    uint64_t tot_bytes = 0, tot_n = 0;
-    uint32_t counts[2] = {0, 0};
-    HIPCHK(hipMemcpyAsync(&tot_bytes, P_<uint64_t>(ctx->u_hoff) + ne, 8, hipMemcpyDeviceToHost, ctx->stream));
-    HIPCHK(hipMemcpyAsync(&tot_n, P_<uint64_t>(ctx->u_hidx) + ne, 8, hipMemcpyDeviceToHost, ctx->stream));
-    HIPCHK(hipMemcpyAsync(counts, ctx->u_rest_n.p, 8, hipMemcpyDeviceToHost, ctx->stream));
+    uint64_t totals[3] = {0, 0, 0};  // unitigs, bytes, duplicate entries
+    HIPCHK(hipMemcpyAsync(totals, ctx->u_totals.p, 24, hipMemcpyDeviceToHost, ctx->stream));
     HIPCHK(hipStreamSynchronize(ctx->stream));
+    const uint64_t tot_n = totals[0], tot_bytes = totals[1];
+    ENSURE(ctx->u_uoff, (tot_n + 1) * 8);
+    U.uni_off = P_<uint64_t>(ctx->u_uoff);
+    const int r = device_scan(ctx, U.uni_bytes, P_<uint64_t>(ctx->u_uoff), (uint32_t)tot_n);
+    if (r != GGCAT_GPU_OK) return r;
     // Paths cover every node unless there are cycles: only then are the path
     // nodes marked, so that the remaining ones can be collected.
-    const uint64_t n_nodes = joined ? counts[1] : n_pos;
+    const uint64_t n_nodes = n_pos - totals[2];
     const bool cycles = tot_bytes - (uint64_t)ctx->P.k * tot_n != n_nodes;
     U.mark_visited = cycles ? 1u : 0u;
     ENSURE(ctx->u_seq, tot_bytes + 8);
@@ -2476,7 +2486,7 @@ static int build_unitigs(ggcat_gpu_ctx* ctx, bool joined, uint64_t* n_unitigs, u
     const uint32_t cap = 1u << 20;
     ENSURE(ctx->u_rest, (size_t)cap * 4);
     if (n_pos) {
-        hipLaunchKernelGGL(walk_kernel<true>, dim3(grid), dim3(256), 0, ctx->stream, U, n_pos);
+        hipLaunchKernelGGL(seg_write_kernel, dim3(grid), dim3(256), 0, ctx->stream, U, n_pos);
         if (cycles)
             hipLaunchKernelGGL(unvisited_kernel, dim3(grid), dim3(256), 0, ctx->stream, U, n_pos,
                                P_<uint32_t>(ctx->u_rest), P_<unsigned int>(ctx->u_rest_n), cap);

@@ -43,20 +43,22 @@ struct UnitigArgs {
     uint32_t* nb;  // [2 n_pos] only neighbour (q << 1 | t) or NO_LINK
     uint8_t* ext;  // [n_pos] degree side 0 (0, 1, 2 = more) | degree side 1 << 2
     uint32_t* link;  // [2 n_pos]
-    uint32_t* head_bytes;  // [2 n_pos] bytes of the unitig written from this end (0 if not its start)
-    uint32_t* head_count;  // [2 n_pos] 1 when the unitig starts here
-    const uint64_t* head_off;  // [2 n_pos + 1] exclusive scan of head_bytes
-    const uint64_t* head_idx;  // [2 n_pos + 1] exclusive scan of head_count
+    uint64_t* seg;  // [2 groups of SPLIT positions] rest of the path behind each splitter, see seg_pair
+    uint64_t* head;  // [2 n_pos] the same for path ends (other entries unused)
+    uint32_t* uni_of;  // [2 n_pos] unitig written from this end, NO_LINK when written from its other end
+    uint32_t* uni_head;  // [unitigs] the end it is written from
+    uint32_t* uni_bytes;  // [unitigs]
+    const uint64_t* uni_off;  // [unitigs + 1] exclusive scan of uni_bytes
+    unsigned long long* totals;  // unitigs, bytes, duplicate entries (joined mode)
     uint8_t* seq;
     uint32_t* uni_sub;
     uint8_t* uni_flags;
     uint8_t* visited;  // [n_pos]
     uint32_t global;  // joined mode: one graph over all sub-buckets
     uint8_t* rep;  // [n_pos] joined mode: 1 where p is its key's smallest position
-    unsigned int* n_nodes;  // joined mode: number of representatives
     uint32_t mark_visited;  // write pass: mark path nodes (needed only when cycles exist)
     uint32_t* path_pos;  // write pass, optional: the table position of every k-mer of every unitig, in
-                         // written order (unitig i's k-mers start at head_off - i * k)
+                         // written order (unitig i's k-mers start at uni_off[i] - i * k)
 };
 
 // Position p is a node of the graph being compacted.
@@ -87,56 +89,53 @@ GG_DEV bool side_flagged(const UnitigArgs& A, uint64_t p, uint32_t s) {
     return (fl == 1 && s == 0) || (fl == 2 && s == 1);
 }
 
-// Every position goes into the lookup table (linear probing; the
-// table has at least twice as many slots as positions, so probing ends).
-__global__ void utab_insert_kernel(UnitigArgs A, uint64_t n_pos) {
+// Every position goes into the lookup table (linear probing; the table has at
+// least twice as many slots as positions, so probing ends).  In joined mode a
+// key's second entry is found here: the slot keeps the smaller position, the
+// other one stops being a representative (rep starts at 1 everywhere) and is
+// counted, so each key has one slot and a lookup ends at its first match.
+__global__ __launch_bounds__(256) void utab_insert_kernel(UnitigArgs A, uint64_t n_pos) {
+    __shared__ unsigned int part[4];
+    unsigned int dup = 0;
     for (uint64_t p = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; p < n_pos;
          p += (uint64_t)gridDim.x * blockDim.x) {
         const u128_t c = key_at(A, p);
         const uint64_t h = index_hash((uint64_t)c, (uint64_t)(c >> 64));
-        const uint64_t v = (h & 0xFFFFFFFF00000000ULL) | (p + 1);
-        for (uint64_t i = h & A.tab_mask;; i = (i + 1) & A.tab_mask)
-            if (atomicCAS(reinterpret_cast<unsigned long long*>(A.tab + i), 0ULL, (unsigned long long)v) == 0ULL) break;
+        const unsigned long long v = (h & 0xFFFFFFFF00000000ULL) | (p + 1);
+        for (uint64_t i = h & A.tab_mask;; i = (i + 1) & A.tab_mask) {
+            unsigned long long* slot = reinterpret_cast<unsigned long long*>(A.tab + i);
+            const unsigned long long cur = atomicCAS(slot, 0ULL, v);
+            if (cur == 0ULL) break;
+            // a slot's key never changes, only which of its positions it names
+            if (A.global && (uint32_t)(cur >> 32) == (uint32_t)(v >> 32) && key_at(A, (uint32_t)cur - 1u) == c) {
+                const unsigned long long old = atomicMin(slot, v);
+                A.rep[old > v ? (uint32_t)old - 1u : (uint32_t)p] = 0;
+                dup++;
+                break;
+            }
+        }
+    }
+    if (!A.global) return;
+    for (uint32_t d = 32; d; d >>= 1) dup += __shfl_down(dup, d);
+    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = dup;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        const unsigned int t = part[0] + part[1] + part[2] + part[3];
+        if (t) atomicAdd(A.totals + 2, (unsigned long long)t);
     }
 }
 
 // Position of key `c` inside sub-bucket `sub`, or NO_LINK.  In joined mode
-// the sub-bucket is ignored and the key's smallest position is returned.
+// the sub-bucket is ignored and the key's representative is returned.
 GG_DEV uint32_t lookup_in_sub(const UnitigArgs& A, u128_t c, uint32_t sub) {
     const uint64_t h = index_hash((uint64_t)c, (uint64_t)(c >> 64));
     const uint32_t fp = (uint32_t)(h >> 32);
-    uint32_t best = NO_LINK;
     for (uint64_t i = h & A.tab_mask;; i = (i + 1) & A.tab_mask) {
         const uint64_t v = A.tab[i];
-        if (v == 0) break;
+        if (v == 0) return NO_LINK;
         if ((uint32_t)(v >> 32) != fp) continue;
         const uint32_t q = (uint32_t)v - 1u;
-        if (key_at(A, q) != c) continue;
-        if (!A.global) {
-            if (A.out_sub[q] == sub) return q;
-        } else if (q < best) {
-            best = q;
-        }
-    }
-    return best;
-}
-
-// Joined mode: marks each position that is its key's smallest one.
-// Counts them into *n_nodes (blocks of 256 threads: one atomic per block).
-__global__ __launch_bounds__(256) void rep_kernel(UnitigArgs A, uint64_t n_pos) {
-    __shared__ unsigned int part[4];
-    unsigned int cnt = 0;
-    for (uint64_t p = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; p < n_pos; p += (uint64_t)gridDim.x * blockDim.x) {
-        const bool r = lookup_in_sub(A, key_at(A, p), 0) == (uint32_t)p;
-        A.rep[p] = r;
-        cnt += r ? 1u : 0u;
-    }
-    for (uint32_t d = 32; d; d >>= 1) cnt += __shfl_down(cnt, d);
-    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = cnt;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        const unsigned int t = part[0] + part[1] + part[2] + part[3];
-        if (t) atomicAdd(A.n_nodes, t);
+        if (key_at(A, q) == c && (A.global || A.out_sub[q] == sub)) return q;
     }
 }
 
@@ -222,63 +221,189 @@ struct SeqWriter {
     }
 };
 
-// Pass 1 (write == false): every end of a path walks to its other end; the
-// end with the smaller (key, side) records the unitig's bytes.  Pass 2
-// (write == true): those ends write the sequence, its sub-bucket and flags.
-template <bool WRITE>
-__global__ void walk_kernel(UnitigArgs A, uint64_t n_pos) {
+// ---- paths ------------------------------------------------------------------
+// A path is walked along directed elements e = 2 p + side entered; the next one
+// is link[e ^ 1].  Walking a whole path by one thread costs its length times
+// the latency of a dependent read (one error-free genome is one path), so paths
+// are cut at splitters: one position in each group of SPLIT, chosen by a hash.
+// Every splitter and every path end walks to the next splitter (SPLIT nodes on
+// average), splitters then jump over each other (pointer doubling on 1 / SPLIT
+// of the nodes), after which every end knows its path's length and other end,
+// and the segments write their part of the unitig, all at once.
+// 14.4 M entries, joined: lengths and ends 1.5 -> 1.2 ms, writing 2.9 -> 2.0 ms
+// (now bound by a random link and key read per node); one path of 400 K nodes
+// no longer sets the time.
+constexpr uint32_t SPLIT = 16;
+
+GG_DEV uint64_t split_pos(uint64_t group) { return group * SPLIT + (mix64(group) & (SPLIT - 1)); }
+GG_DEV bool is_split(uint64_t p) { return split_pos(p / SPLIT) == p; }
+
+// From an element: nodes up to `to` (exclusive of it while not done), and
+// whether the path ends there: `to` is then the path's last element, else the
+// next splitter's.
+constexpr uint32_t SEG_DONE = 1u << 31;
+GG_DEV uint64_t seg_pair(uint32_t nodes, bool done, uint32_t to) {
+    return ((uint64_t)(nodes | (done ? SEG_DONE : 0u)) << 32) | to;
+}
+GG_DEV bool seg_done(uint64_t x) { return (x >> 63) != 0; }
+GG_DEV uint32_t seg_nodes(uint64_t x) { return (uint32_t)(x >> 32) & ~SEG_DONE; }
+// x followed by y, the pair of the element x leads to (cycles never end: their
+// count wraps inside its 31 bits and is not used)
+GG_DEV uint64_t seg_join(uint64_t x, uint64_t y) {
+    return seg_pair((seg_nodes(x) + seg_nodes(y)) & ~SEG_DONE, seg_done(y), (uint32_t)y);
+}
+GG_DEV uint64_t* seg_of(const UnitigArgs& A, uint64_t e) { return A.seg + 2 * ((e >> 1) / SPLIT) + (e & 1); }
+
+// Every splitter and path end to the next splitter or the path's end.
+__global__ void seg_walk_kernel(UnitigArgs A, uint64_t n_pos) {
+    for (uint64_t e = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; e < 2 * n_pos;
+         e += (uint64_t)gridDim.x * blockDim.x) {
+        const bool split = is_split(e >> 1), head = A.link[e] == NO_LINK;
+        if ((!split && !head) || !unitig_valid(A, e >> 1)) continue;
+        uint64_t cur = e, x = 0;
+        for (uint32_t nodes = 1;; nodes++) {
+            const uint32_t nx = A.link[cur ^ 1];
+            if (nx == NO_LINK || is_split(nx >> 1)) {
+                x = seg_pair(nodes, nx == NO_LINK, nx == NO_LINK ? (uint32_t)cur : nx);
+                break;
+            }
+            cur = nx;
+        }
+        if (split) *seg_of(A, e) = x;
+        if (head) A.head[e] = x;
+    }
+}
+
+// One round: every splitter's pair joined with those of the splitters it leads
+// to, up to SEG_HOPS times.  In place: a pair is one 8-byte word, and whatever
+// round's pair is read leads as far as it says.
+constexpr uint32_t SEG_HOPS = 8;
+__global__ void seg_jump_kernel(UnitigArgs A, uint64_t n_pos) {
+    const uint64_t n = 2 * ((n_pos + SPLIT - 1) / SPLIT);
+    for (uint64_t i = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x) {
+        const uint64_t p = split_pos(i >> 1);
+        if (p >= n_pos || !unitig_valid(A, p)) continue;
+        uint64_t x = A.seg[i];
+        if (seg_done(x)) continue;
+        for (uint32_t h = 0; h < SEG_HOPS && !seg_done(x); h++)
+            x = seg_join(x, __hip_atomic_load(seg_of(A, (uint32_t)x), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+        atomicExch(reinterpret_cast<unsigned long long*>(A.seg + i), (unsigned long long)x);
+    }
+}
+
+// Path ends: the end with the smaller (key, side) becomes the head of a unitig
+// (listed in arrival order, with its bytes: k-mer, one base per further k-mer,
+// '\n').  Each thread takes two positions; one atomic per workgroup and step.
+__global__ __launch_bounds__(256) void head_kernel(UnitigArgs A, uint64_t n_pos) {
+    __shared__ uint32_t wave_n[4];
+    __shared__ uint32_t s_base;
+    __shared__ unsigned long long s_bytes[4];
+    const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6, k = A.k;
+    const uint64_t ne = 2 * n_pos, step = (uint64_t)gridDim.x * 1024;
+    unsigned long long bytes = 0;
+    for (uint64_t e0 = (uint64_t)blockIdx.x * 1024; e0 < ne; e0 += step) {
+        uint32_t len[4], n = 0;
+#pragma unroll
+        for (uint32_t j = 0; j < 4; j++) {
+            const uint64_t e = e0 + 4 * threadIdx.x + j;
+            len[j] = 0;
+            if (e >= ne || A.link[e] != NO_LINK || !unitig_valid(A, e >> 1)) continue;
+            uint64_t x = A.head[e];
+            if (!seg_done(x)) x = seg_join(x, *seg_of(A, (uint32_t)x));
+            A.head[e] = x;
+            const uint64_t p = e >> 1, last = (uint32_t)x, q = last >> 1;
+            const u128_t kp = key_at(A, p), kq = key_at(A, q);
+            const bool canon = kp < kq || (kp == kq && (uint32_t)(e & 1) < (uint32_t)((last ^ 1) & 1));
+            if (canon) {
+                len[j] = seg_nodes(x) + k;
+                bytes += len[j];
+                n++;
+            } else {
+                A.uni_of[e] = NO_LINK;
+            }
+        }
+        uint32_t inc = n;
+        for (uint32_t d = 1; d < 64; d <<= 1) {
+            const uint32_t y = __shfl_up(inc, d);
+            if (lane >= d) inc += y;
+        }
+        if (lane == 63) wave_n[wave] = inc;
+        __syncthreads();
+        uint32_t before = 0, all = 0;
+        for (uint32_t w = 0; w < 4; w++) {
+            if (w < wave) before += wave_n[w];
+            all += wave_n[w];
+        }
+        if (threadIdx.x == 0) s_base = all ? (uint32_t)atomicAdd(A.totals, (unsigned long long)all) : 0u;
+        __syncthreads();
+        uint32_t i = s_base + before + inc - n;
+#pragma unroll
+        for (uint32_t j = 0; j < 4; j++) {
+            if (!len[j]) continue;
+            const uint64_t e = e0 + 4 * threadIdx.x + j;
+            A.uni_head[i] = (uint32_t)e;
+            A.uni_bytes[i] = len[j];
+            A.uni_of[e] = i++;
+        }
+        __syncthreads();  // wave_n and s_base are reused
+    }
+    for (uint32_t d = 32; d; d >>= 1) bytes += __shfl_down(bytes, d);
+    if (lane == 0) s_bytes[wave] = bytes;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        const unsigned long long t = s_bytes[0] + s_bytes[1] + s_bytes[2] + s_bytes[3];
+        if (t) atomicAdd(A.totals + 1, t);
+    }
+}
+
+// Every segment of a unitig writes its bases (its first node's place is the
+// path's length less what is left of it), the head's segment the first k-mer,
+// the last one the '\n'; segments against the unitig's direction write nothing.
+__global__ void seg_write_kernel(UnitigArgs A, uint64_t n_pos) {
     const uint32_t k = A.k;
+    constexpr uint32_t ASCII = 'A' | ('C' << 8) | ('T' << 16) | ('G' << 24);
     for (uint64_t e = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; e < 2 * n_pos;
          e += (uint64_t)gridDim.x * blockDim.x) {
         const uint64_t p = e >> 1;
         const uint32_t s = (uint32_t)(e & 1);
-        bool head = unitig_valid(A, p) && A.link[e] == NO_LINK;
-        if (!WRITE) {
-            uint32_t bytes = 0, cnt = 0;
-            if (head) {
-                uint64_t cur = e;
-                uint64_t steps = 1;
-                while (A.link[cur ^ 1] != NO_LINK && steps <= n_pos) {
-                    cur = A.link[cur ^ 1];
-                    steps++;
-                }
-                const uint64_t q = cur >> 1;
-                const uint32_t qs = (uint32_t)((cur ^ 1) & 1);
-                const u128_t kp = key_at(A, p), kq = key_at(A, q);
-                const bool canon = kp < kq || (kp == kq && s < qs);
-                if (canon) {
-                    bytes = (uint32_t)(steps + k);  // k-mer, one base per further k-mer, '\n'
-                    cnt = 1;
-                }
-            }
-            A.head_bytes[e] = bytes;
-            A.head_count[e] = cnt;
-            continue;
+        const bool is_head = A.link[e] == NO_LINK;
+        if ((!is_head && !is_split(p)) || !unitig_valid(A, p)) continue;
+        const uint64_t x = is_head ? A.head[e] : *seg_of(A, e);
+        if (!seg_done(x)) continue;  // on a cycle
+        // the path's last element entered from behind is the end of the
+        // opposite direction, whose last element is this direction's head
+        const uint32_t h = is_head ? (uint32_t)e : (uint32_t)A.head[(uint32_t)x ^ 1u] ^ 1u;
+        const uint32_t ui = A.uni_of[h];
+        if (ui == NO_LINK) continue;
+        const uint64_t off = A.uni_off[ui];
+        uint32_t j = seg_nodes(A.head[h]) - seg_nodes(x);  // index of node p in the path
+        SeqWriter out(A.seq, j ? off + k - 1 + j : off);
+        if (j == 0) {
+            const u128_t y = s == 0 ? key_at(A, p) : kmer_rc128(key_at(A, p), k);
+            for (uint32_t i = 0; i < k; i++) out.put((ASCII >> (8 * ((uint32_t)(y >> (2 * i)) & 3u))) & 0xFFu);
+            A.uni_sub[ui] = A.global ? 0u : A.out_sub[p];
+            const uint64_t last = (uint32_t)x;
+            A.uni_flags[ui] = (uint8_t)((side_flagged(A, p, s) ? 1u : 0u) |
+                                        (side_flagged(A, last >> 1, (uint32_t)((last ^ 1) & 1)) ? 2u : 0u));
+        } else {
+            out.put((ASCII >> (8 * entry_base(A, p, s))) & 0xFFu);
         }
-        if (!head || A.head_off[e + 1] == A.head_off[e]) continue;
-        SeqWriter out(A.seq, A.head_off[e]);
-        const uint64_t ui = A.head_idx[e];
-        constexpr uint32_t ASCII = 'A' | ('C' << 8) | ('T' << 16) | ('G' << 24);
-        const u128_t x = s == 0 ? key_at(A, p) : kmer_rc128(key_at(A, p), k);
-        for (uint32_t i = 0; i < k; i++) out.put((ASCII >> (8 * ((uint32_t)(x >> (2 * i)) & 3u))) & 0xFFu);
-        if (A.mark_visited) A.visited[p] = 1;
-        uint32_t* pp = A.path_pos ? A.path_pos + (A.head_off[e] - ui * k) : nullptr;
-        if (pp) *pp++ = (uint32_t)p;
+        uint32_t* pp = A.path_pos ? A.path_pos + (off - (uint64_t)ui * k) : nullptr;
         uint64_t cur = e;
-        // the count pass found this path's end within n_pos steps
-        for (uint64_t steps = 1; A.link[cur ^ 1] != NO_LINK && steps <= n_pos; steps++) {
-            cur = A.link[cur ^ 1];
+        while (true) {
             const uint64_t q = cur >> 1;
             if (A.mark_visited) A.visited[q] = 1;
-            if (pp) *pp++ = (uint32_t)q;
-            out.put((ASCII >> (8 * entry_base(A, q, (uint32_t)(cur & 1)))) & 0xFFu);
+            if (pp) pp[j++] = (uint32_t)q;
+            const uint32_t nx = A.link[cur ^ 1];
+            if (nx == NO_LINK) {
+                out.put('\n');
+                break;
+            }
+            if (is_split(nx >> 1)) break;
+            cur = nx;
+            out.put((ASCII >> (8 * entry_base(A, cur >> 1, (uint32_t)(cur & 1)))) & 0xFFu);
         }
-        out.put('\n');
         out.finish();
-        const uint64_t qend = cur >> 1;
-        const uint32_t exit_side = (uint32_t)((cur ^ 1) & 1);
-        A.uni_sub[ui] = A.global ? 0u : A.out_sub[p];
-        A.uni_flags[ui] = (uint8_t)((side_flagged(A, p, s) ? 1u : 0u) | (side_flagged(A, qend, exit_side) ? 2u : 0u));
     }
 }
 
