@@ -168,7 +168,8 @@ T* P_(DevBuf& b) {
 }
 
 // ntHash rolling tables, index out*4+in with out == 4 meaning "no base leaves"
-// (crates/hashes/src/nthash_base.rs:49-61 on 2-bit codes A=0,C=1,T=2,G=3).
+// (crates/hashes/src/nthash_base.rs:49-61 on 2-bit codes A=0,C=1,T=2,G=3);
+// entries 20 + (c0 | c1 << 2) take two bases at once, c0 first.
 void nthash_tables(uint32_t m, uint64_t* gtab) {
     auto rotl = [](uint64_t x, unsigned r) { r &= 63; return r ? (x << r) | (x >> (64 - r)) : x; };
     auto rotr = [](uint64_t x, unsigned r) { r &= 63; return r ? (x >> r) | (x << (64 - r)) : x; };
@@ -185,6 +186,11 @@ void nthash_tables(uint32_t m, uint64_t* gtab) {
             gtab[2 * e] = f;
             gtab[2 * e + 1] = r;
         }
+    }
+    for (uint32_t c = 0; c < 16; c++) {
+        const uint32_t e0 = 16 + (c & 3), e1 = 16 + (c >> 2);
+        gtab[2 * (20 + c)] = rotl(gtab[2 * e0], 1) ^ gtab[2 * e1];
+        gtab[2 * (20 + c) + 1] = rotr(gtab[2 * e0 + 1], 1) ^ gtab[2 * e1 + 1];
     }
 }
 

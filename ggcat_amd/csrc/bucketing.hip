@@ -36,6 +36,9 @@
 
 namespace gg {
 
+// 64-bit words of the rolling-hash tables (BucketArgs::gtab).
+constexpr uint32_t GTAB_WORDS = 2 * (20 + 16);
+
 // Records are scattered by physical unit: the sub-bucket (the semantic unit,
 // one kmers_transform job) refined by `xb` further bits of the minimizer hash
 // for unique minimizers.  Units of one sub-bucket are contiguous, so the merge
@@ -87,7 +90,9 @@ struct BucketArgs {
     uint32_t n_colors;
     uint32_t* slot_color;
     uint32_t* error_flag;  // set when a consistency check fails
-    uint64_t gtab[40];  // interleaved (fw, rc) rolling tables, index out*4+in
+    // interleaved (fw, rc) rolling tables: entries 0..19 index out*4+in, then
+    // two bases c0 | c1 << 2 that come in while none leaves
+    uint64_t gtab[GTAB_WORDS];
 };
 
 // m-mers of one tile: 16 per lane of its wavefront.
@@ -130,7 +135,7 @@ __host__ __device__ inline TileGeom tile_geom(uint32_t T, uint32_t w, uint32_t k
     uint32_t need = 48 + (TILE_MMERS + m > g.NW + k ? TILE_MMERS + m : g.NW + k);
     g.NB = (need + 31) / 32 * 32;
     uint32_t o = 0;
-    g.off_g = o; o += 40 * 8;
+    g.off_g = o; o += GTAB_WORDS * 8;
     g.off_px = o;
     g.off_wv = o;
     g.off_wp = (o + 64 * 17 * 4 + 7) / 8 * 8;
@@ -152,6 +157,26 @@ __host__ __device__ inline TileGeom tile_geom(uint32_t T, uint32_t w, uint32_t k
 GG_DEV bool is_acgt(uint8_t c) {
     uint8_t u = c & 0xDF;
     return u == 'A' || u == 'C' || u == 'G' || u == 'T';
+}
+
+// Four bytes at a time.  2-bit codes (bits 1..2 of each letter) as 8 bits.
+GG_DEV uint32_t codes4(uint32_t w) {
+    const uint32_t x = (w >> 1) & 0x03030303u, y = (x << 6) | (x << 12);
+    return (y | (y << 12)) >> 24;
+}
+// Bit j set when byte j of z is not zero.
+GG_DEV uint32_t nonzero4(uint32_t z) {
+    uint32_t f = (((z & 0x7F7F7F7Fu) + 0x7F7F7F7Fu) | z) & 0x80808080u;
+    f |= f << 7;
+    f |= f << 14;
+    return f >> 28;
+}
+// Bit j set when byte j is none of ACGTacgt: bits 1..2 of a byte name its
+// letter, whose bits 0 and 4 are those of 'A' for A, C and G and the opposite
+// for T; bits 3, 6 and 7 are those of 'A' for all, bit 5 is the case.
+GG_DEV uint32_t not_acgt4(uint32_t w) {
+    const uint32_t t = (w >> 2) & ~(w >> 1) & 0x01010101u;
+    return nonzero4((w ^ 0x41414141u ^ (t | (t << 4))) & 0xD9D9D9D9u);
 }
 
 struct Tile {
@@ -181,18 +206,15 @@ struct Tile {
     GG_DEV bool fwd_at(uint32_t p) const { return ((fwd16[p >> 4] >> (p & 15)) & 1u) != 0; }
 };
 
-// 16 codes of relative positions [r, r+16) packed (position r at bits 0..1);
-// positions below 0 read as zero.
+// Low 32 bits of hi:lo >> s, 0 <= s < 32 (one v_alignbit).
+GG_DEV uint32_t shift_pair(uint32_t lo, uint32_t hi, uint32_t s) { return ((hi << 1) << (s ^ 31u)) | (lo >> s); }
+
+// 16 codes of relative positions [r, r+16) packed (position r at bits 0..1), r
+// >= -16; positions below 0 read as whatever lies in front of the codes.
 GG_DEV uint32_t extract16(const Tile& t, int64_t r) {
-    if (r >= 0) {
-        uint32_t wi = (uint32_t)(r >> 4), s = (uint32_t)(r & 15) * 2;
-        uint32_t lo = t.pk[wi];
-        if (s == 0) return lo;
-        return (lo >> s) | (t.pk[wi + 1] << (32 - s));
-    }
-    if (r <= -16) return 0;
-    uint32_t sh = (uint32_t)(-r) * 2;
-    return t.pk[0] << sh;
+    const int32_t i = (int32_t)r;
+    const uint32_t* p = t.pk + (i >> 4);
+    return shift_pair(p[0], p[1], (i & 15) * 2);
 }
 
 GG_DEV uint32_t rev_comp16(uint32_t x) {
@@ -214,7 +236,7 @@ GG_DEV void tile_compute(Tile& t) {
     const TileGeom& G = t.G;
     const uint32_t lane = threadIdx.x;
 
-    for (uint32_t i = lane; i < 40; i += 64) t.gt[i] = A.gtab[i];
+    for (uint32_t i = lane; i < GTAB_WORDS; i += 64) t.gt[i] = A.gtab[i];
 
     // ---- phase 0: bases -> 2-bit codes + invalid bits --------------------
     const uint32_t nchunk = G.NB / 16;
@@ -223,17 +245,8 @@ GG_DEV void tile_compute(Tile& t) {
         uint32_t packed = 0, invm = 0;
         if (a >= 0 && a + 16 <= (int64_t)A.n) {
             uint4 v = *reinterpret_cast<const uint4*>(A.seq + a);
-            uint32_t wds[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-            for (int q = 0; q < 4; q++) {
-#pragma unroll
-                for (int bb = 0; bb < 4; bb++) {
-                    uint8_t ch = (wds[q] >> (8 * bb)) & 0xFF;
-                    uint32_t idx = q * 4 + bb;
-                    packed |= (uint32_t)((ch >> 1) & 3) << (2 * idx);
-                    invm |= (is_acgt(ch) ? 0u : 1u) << idx;
-                }
-            }
+            packed = codes4(v.x) | codes4(v.y) << 8 | codes4(v.z) << 16 | codes4(v.w) << 24;
+            invm = not_acgt4(v.x) | not_acgt4(v.y) << 4 | not_acgt4(v.z) << 8 | not_acgt4(v.w) << 12;
         } else {
             for (uint32_t idx = 0; idx < 16; idx++) {
                 int64_t p = a + idx;
@@ -256,9 +269,8 @@ GG_DEV void tile_compute(Tile& t) {
 // 64 bits of a bit array starting at bit `r` (r >= 0).
 GG_DEV uint64_t bits64(const uint32_t* a, int64_t r) {
     const uint32_t wi = (uint32_t)(r >> 5), sh = (uint32_t)(r & 31);
-    const uint64_t lo = (uint64_t)a[wi] | ((uint64_t)a[wi + 1] << 32);
-    if (sh == 0) return lo;
-    return (lo >> sh) | ((uint64_t)a[wi + 2] << (64 - sh));
+    const uint32_t w0 = a[wi], w1 = a[wi + 1], w2 = a[wi + 2];
+    return (uint64_t)shift_pair(w0, w1, sh) | (uint64_t)shift_pair(w1, w2, sh) << 32;
 }
 
 // Phases 1-3 for w == 16 and k <= 47, one window block of 16 per lane (NWB <=
@@ -268,6 +280,10 @@ GG_DEV uint64_t bits64(const uint32_t* a, int64_t r) {
 // combination of the two (van Herk / Gil-Werman in registers).  The window
 // flags of phase 3 are formed in the same pass from a 64-bit slice of the
 // invalid-base bitmap and written as 16-bit pieces.
+// Bound by the record part's atomics and 16-byte stores (17 G/s each), which
+// get slower the more wavefronts wait in them at once.  With the hashes, minima
+// and flags of tile_minima (28 % fewer VALU instructions) a wavefront reaches
+// them sooner and the pass of 1.6 Gbases takes 10.2 ms instead of 9.0.
 GG_DEV void tile_minima_w16(Tile& t) {
     const TileGeom& G = t.G;
     const uint32_t lane = threadIdx.x;
@@ -399,18 +415,41 @@ GG_DEV void tile_minima_w16(Tile& t) {
 //   fw_i = rotl1(fw_{i-1}) ^ rotl(h(s_{i-1}), m) ^ h(s_{i+m-1})
 //   rc_i = rotr1(rc_{i-1}) ^ rotr1(rc(s_{i-1})) ^ rotl(rc(s_{i+m-1}), m-1)
 // with the "out" term dropped while the first m bases are fed.
+// The hashes are kept as 32-bit halves: as 64-bit values the compiler rotates
+// them with 64-bit shifts, four times an alignbit's cost each.
+struct Halves {
+    uint32_t lo, hi;
+};
+template <int N>
+GG_DEV Halves rotl_xor(Halves x, uint64_t g) {
+    return {shift_pair(x.hi, x.lo, 32 - N) ^ (uint32_t)g, shift_pair(x.lo, x.hi, 32 - N) ^ (uint32_t)(g >> 32)};
+}
+template <int N>
+GG_DEV Halves rotr_xor(Halves x, uint64_t g) {
+    return {shift_pair(x.lo, x.hi, N) ^ (uint32_t)g, shift_pair(x.hi, x.lo, N) ^ (uint32_t)(g >> 32)};
+}
+GG_DEV uint64_t whole(Halves x) { return (uint64_t)x.hi << 32 | x.lo; }
+
 GG_DEV uint32_t hash_block16(const Tile& t, uint32_t p0, uint64_t* v) {
     const ulonglong2* gt2 = reinterpret_cast<const ulonglong2*>(t.gt);
     const int64_t rb = (int64_t)t.d0 + p0;
     const uint32_t m = t.A->m;
-    uint64_t fw = 0, rc = 0;
-    for (uint32_t j0 = 0; j0 + 1 < m; j0 += 16) {
-        const uint32_t c = extract16(t, rb + j0), n = m - 1 - j0 < 16 ? m - 1 - j0 : 16;
+    Halves fw{0u, 0u}, rc{0u, 0u};
+    // the first m - 1 bases two at a time, then the odd one
+    for (uint32_t j0 = 0; j0 + 2 < m; j0 += 16) {
+        uint32_t c = extract16(t, rb + j0);
+        const uint32_t n = m - 1 - j0 < 16 ? (m - 1 - j0) / 2 : 8;
         for (uint32_t j = 0; j < n; j++) {
-            const ulonglong2 g = gt2[16 + ((c >> (2 * j)) & 3u)];
-            fw = rotl1_64(fw) ^ g.x;
-            rc = rotr1_64(rc) ^ g.y;
+            const ulonglong2 g = gt2[20 + (c & 15u)];
+            fw = rotl_xor<2>(fw, g.x);
+            rc = rotr_xor<2>(rc, g.y);
+            c >>= 4;
         }
+    }
+    if ((m & 1) == 0) {
+        const ulonglong2 g = gt2[16 + t.code_rel(rb + m - 2)];
+        fw = rotl_xor<1>(fw, g.x);
+        rc = rotr_xor<1>(rc, g.y);
     }
     const uint32_t inw = extract16(t, rb + m - 1);
     const uint32_t outw = extract16(t, rb - 1);
@@ -419,11 +458,13 @@ GG_DEV uint32_t hash_block16(const Tile& t, uint32_t p0, uint64_t* v) {
     for (int i = 0; i < 16; i++) {
         const uint32_t in = (inw >> (2 * i)) & 3u, out = (outw >> (2 * i)) & 3u;
         const ulonglong2 g = gt2[(i == 0 ? 16u : out * 4u) + in];
-        fw = rotl1_64(fw) ^ g.x;
-        rc = rotr1_64(rc) ^ g.y;
-        const uint64_t mn = fw < rc ? fw : rc;
-        v[i] = (mn << 1) | (fw != rc ? 1ULL : 0ULL);
-        fbits |= (fw < rc ? 1u : 0u) << i;
+        fw = rotl_xor<1>(fw, g.x);
+        rc = rotr_xor<1>(rc, g.y);
+        const uint64_t f = whole(fw), r = whole(rc);
+        const bool less = f < r;
+        const Halves mn{less ? fw.lo : rc.lo, less ? fw.hi : rc.hi};
+        v[i] = whole({(mn.lo << 1) | (uint32_t)(f != r), shift_pair(mn.lo, mn.hi, 31)});
+        fbits |= (uint32_t)less << i;
     }
     return fbits;
 }
@@ -454,6 +495,12 @@ GG_DEV void window_flags16(const Tile& t, uint32_t p0, uint32_t* ok, uint32_t* f
     *last = l;
 }
 
+// Whether a window's minimum differs from the one of the window before (its
+// value, or its position when unique), as 0 or 1.
+GG_DEV uint32_t window_differs(uint64_t v, uint32_t p, uint64_t before_v, uint32_t before_p) {
+    return (uint32_t)(v != before_v) | ((uint32_t)v & (uint32_t)(p != before_p) & 1u);
+}
+
 // Bitmaps of the tile's windows from the lanes' 16-bit pieces; words past the
 // last window are zero.
 GG_DEV void write_bitmaps16(Tile& t, uint32_t segm, uint32_t okm, uint32_t lastm) {
@@ -467,6 +514,14 @@ GG_DEV void write_bitmaps16(Tile& t, uint32_t segm, uint32_t okm, uint32_t lastm
     }
 }
 
+// mm_combine by selects: its if / else becomes exec-mask branches, one to three
+// per combination.
+GG_DEV void mm_select(uint64_t av, uint32_t ap, uint64_t bv, uint32_t bp, uint64_t& rv, uint32_t& rp) {
+    const bool b = bv < av;
+    rv = (b ? bv : av) & (av == bv ? ~1ULL : ~0ULL);
+    rp = b ? bp : ap;
+}
+
 // Phases 1-3 for any w >= B: lane q hashes m-mers 16q .. 16q + 15 and keeps
 // the suffix minima of their blocks of B in registers; the blocks' prefix
 // minima go to LDS.  Window x = 16q + i covers the suffix of its block from
@@ -477,7 +532,9 @@ GG_DEV void write_bitmaps16(Tile& t, uint32_t segm, uint32_t okm, uint32_t lastm
 // each window costs one 64-bit LDS read and two or three combinations, on all
 // 64 lanes; LDS arrays of every m-mer and one lane per block of w before.
 // Bound by VALU issue (64-bit hashing and compares).  Staging pass of 0.9
-// Gbases at w = 42: 22.1 -> 5.4 ms; of 0.24 Gbases at w = 33: 5.5 -> 1.4 ms.
+// Gbases at w = 42: 22.1 -> 5.4 ms; of 0.24 Gbases at w = 33: 5.5 -> 1.4 ms;
+// with selects for branches, two bases per step of the first hash and four
+// input bytes at a time 5.4 -> 4.4 and 1.4 -> 1.2 ms.
 template <int B>
 GG_DEV void tile_minima(Tile& t) {
     const uint32_t q = threadIdx.x, p0 = 16 * q, w = t.A->w;
@@ -497,7 +554,7 @@ GG_DEV void tile_minima(Tile& t) {
                 pv = sv[i];
                 pp = i;
             } else {
-                mm_combine(pv, pp, sv[i], i, pv, pp);
+                mm_select(pv, pp, sv[i], i, pv, pp);
             }
             t.px[17 * q + i] = pv;
             nib |= (uint64_t)pp << (4 * i);
@@ -505,7 +562,7 @@ GG_DEV void tile_minima(Tile& t) {
         t.pn[q] = nib;
 #pragma unroll
         for (int i = 14; i >= 0; i--)
-            if (i % B != B - 1) mm_combine(sv[i], sp[i], sv[i + 1], sp[i + 1], sv[i], sp[i]);
+            if (i % B != B - 1) mm_select(sv[i], sp[i], sv[i + 1], sp[i + 1], sv[i], sp[i]);
     }
     __syncthreads();
     // window minima: low words, offsets, and where a window's minimum differs
@@ -530,34 +587,32 @@ GG_DEV void tile_minima(Tile& t) {
                     mv = bv;
                     mp = bp;
                 } else {
-                    mm_combine(mv, mp, bv, bp, mv, mp);
+                    mm_select(mv, mp, bv, bp, mv, mp);
                 }
             }
-            if (n_mid) mm_combine(rv, rp, mv, mp, rv, rp);
+            if (n_mid) mm_select(rv, rp, mv, mp, rv, rp);
         } else if (d == 2) {
             const uint32_t z = (i / B + 1) * B + B - 1;
             const uint32_t qb = q + (z >> 4) < 64 ? q + (z >> 4) : 63u;
-            mm_combine(rv, rp, t.px[17 * qb + (z & 15)], 16 * qb + (uint32_t)((t.pn[qb] >> (4 * (z & 15))) & 15), rv, rp);
+            mm_select(rv, rp, t.px[17 * qb + (z & 15)], 16 * qb + (uint32_t)((t.pn[qb] >> (4 * (z & 15))) & 15), rv, rp);
         }
         if (d) {
             const uint32_t qe = q + (e >> 4) < 64 ? q + (e >> 4) : 63u;
-            mm_combine(rv, rp, t.px[17 * qe + (e & 15)], 16 * qe + (uint32_t)((t.pn[qe] >> (4 * (e & 15))) & 15), rv, rp);
+            mm_select(rv, rp, t.px[17 * qe + (e & 15)], 16 * qe + (uint32_t)((t.pn[qe] >> (4 * (e & 15))) & 15), rv, rp);
         }
         rv32[i] = (uint32_t)rv;
         offs[i >> 2] |= (rp - (p0 + i)) << (8 * (i & 3));
         if (i == 0) {
             first_v = rv;
             first_p = rp;
-        } else if (rv != last_v || ((rv & 1) && rp != last_p)) {
-            diffm |= 1u << i;
+        } else {
+            diffm |= window_differs(rv, rp, last_v, last_p) << i;
         }
         last_v = rv;
         last_p = rp;
     }
     // window p0 against the previous lane's last window
-    const uint64_t prev_v = lane_prev64(last_v);
-    const uint32_t prev_p = lane_prev32(last_p);
-    if (prev_v != first_v || ((first_v & 1) && first_p != prev_p)) diffm |= 1u;
+    diffm |= window_differs(first_v, first_p, lane_prev64(last_v), lane_prev32(last_p));
     const uint32_t segm = okm & (firstm | diffm);
     __syncthreads();  // the prefix minima were read: their LDS is reused
 #pragma unroll
@@ -712,16 +767,13 @@ GG_DEV RecInfo rec_info(const Tile& t, uint32_t x) {
     // group start: latest group-start bit at or before x inside the tile
     int64_t a = -1;
     {
+        // (the word of x or the one before it holds the start of most groups)
         int32_t wi = (int32_t)(x >> 5);
-        uint32_t msk = t.seg[wi] & ((2u << (x & 31)) - 1u);
-        while (true) {
-            if (msk) {
-                a = t.wlo + (int64_t)wi * 32 + (31 - __clz(msk));
-                break;
-            }
-            if (--wi < 0) break;
-            msk = t.seg[wi];
-        }
+        const uint32_t m1 = t.seg[wi] & ((2u << (x & 31)) - 1u);
+        uint32_t msk = m1;
+        if (!m1 && wi > 0) msk = t.seg[--wi];
+        while (msk == 0 && wi > 0) msk = t.seg[--wi];
+        if (msk) a = t.wlo + (int64_t)wi * 32 + (31 - __clz(msk));
     }
     if (a < 0) return r;  // group starts before the halo: deferred
     const uint64_t v = t.wval(x);
@@ -812,27 +864,24 @@ GG_DEV bool record_words(const Tile& t, const RecInfo& r, uint4* w4) {
     const uint32_t len = (uint32_t)(r.end - r.start);
     const int64_t rs = r.start - t.borg;
     if (SW > 8 || len > (SW - 1) * 16 || rs < 0) return false;
-    const uint32_t nw = (len + 15) / 16;
+    // Word q holds 16 bases from rs + 16 q, or the reverse complement of the 16
+    // before the end less 16 q.  Words past the record's bases are zero: they
+    // read codes in the tile or, up to 7 words behind them, the invalid bits.
+    const int32_t first = (int32_t)(r.rc ? r.end - t.borg - 16 : rs), step = r.rc ? -16 : 16;
+    uint32_t wv[8];
+    wv[0] = len | r.meta;
 #pragma unroll
-    for (uint32_t g = 0; g < 2; g++) {
-        if (4 * g >= SW) break;
-        uint32_t wv[4];
-#pragma unroll
-        for (uint32_t j = 0; j < 4; j++) {
-            const uint32_t q = 4 * g + j;
-            uint32_t wq = 0;
-            if (q == 0) {
-                wq = len | r.meta;
-            } else if (q - 1 < nw) {
-                const uint32_t qi = q - 1;
-                wq = !r.rc ? extract16(t, rs + 16 * qi) : rev_comp16(extract16(t, (r.end - t.borg) - 16 * (int64_t)qi - 16));
-                const uint32_t rem = len - 16 * qi;
-                if (rem < 16) wq &= (1u << (2 * rem)) - 1u;
-            }
-            wv[j] = wq;
+    for (uint32_t q = 0; q < 7; q++) {
+        wv[q + 1] = 0;
+        if (q < 3 || SW == 8) {
+            const int32_t p = first + step * (int32_t)q, rem = (int32_t)len - 16 * (int32_t)q;
+            const uint32_t x = extract16(t, p > -16 ? p : -16), y = rev_comp16(x);
+            const uint32_t keep = rem >= 16 ? ~0u : (1u << (2 * (rem > 0 ? rem : 0))) - 1u;
+            wv[q + 1] = (r.rc ? y : x) & keep;
         }
-        w4[g] = make_uint4(wv[0], wv[1], wv[2], wv[3]);
     }
+    w4[0] = make_uint4(wv[0], wv[1], wv[2], wv[3]);
+    w4[1] = make_uint4(wv[4], wv[5], wv[6], wv[7]);
     return true;
 }
 
@@ -924,19 +973,33 @@ __global__ __launch_bounds__(64) void bucket_stage_kernel(BucketArgs A) {
         bool in_regs[STAGE_R];
 #pragma unroll
         for (uint32_t r = 0; r < STAGE_R; r++) in_regs[r] = ri[r].ok && record_words(t, ri[r], wv[r]);
+        // every rank, then every store of a record that takes its region slot,
+        // then whatever reads memory: one counter orders loads, atomics and
+        // stores, so a wait between two stores waits for the first of them
+        uint32_t rank[STAGE_R];
+        bool done[STAGE_R];
+#pragma unroll
+        for (uint32_t r = 0; r < STAGE_R; r++) rank[r] = ri[r].ok ? rank_of(A, old[r], ri[r].nk) : 0u;
 #pragma unroll
         for (uint32_t r = 0; r < STAGE_R; r++) {
-            if (!ri[r].ok) continue;
+            done[r] = in_regs[r] && rank[r] < A.unit_cap;
+            if (!done[r]) continue;
+            uint4* o4 = reinterpret_cast<uint4*>(A.region + ((uint64_t)ri[r].unit * A.unit_cap + rank[r]) * SW);
+            o4[0] = wv[r][0];
+            if (SW == 8) o4[1] = wv[r][1];
+        }
+        if (A.region_color) {
+#pragma unroll
+            for (uint32_t r = 0; r < STAGE_R; r++)
+                if (done[r]) A.region_color[(uint64_t)ri[r].unit * A.unit_cap + rank[r]] = color_of(A, ri[r].start);
+        }
+        // spilled, long and other records
+#pragma unroll
+        for (uint32_t r = 0; r < STAGE_R; r++) {
+            if (!ri[r].ok || done[r]) continue;
             uint32_t* color_at;
-            uint32_t* out = record_dest(A, ri[r].unit, rank_of(A, old[r], ri[r].nk), &color_at);
-            if (!out) continue;  // spill list full: retried
-            if (in_regs[r]) {
-                uint4* o4 = reinterpret_cast<uint4*>(out);
-                o4[0] = wv[r][0];
-                if (SW == 8) o4[1] = wv[r][1];
-            } else if (!write_record(t, ri[r], out)) {
-                continue;  // pool full: retried
-            }
+            uint32_t* out = record_dest(A, ri[r].unit, rank[r], &color_at);
+            if (!out || !write_record(t, ri[r], out)) continue;  // spill list or pool full: retried
             if (color_at) *color_at = color_of(A, ri[r].start);
         }
     }
