@@ -34,6 +34,17 @@ __global__ void fill32_kernel(uint32_t* p, uint32_t v, uint64_t n) {
 }
 
 
+// Cursors and counters of the passes, CURSOR_STRIDE 64-bit words apart (a line
+// each), cleared by one launch and read back by one copy into pinned memory:
+// single fills and copies cost 10 to 40 us apiece, most of a small build's time
+// (30 kbp genome with its table 0.94 -> 0.69 ms, 64 colors of 41 MB 2.42 -> 2.21).
+enum Cursor : uint32_t { CU_SPILL, CU_POOL, CU_KMERS, CU_DEFER, CU_ERROR, CU_ITEMS, CU_WORK, CU_REDO, CU_CHUNK, CU_FIX, CU_ADDED, CU_TOTAL, N_CURSORS };
+constexpr uint32_t CURSOR_STRIDE = 8;
+constexpr size_t CURSOR_BYTES = (size_t)N_CURSORS * CURSOR_STRIDE * 8;
+__global__ void clear_cursors_kernel(unsigned long long* c, uint32_t which) {
+    if (threadIdx.x < N_CURSORS && ((which >> threadIdx.x) & 1u)) c[threadIdx.x * CURSOR_STRIDE] = 0;
+}
+
 namespace {
 
 struct DevBuf {
@@ -52,14 +63,18 @@ struct ggcat_gpu_ctx {
     hipStream_t stream = nullptr;
     std::string err;
     hipEvent_t ev[16];
+    DevBuf cursors;  // Cursor slots
+    uint64_t* seen = nullptr;  // their last copy on the host (pinned)
+    size_t dd_lds[2] = {0, 0};  // LDS of a deduplication workgroup and how many a CU holds with it
+    int dd_fit[2] = {0, 0};
     // bucketing buffers
-    DevBuf input, seg_bits, unit_count, unit_cursor, unit_off, unit_kmers, scan_part, slots, pool, pool_cursor,
-        slot_color, color_starts, colors, error_flag, stage_slots, stage_unit, stage_rank, stage_color, stage_cursor, defer,
-        defer_count, kmer_total, spill_slots, spill_color,  // stage_*: the unit regions, the spill list's units and ranks
+    DevBuf input, seg_bits, unit_count, unit_cursor, unit_off, unit_kmers, scan_part, slots, pool,
+        slot_color, color_starts, colors, error_flag, stage_slots, stage_unit, stage_rank, stage_color, defer,
+        spill_slots, spill_color,  // stage_*: the unit regions, the spill list's units and ranks
         unit_dcount, unit_dregion, unit_skmers;  // per unit after deduplication
     // merge buffers
-    DevBuf items, n_items, work, parts, redo, redo_count, out_key, out_val, out_sub, chunk_cursor, chunk_fill_dev,
-        chunk_off, fix_key, fix_val, fix_sub, fix_cursor, out_colors, fix_colors;
+    DevBuf items, parts, redo, out_key, out_val, out_sub, chunk_fill_dev,
+        chunk_off, fix_key, fix_val, fix_sub, out_colors, fix_colors;
     // state
     ggcat_gpu_params P{};
     bool have_records = false, have_solid = false;
@@ -166,6 +181,30 @@ template <class T>
 T* P_(DevBuf& b) {
     return reinterpret_cast<T*>(b.p);
 }
+
+template <class T>
+T* cursor(ggcat_gpu_ctx* ctx, Cursor c) {
+    return reinterpret_cast<T*>(P_<uint64_t>(ctx->cursors) + c * CURSOR_STRIDE);
+}
+// The slot's value at the last fetch_cursors (word w of it).
+template <class T>
+T seen(const ggcat_gpu_ctx* ctx, Cursor c, uint32_t w = 0) {
+    return (T)ctx->seen[c * CURSOR_STRIDE + w];
+}
+// Copies the cursors, and the 64-bit word *total (when given) as CU_TOTAL, to
+// the host once the stream's work is done.
+int fetch_cursors(ggcat_gpu_ctx* ctx, const uint64_t* total) {
+    HIPCHK(hipMemcpyAsync(ctx->seen, ctx->cursors.p, CURSOR_BYTES, hipMemcpyDeviceToHost, ctx->stream));
+    if (total)
+        HIPCHK(hipMemcpyAsync(ctx->seen + CU_TOTAL * CURSOR_STRIDE, total, 8, hipMemcpyDeviceToHost, ctx->stream));
+    HIPCHK(hipStreamSynchronize(ctx->stream));
+    return GGCAT_GPU_OK;
+}
+#define FETCH(total)                                \
+    do {                                            \
+        const int r_ = fetch_cursors(ctx, (total)); \
+        if (r_ != GGCAT_GPU_OK) return r_;          \
+    } while (0)
 
 // ntHash rolling tables, index out*4+in with out == 4 meaning "no base leaves"
 // (crates/hashes/src/nthash_base.rs:49-61 on 2-bit codes A=0,C=1,T=2,G=3);
@@ -510,6 +549,9 @@ int ggcat_gpu_create(int device, ggcat_gpu_ctx** out) {
     for (int i = 0; i < 2 && e == hipSuccess; i++) e = hipEventCreateWithFlags(&ctx->dd_ev[i], hipEventDisableTiming);
     hipDeviceProp_t prop;
     if (e == hipSuccess && hipGetDeviceProperties(&prop, device) == hipSuccess) ctx->n_cu = prop.multiProcessorCount;
+    if (e == hipSuccess) e = hipMalloc(&ctx->cursors.p, CURSOR_BYTES);
+    if (e == hipSuccess) ctx->cursors.cap = CURSOR_BYTES;
+    if (e == hipSuccess) e = hipHostMalloc(&ctx->seen, CURSOR_BYTES, hipHostMallocDefault);
     // the no-allocation entry point's scratch array: its address on this device
     if (e == hipSuccess && noalloc_scratch_setup(device) != GGCAT_GPU_OK) e = hipErrorInvalidSymbol;
     if (e != hipSuccess) {
@@ -526,22 +568,21 @@ void ggcat_gpu_destroy(ggcat_gpu_ctx* ctx) {
     if (ctx->stream) (void)hipStreamSynchronize(ctx->stream);
     if (ctx->copy_stream) (void)hipStreamSynchronize(ctx->copy_stream);
     DevBuf* bufs[] = {&ctx->input, &ctx->seg_bits, &ctx->unit_count, &ctx->unit_cursor, &ctx->unit_off,
-                      &ctx->unit_kmers, &ctx->scan_part, &ctx->slots, &ctx->pool, &ctx->pool_cursor,
-                      &ctx->unit_dcount, &ctx->unit_dregion, &ctx->unit_skmers,
+                      &ctx->unit_kmers, &ctx->scan_part, &ctx->slots, &ctx->pool, &ctx->unit_dcount, &ctx->unit_dregion, &ctx->unit_skmers,
                       &ctx->slot_color, &ctx->color_starts, &ctx->colors, &ctx->error_flag, &ctx->items,
-                      &ctx->n_items, &ctx->work, &ctx->parts, &ctx->redo, &ctx->redo_count, &ctx->out_key,
-                      &ctx->out_val, &ctx->out_sub, &ctx->chunk_cursor, &ctx->chunk_fill_dev, &ctx->chunk_off, &ctx->fix_key,
-                      &ctx->fix_val, &ctx->fix_sub, &ctx->fix_cursor, &ctx->out_colors, &ctx->fix_colors,
+                      &ctx->parts, &ctx->redo, &ctx->out_key,
+                      &ctx->out_val, &ctx->out_sub, &ctx->chunk_fill_dev, &ctx->chunk_off, &ctx->fix_key,
+                      &ctx->fix_val, &ctx->fix_sub, &ctx->out_colors, &ctx->fix_colors,
                       &ctx->idx_slots, &ctx->idx_count,
                       &ctx->q_seq, &ctx->q_off, &ctx->q_matched, &ctx->q_counts,
                       &ctx->u_nb, &ctx->u_ext, &ctx->u_link, &ctx->u_seg, &ctx->u_head, &ctx->u_uhead,
                       &ctx->u_ubytes, &ctx->u_uoff, &ctx->u_totals, &ctx->u_seq, &ctx->u_sub, &ctx->u_flags, &ctx->u_visited, &ctx->u_rest,
                       &ctx->u_rest_n, &ctx->u_rep, &ctx->u_tab, &ctx->u_path, &ctx->stage_slots, &ctx->stage_unit,
-                      &ctx->stage_rank, &ctx->stage_color, &ctx->stage_cursor, &ctx->defer, &ctx->defer_count,
-                      &ctx->kmer_total, &ctx->spill_slots, &ctx->spill_color, &ctx->raw, &ctx->p_stats,
+                      &ctx->stage_rank, &ctx->stage_color, &ctx->defer, &ctx->spill_slots, &ctx->spill_color, &ctx->raw, &ctx->p_stats,
                       &ctx->p_carry, &ctx->p_keep, &ctx->p_keep_off, &ctx->p_flags, &ctx->p_bits, &ctx->rk_pos, &ctx->rk_tri,
-                      &ctx->copy_mult, &ctx->copy_flags};
+                      &ctx->copy_mult, &ctx->copy_flags, &ctx->cursors};
     if (ctx->pin_ring) (void)hipHostFree(ctx->pin_ring);
+    if (ctx->seen) (void)hipHostFree(ctx->seen);
     if (ctx->server) (void)ggcat_gpu_serve_close(ctx);
     if (ctx->graph_a) (void)hipGraphExecDestroy(ctx->graph_a);
     for (DevBuf* b : bufs)
@@ -656,7 +697,6 @@ int ggcat_gpu_bucketing(ggcat_gpu_ctx* ctx, const uint8_t* data, uint64_t n_byte
     ENSURE(ctx->unit_dcount, (size_t)n_units * 4);
     ENSURE(ctx->unit_dregion, (size_t)n_units * 4);
     ENSURE(ctx->unit_skmers, (size_t)n_units * 4);
-    ENSURE(ctx->pool_cursor, 8);
     ENSURE(ctx->error_flag, 8);
     if (n_colors) {
         ENSURE(ctx->color_starts, (size_t)n_colors * 8);
@@ -687,21 +727,18 @@ int ggcat_gpu_bucketing(ggcat_gpu_ctx* ctx, const uint8_t* data, uint64_t n_byte
     A.unit_dregion = P_<uint32_t>(ctx->unit_dregion);
     A.unit_skmers = P_<uint32_t>(ctx->unit_skmers);
     A.slot_words = slot_words;
-    A.pool_cursor = P_<unsigned long long>(ctx->pool_cursor);
+    A.pool_cursor = cursor<unsigned long long>(ctx, CU_POOL);
     A.color_starts = n_colors ? P_<uint64_t>(ctx->color_starts) : nullptr;
     A.colors = n_colors ? P_<uint32_t>(ctx->colors) : nullptr;
     A.n_colors = n_colors;
-    A.error_flag = P_<uint32_t>(ctx->error_flag);
+    A.error_flag = cursor<uint32_t>(ctx, CU_ERROR);
     nthash_tables(p.m, A.gtab);
     const TileGeom G = tile_geom(T, w, p.k, p.m);
-    ENSURE(ctx->stage_cursor, 8);
-    ENSURE(ctx->defer_count, 8);
-    ENSURE(ctx->kmer_total, 16);  // k-mer occurrences, records
     ENSURE(ctx->defer, std::max<uint64_t>(n_tiles, 1) * 24);
-    A.spill_cursor = P_<unsigned long long>(ctx->stage_cursor);
+    A.spill_cursor = cursor<unsigned long long>(ctx, CU_SPILL);
     A.defer = P_<uint64_t>(ctx->defer);
-    A.defer_count = P_<uint32_t>(ctx->defer_count);
-    A.kmer_total = P_<unsigned long long>(ctx->kmer_total);
+    A.defer_count = cursor<uint32_t>(ctx, CU_DEFER);
+    A.kmer_total = cursor<unsigned long long>(ctx, CU_KMERS);  // k-mer occurrences, records
     ENSURE(ctx->scan_part, (((size_t)n_units + SCAN_CHUNK - 1) / SCAN_CHUNK + 1) * 8);
 
     // Pass 1: clear the unit counts, k-mer counts, group-start bitmap and
@@ -844,10 +881,10 @@ int ggcat_gpu_bucketing(ggcat_gpu_ctx* ctx, const uint8_t* data, uint64_t n_byte
         }
         HIPCHK(hipGetLastError());
         HIPCHK(hipEventRecord(ctx->ev[1], ctx->stream));
-        HIPCHK(hipMemcpyAsync(&staged, ctx->stage_cursor.p, 8, hipMemcpyDeviceToHost, ctx->stream));
-        HIPCHK(hipMemcpyAsync(&pool_used, ctx->pool_cursor.p, 8, hipMemcpyDeviceToHost, ctx->stream));
-        HIPCHK(hipMemcpyAsync(&errf, ctx->error_flag.p, 4, hipMemcpyDeviceToHost, ctx->stream));
-        HIPCHK(hipStreamSynchronize(ctx->stream));
+        FETCH(nullptr);
+        staged = seen<uint64_t>(ctx, CU_SPILL);
+        pool_used = seen<uint64_t>(ctx, CU_POOL);
+        errf = seen<uint32_t>(ctx, CU_ERROR);
         if (errf & 8) return fail(ctx, GGCAT_GPU_ENOMEM, "a physical unit exceeds 2^32 k-mer occurrences");
         if (errf) return fail(ctx, GGCAT_GPU_EHIP, "bucketing: a group start was not found");
         if (staged <= spill_cap && pool_used <= pool_cap) break;
@@ -857,6 +894,7 @@ int ggcat_gpu_bucketing(ggcat_gpu_ctx* ctx, const uint8_t* data, uint64_t n_byte
     }
     ctx->pool_words = pool_used;
     ctx->n_spill = staged;
+    const uint64_t kmer_total[2] = {seen<uint64_t>(ctx, CU_KMERS, 0), seen<uint64_t>(ctx, CU_KMERS, 1)};
 
     // Pass 2: identical records of a unit counted once, unit offsets of the
     // stored records, then every stored record to its unit's slots.
@@ -870,14 +908,19 @@ int ggcat_gpu_bucketing(ggcat_gpu_ctx* ctx, const uint8_t* data, uint64_t n_byte
         ctx->dd_max = wide ? DEDUP_WIDE : std::min(DEDUP_SMALL, 8 * 64 * 4 / slot_words);
         const size_t lds_small = dedup_lds_bytes(DEDUP_SMALL, slot_words, n_colors != 0);
         const size_t lds_wide = dedup_lds_bytes(DEDUP_WIDE, slot_words, n_colors != 0);
-        int occ = 0;
-        HIPCHK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, reinterpret_cast<const void*>(unit_dedup_kernel), 64,
-                                                            lds_small));
-        const uint32_t grid = (uint32_t)std::min<uint64_t>(n_units, (uint64_t)ctx->n_cu * std::max(occ, 1));
+        // (the runtime's answer depends on the LDS alone: asked again when that changes)
+        auto fit = [&](int w, const void* kernel, int threads, size_t lds) -> hipError_t {
+            if (ctx->dd_fit[w] && ctx->dd_lds[w] == lds) return hipSuccess;
+            ctx->dd_lds[w] = lds;
+            const hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&ctx->dd_fit[w], kernel, threads, lds);
+            ctx->dd_fit[w] = std::max(ctx->dd_fit[w], 1);
+            return e;
+        };
+        HIPCHK(fit(0, reinterpret_cast<const void*>(unit_dedup_kernel), 64, lds_small));
+        const uint32_t grid = (uint32_t)std::min<uint64_t>(n_units, (uint64_t)ctx->n_cu * ctx->dd_fit[0]);
         if (wide) {
-            HIPCHK(hipOccupancyMaxActiveBlocksPerMultiprocessor(
-                &occ, reinterpret_cast<const void*>(unit_dedup_wide_kernel), 256, lds_wide));
-            const uint32_t wgrid = (uint32_t)std::min<uint64_t>(n_units, (uint64_t)ctx->n_cu * std::max(occ, 1));
+            HIPCHK(fit(1, reinterpret_cast<const void*>(unit_dedup_wide_kernel), 256, lds_wide));
+            const uint32_t wgrid = (uint32_t)std::min<uint64_t>(n_units, (uint64_t)ctx->n_cu * ctx->dd_fit[1]);
             HIPCHK(hipEventRecord(ctx->dd_ev[0], ctx->stream));
             HIPCHK(hipStreamWaitEvent(ctx->copy_stream, ctx->dd_ev[0], 0));
             hipLaunchKernelGGL(unit_dedup_wide_kernel, dim3(wgrid), dim3(256), lds_wide, ctx->copy_stream, A, n_units);
@@ -892,10 +935,10 @@ int ggcat_gpu_bucketing(ggcat_gpu_ctx* ctx, const uint8_t* data, uint64_t n_byte
     const int rs = device_scan(ctx, A.unit_dcount, P_<uint64_t>(ctx->unit_off), n_units);
     if (rs != GGCAT_GPU_OK) return rs;
     HIPCHK(hipEventRecord(ctx->ev[2], ctx->stream));
-    uint64_t total = 0, kmer_total[2] = {0, 0};
-    HIPCHK(hipMemcpyAsync(&total, P_<uint64_t>(ctx->unit_off) + n_units, 8, hipMemcpyDeviceToHost, ctx->stream));
-    HIPCHK(hipMemcpyAsync(kmer_total, A.kmer_total, 16, hipMemcpyDeviceToHost, ctx->stream));
+    HIPCHK(hipMemcpyAsync(ctx->seen + CU_TOTAL * CURSOR_STRIDE, P_<uint64_t>(ctx->unit_off) + n_units, 8,
+                          hipMemcpyDeviceToHost, ctx->stream));
     HIPCHK(hipStreamSynchronize(ctx->stream));
+    const uint64_t total = seen<uint64_t>(ctx, CU_TOTAL);
     ctx->n_records = kmer_total[1];
     ctx->n_stored = total;
     ENSURE(ctx->slots, std::max<uint64_t>(total, 1) * slot_words * 4);
@@ -914,9 +957,8 @@ int ggcat_gpu_bucketing(ggcat_gpu_ctx* ctx, const uint8_t* data, uint64_t n_byte
     }
     HIPCHK(hipGetLastError());
     HIPCHK(hipEventRecord(ctx->ev[4], ctx->stream));
-    HIPCHK(hipMemcpyAsync(&errf, ctx->error_flag.p, 4, hipMemcpyDeviceToHost, ctx->stream));
-    HIPCHK(hipStreamSynchronize(ctx->stream));
-    if (errf) return fail(ctx, GGCAT_GPU_EHIP, "bucketing: a record rank outside its unit");
+    FETCH(nullptr);
+    if (seen<uint32_t>(ctx, CU_ERROR)) return fail(ctx, GGCAT_GPU_EHIP, "bucketing: a record rank outside its unit");
     float t;
     HIPCHK(hipEventElapsedTime(&t, ctx->ev[0], ctx->ev[1]));
     ctx->ms[0] = t;
@@ -1511,22 +1553,21 @@ int ggcat_gpu_kmers_merge(ggcat_gpu_ctx* ctx) {
 
     // work items: runs of units of one sub-bucket
     ENSURE(ctx->items, (size_t)ctx->n_units * sizeof(WorkItem));
-    ENSURE(ctx->n_items, 8);
-    ENSURE(ctx->work, 8);
-    ENSURE(ctx->redo_count, 8);
-    ENSURE(ctx->chunk_cursor, 8);
-    ENSURE(ctx->fix_cursor, 8);
-    ENSURE(ctx->error_flag, 8);
-    M.error_flag = P_<uint32_t>(ctx->error_flag);
+    M.error_flag = cursor<uint32_t>(ctx, CU_ERROR);
+    auto clear = [&](uint32_t which) {
+        hipLaunchKernelGGL(clear_cursors_kernel, dim3(1), dim3(64), 0, ctx->stream,
+                           P_<unsigned long long>(ctx->cursors), which);
+    };
+    const uint32_t per_pass = 1u << CU_WORK | 1u << CU_REDO;
+    const uint32_t per_attempt = per_pass | 1u << CU_CHUNK | 1u << CU_FIX | 1u << CU_ADDED | 1u << CU_ERROR;
     HIPCHK(hipEventRecord(ctx->ev[5], ctx->stream));
-    HIPCHK(hipMemsetAsync(ctx->n_items.p, 0, 8, ctx->stream));
+    clear(per_attempt | 1u << CU_ITEMS);
     hipLaunchKernelGGL(make_items_kernel, dim3((ctx->n_sub_all + 255) / 256), dim3(256), 0, ctx->stream,
                        P_<uint32_t>(ctx->unit_skmers), P_<uint64_t>(ctx->unit_off), ctx->n_sub_all, ctx->xb, item_occ,
-                       ctx->dd_max, P_<WorkItem>(ctx->items), P_<unsigned int>(ctx->n_items));
+                       ctx->dd_max, P_<WorkItem>(ctx->items), cursor<unsigned int>(ctx, CU_ITEMS));
     HIPCHK(hipGetLastError());
-    uint32_t n_items = 0;
-    HIPCHK(hipMemcpyAsync(&n_items, ctx->n_items.p, 4, hipMemcpyDeviceToHost, ctx->stream));
-    HIPCHK(hipStreamSynchronize(ctx->stream));
+    FETCH(nullptr);
+    const uint32_t n_items = seen<uint32_t>(ctx, CU_ITEMS);
     M.items = P_<WorkItem>(ctx->items);
 
     // resident workgroups per CU: what the 160 KiB LDS holds with the
@@ -1562,22 +1603,20 @@ int ggcat_gpu_kmers_merge(ggcat_gpu_ctx* ctx) {
         }
         M.out_colors = W ? P_<uint32_t>(ctx->out_colors) : nullptr;
         M.fix_colors = W ? P_<uint32_t>(ctx->fix_colors) : nullptr;
-        M.work = P_<unsigned int>(ctx->work);
-        M.redo_count = P_<unsigned int>(ctx->redo_count);
+        M.work = cursor<unsigned int>(ctx, CU_WORK);
+        M.redo_count = cursor<unsigned int>(ctx, CU_REDO);
         M.out_key = P_<uint64_t>(ctx->out_key);
         M.out_val = P_<uint32_t>(ctx->out_val);
         M.out_sub = P_<uint32_t>(ctx->out_sub);
-        M.chunk_cursor = P_<unsigned int>(ctx->chunk_cursor);
+        M.chunk_cursor = cursor<unsigned int>(ctx, CU_CHUNK);
         M.chunk_fill = P_<uint32_t>(ctx->chunk_fill_dev);
         M.n_chunks = (uint32_t)n_chunks;
         M.fix_key = P_<uint64_t>(ctx->fix_key);
         M.fix_val = P_<uint32_t>(ctx->fix_val);
         M.fix_sub = P_<uint32_t>(ctx->fix_sub);
-        M.fix_cursor = P_<unsigned long long>(ctx->fix_cursor);
+        M.fix_cursor = cursor<unsigned long long>(ctx, CU_FIX);
         M.fix_cap = fix_cap;
-        HIPCHK(hipMemsetAsync(ctx->chunk_cursor.p, 0, 8, ctx->stream));
-        HIPCHK(hipMemsetAsync(ctx->fix_cursor.p, 0, 8, ctx->stream));
-        HIPCHK(hipMemsetAsync(ctx->error_flag.p, 0, 8, ctx->stream));
+        if (attempt) clear(per_attempt);
         HIPCHK(hipEventRecord(ctx->ev[6], ctx->stream));
         HIPCHK(hipEventRecord(ctx->ev[7], ctx->stream));
         // Pass 0: one work entry per item.  Entries whose table overflows (or
@@ -1594,16 +1633,14 @@ int ggcat_gpu_kmers_merge(ggcat_gpu_ctx* ctx) {
             // still gets about 32 claims
             M.claim = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(8, n_work / ((uint64_t)lds_wgs * 32)));
             M.parts = pass ? P_<PartWork>(ctx->parts) : nullptr;
-            HIPCHK(hipMemsetAsync(ctx->work.p, 0, 8, ctx->stream));
-            HIPCHK(hipMemsetAsync(ctx->redo_count.p, 0, 8, ctx->stream));
+            if (pass) clear(per_pass);
             if (pass) HIPCHK(hipEventRecord(ctx->ev[8], ctx->stream));
             hipLaunchKernelGGL(merge_kernel, dim3(lds_wgs), dim3(merge_threads), lds_bytes, ctx->stream, M);
             HIPCHK(hipGetLastError());
             n_passes_run++;
             HIPCHK(hipEventRecord(ctx->ev[pass ? 9 : 7], ctx->stream));
-            uint32_t n_redo = 0;
-            HIPCHK(hipMemcpyAsync(&n_redo, ctx->redo_count.p, 4, hipMemcpyDeviceToHost, ctx->stream));
-            HIPCHK(hipStreamSynchronize(ctx->stream));
+            FETCH(nullptr);
+            const uint32_t n_redo = seen<uint32_t>(ctx, CU_REDO);
             if (pass) {
                 float tp;
                 HIPCHK(hipEventElapsedTime(&tp, ctx->ev[8], ctx->ev[9]));
@@ -1641,12 +1678,10 @@ int ggcat_gpu_kmers_merge(ggcat_gpu_ctx* ctx) {
         }
         ctx->n_big = n_split_items;
         ctx->n_passes = n_passes_run;
-        uint64_t n_fix = 0;
-        uint32_t used_chunks = 0, errf = 0;
-        HIPCHK(hipMemcpyAsync(&used_chunks, ctx->chunk_cursor.p, 4, hipMemcpyDeviceToHost, ctx->stream));
-        HIPCHK(hipMemcpyAsync(&n_fix, ctx->fix_cursor.p, 8, hipMemcpyDeviceToHost, ctx->stream));
-        HIPCHK(hipMemcpyAsync(&errf, ctx->error_flag.p, 4, hipMemcpyDeviceToHost, ctx->stream));
-        HIPCHK(hipStreamSynchronize(ctx->stream));
+        // (without work items the last fetch is the one behind the clear)
+        if (!n_items) HIPCHK(hipStreamSynchronize(ctx->stream));
+        const uint64_t n_fix = seen<uint64_t>(ctx, CU_FIX);
+        const uint32_t used_chunks = seen<uint32_t>(ctx, CU_CHUNK), errf = seen<uint32_t>(ctx, CU_ERROR);
         if (errf & 1) return fail(ctx, GGCAT_GPU_EHIP, "k-mer table overflow");
         if (errf & 2) return fail(ctx, GGCAT_GPU_EHIP, "malformed record slot");
         float t;
@@ -1661,21 +1696,33 @@ int ggcat_gpu_kmers_merge(ggcat_gpu_ctx* ctx) {
         }
         // the partly filled chunks' entries close up; combined fixups are
         // appended behind the dense table
-        uint64_t tail0 = 0;
+        uint64_t tail0 = 0, n_add = 0;
+        const bool join = n_fix && n_fix <= FIX_JOIN_MAX && used_chunks;  // fixups combined on the device
         if (used_chunks) {
             ENSURE(ctx->chunk_off, ((size_t)used_chunks + 1) * 8);
             const int rs = device_scan(ctx, P_<uint32_t>(ctx->chunk_fill_dev), P_<uint64_t>(ctx->chunk_off), used_chunks);
             if (rs != GGCAT_GPU_OK) return rs;
-            HIPCHK(hipMemcpyAsync(&tail0, P_<uint64_t>(ctx->chunk_off) + used_chunks, 8, hipMemcpyDeviceToHost, ctx->stream));
             hipLaunchKernelGGL(out_close_holes_kernel, dim3(used_chunks), dim3(256), 0, ctx->stream,
                                P_<uint64_t>(ctx->chunk_off), used_chunks, M.out_key, key_words, M.out_val, M.out_sub,
                                M.out_colors, W);
+            if (join)
+                hipLaunchKernelGGL(fix_join_kernel, dim3(((uint32_t)n_fix + 255) / 256), dim3(256), 0, ctx->stream,
+                                   M.fix_key, M.fix_val, M.fix_sub, M.fix_colors, (uint32_t)n_fix, key_words, W,
+                                   P_<uint64_t>(ctx->chunk_off) + used_chunks, out_cap, M.out_key, M.out_val, M.out_sub,
+                                   M.out_colors, cursor<unsigned long long>(ctx, CU_ADDED));
             HIPCHK(hipGetLastError());
-            HIPCHK(hipStreamSynchronize(ctx->stream));
+            FETCH(P_<uint64_t>(ctx->chunk_off) + used_chunks);
+            tail0 = seen<uint64_t>(ctx, CU_TOTAL);
+            n_add = seen<uint64_t>(ctx, CU_ADDED);
         }
-        uint64_t n_out = tail0, n_add = 0;
+        uint64_t n_out = tail0;
+        if (tail0 + n_add > out_cap) {
+            if (attempt == 1) return fail(ctx, GGCAT_GPU_ENOMEM, "solid output overflow");
+            n_chunks = (tail0 + n_add) / OUT_CHUNK + 64;
+            continue;
+        }
         // combine the two halves of cross-unit boundary k-mers
-        if (n_fix) {
+        if (n_fix && !join) {
             const uint32_t kw = key_words;
             std::vector<uint64_t> fk(n_fix * kw);
             std::vector<uint32_t> fv(n_fix), fs(n_fix), fc(n_fix * W);
