@@ -103,7 +103,7 @@ struct ggcat_gpu_ctx {
     DevBuf idx_slots, idx_count;
     bool have_index = false;
     gg::KmerTable idx{};
-    DevBuf q_seq, q_off, q_matched, q_counts;
+    DevBuf q_seq, q_off, q_matched, q_counts, q_kmers, q_blocks;
     struct Server* server = nullptr;
     // unitig chains
     DevBuf u_nb, u_ext, u_link, u_seg, u_head, u_uhead, u_ubytes, u_uoff, u_seq, u_sub, u_flags, u_visited, u_rest,
@@ -534,6 +534,8 @@ extern "C" {
 
 namespace {
 static int noalloc_scratch_setup(int device);
+static bool query_offsets_on_device(uint64_t n_bytes, uint32_t n_queries);
+static int query_prepare_uploaded(ggcat_gpu_ctx* ctx, uint64_t n_bytes, uint32_t n_queries, uint32_t nc);
 }  // namespace
 
 int ggcat_gpu_create(int device, ggcat_gpu_ctx** out) {
@@ -574,7 +576,7 @@ void ggcat_gpu_destroy(ggcat_gpu_ctx* ctx) {
                       &ctx->out_val, &ctx->out_sub, &ctx->chunk_fill_dev, &ctx->chunk_off, &ctx->fix_key,
                       &ctx->fix_val, &ctx->fix_sub, &ctx->out_colors, &ctx->fix_colors,
                       &ctx->idx_slots, &ctx->idx_count,
-                      &ctx->q_seq, &ctx->q_off, &ctx->q_matched, &ctx->q_counts,
+                      &ctx->q_seq, &ctx->q_off, &ctx->q_matched, &ctx->q_counts, &ctx->q_kmers, &ctx->q_blocks,
                       &ctx->u_nb, &ctx->u_ext, &ctx->u_link, &ctx->u_seg, &ctx->u_head, &ctx->u_uhead,
                       &ctx->u_ubytes, &ctx->u_uoff, &ctx->u_totals, &ctx->u_seq, &ctx->u_sub, &ctx->u_flags, &ctx->u_visited, &ctx->u_rest,
                       &ctx->u_rest_n, &ctx->u_rep, &ctx->u_tab, &ctx->u_path, &ctx->stage_slots, &ctx->stage_unit,
@@ -2266,10 +2268,13 @@ int ggcat_gpu_query(ggcat_gpu_ctx* ctx, const uint8_t* queries, uint64_t n_bytes
                     uint64_t* query_kmers, uint64_t* matched, uint32_t* color_counts) {
     if (!ctx || (!queries && n_bytes)) return GGCAT_GPU_EINVAL;
     if (!ctx->have_index) return fail(ctx, GGCAT_GPU_ESTATE, "no query index (call ggcat_gpu_index_build)");
+    const bool on_device = query_offsets_on_device(n_bytes, n_queries);
     std::vector<uint64_t> off;
-    if (!query_offsets(queries, n_bytes, n_queries, off))
-        return fail(ctx, GGCAT_GPU_EINVAL, "queries must be n_queries records, each ending with '\\n'");
-    if (query_kmers) query_kmer_counts(off, ctx->P.k, query_kmers);
+    if (!on_device) {
+        if (!query_offsets(queries, n_bytes, n_queries, off))
+            return fail(ctx, GGCAT_GPU_EINVAL, "queries must be n_queries records, each ending with '\\n'");
+        if (query_kmers) query_kmer_counts(off, ctx->P.k, query_kmers);
+    }
     HIPCHK(hipSetDevice(ctx->device));
     const uint32_t nc = ctx->colored ? ctx->n_color_ids : 0;
     ENSURE(ctx->q_seq, n_bytes + 16);
@@ -2277,7 +2282,12 @@ int ggcat_gpu_query(ggcat_gpu_ctx* ctx, const uint8_t* queries, uint64_t n_bytes
     ENSURE(ctx->q_matched, (size_t)n_queries * 8 + 8);
     ENSURE(ctx->q_counts, (size_t)n_queries * nc * 4 + 4);
     if (n_bytes) HIPCHK(hipMemcpy(ctx->q_seq.p, queries, n_bytes, hipMemcpyHostToDevice));
-    HIPCHK(hipMemcpy(ctx->q_off.p, off.data(), off.size() * 8, hipMemcpyHostToDevice));
+    if (on_device) {
+        const int r = query_prepare_uploaded(ctx, n_bytes, n_queries, nc);
+        if (r != GGCAT_GPU_OK) return r;
+    } else {
+        HIPCHK(hipMemcpy(ctx->q_off.p, off.data(), off.size() * 8, hipMemcpyHostToDevice));
+    }
     QueryArgs Q = query_args(ctx);
     Q.seq = P_<uint8_t>(ctx->q_seq);
     Q.qoff = P_<uint64_t>(ctx->q_off);
@@ -2285,12 +2295,16 @@ int ggcat_gpu_query(ggcat_gpu_ctx* ctx, const uint8_t* queries, uint64_t n_bytes
     Q.matched = P_<uint64_t>(ctx->q_matched);
     Q.color_counts = P_<uint32_t>(ctx->q_counts);
     if (n_queries) {
-        HIPCHK(hipMemsetAsync(ctx->q_matched.p, 0, (size_t)n_queries * 8, ctx->stream));
-        if (nc) HIPCHK(hipMemsetAsync(ctx->q_counts.p, 0, (size_t)n_queries * nc * 4, ctx->stream));
+        if (!on_device) {
+            HIPCHK(hipMemsetAsync(ctx->q_matched.p, 0, (size_t)n_queries * 8, ctx->stream));
+            if (nc) HIPCHK(hipMemsetAsync(ctx->q_counts.p, 0, (size_t)n_queries * nc * 4, ctx->stream));
+        }
         launch_query(ctx, Q, n_bytes, ctx->stream);
         HIPCHK(hipGetLastError());
     }
     HIPCHK(hipStreamSynchronize(ctx->stream));
+    if (query_kmers && on_device)
+        HIPCHK(hipMemcpy(query_kmers, ctx->q_kmers.p, (size_t)n_queries * 8, hipMemcpyDeviceToHost));
     if (matched && n_queries) HIPCHK(hipMemcpy(matched, ctx->q_matched.p, (size_t)n_queries * 8, hipMemcpyDeviceToHost));
     if (color_counts && nc && n_queries)
         HIPCHK(hipMemcpy(color_counts, ctx->q_counts.p, (size_t)n_queries * nc * 4, hipMemcpyDeviceToHost));

@@ -64,15 +64,29 @@ __global__ void na_clear_kernel(uint32_t* header) {
     if (threadIdx.x < 64) header[threadIdx.x] = 0;
 }
 
-// Block b counts the '\n' bytes of [b * NA_BLOCK_BYTES, ...) (coalesced byte loads).
+// Bit j set when byte at + j is '\n', for the 16 bytes from `at` on (a
+// multiple of 16); one 16-byte load where the input is aligned and they are all
+// inside it.
+GG_DEV uint32_t newlines16(const uint8_t* seq, uint64_t n, uint64_t at) {
+    if (at >= n) return 0;
+    if (at + 16 <= n && (reinterpret_cast<uintptr_t>(seq) & 15) == 0) {
+        const uint4 v = *reinterpret_cast<const uint4*>(seq + at);
+        const uint32_t other = nonzero4(v.x ^ 0x0A0A0A0Au) | nonzero4(v.y ^ 0x0A0A0A0Au) << 4 |
+                               nonzero4(v.z ^ 0x0A0A0A0Au) << 8 | nonzero4(v.w ^ 0x0A0A0A0Au) << 12;
+        return ~other & 0xFFFFu;
+    }
+    uint32_t m = 0;
+    for (uint32_t i = 0; i < 16 && at + i < n; i++) m |= (seq[at + i] == '\n' ? 1u : 0u) << i;
+    return m;
+}
+
+// Block b counts the '\n' bytes of [b * NA_BLOCK_BYTES, ...), 16 bytes per
+// thread and step.
 __global__ __launch_bounds__(256) void na_count_kernel(const uint8_t* seq, uint64_t n, uint32_t* block_nl) {
     __shared__ uint32_t s_part[4];
     const uint64_t base = (uint64_t)blockIdx.x * NA_BLOCK_BYTES;
     uint32_t c = 0;
-    for (uint32_t i = threadIdx.x; i < NA_BLOCK_BYTES; i += 256) {
-        const uint64_t p = base + i;
-        if (p < n && seq[p] == '\n') c++;
-    }
+    for (uint32_t i = threadIdx.x * 16; i < NA_BLOCK_BYTES; i += 256 * 16) c += __popc(newlines16(seq, n, base + i));
     for (uint32_t d = 32; d; d >>= 1) c += __shfl_down(c, d);
     if ((threadIdx.x & 63) == 0) s_part[threadIdx.x >> 6] = c;
     __syncthreads();
@@ -121,9 +135,10 @@ __global__ __launch_bounds__(256) void na_fill_kernel(const uint8_t* seq, uint64
     constexpr uint32_t PER = NA_BLOCK_BYTES / 256;
     const uint32_t t = threadIdx.x, lane = t & 63, wave = t >> 6;
     const uint64_t p0 = (uint64_t)blockIdx.x * NA_BLOCK_BYTES + (uint64_t)t * PER;
-    uint32_t mine = 0;
-    for (uint32_t i = 0; i < PER; i++)
-        if (p0 + i < n && seq[p0 + i] == '\n') mine++;
+    static_assert(PER == 64, "a thread's newlines are one 64-bit word");
+    uint64_t nl = 0;
+    for (uint32_t i = 0; i < PER; i += 16) nl |= (uint64_t)newlines16(seq, n, p0 + i) << i;
+    const uint32_t mine = (uint32_t)__popcll(nl);
     uint32_t inc = mine;
     for (uint32_t d = 1; d < 64; d <<= 1) {
         const uint32_t y = __shfl_up(inc, d);
@@ -134,14 +149,11 @@ __global__ __launch_bounds__(256) void na_fill_kernel(const uint8_t* seq, uint64
     uint32_t before = block_base[blockIdx.x];
     for (uint32_t q = 0; q < wave; q++) before += s_wave[q];
     uint32_t r = before + inc - mine;
-    for (uint32_t i = 0; i < PER && r < before + inc; i++) {
-        if (p0 + i < n && seq[p0 + i] == '\n') {
-            if (r < n_queries)
-                off[r + 1] = p0 + i + 1;
-            else
-                atomicOr(&header[1], 1u);
-            r++;
-        }
+    for (; nl; nl &= nl - 1, r++) {
+        if (r < n_queries)
+            off[r + 1] = p0 + (uint32_t)__builtin_ctzll(nl) + 1;
+        else
+            atomicOr(&header[1], 1u);
     }
     if (blockIdx.x == 0 && t == 0) off[0] = 0;
 }
@@ -164,6 +176,50 @@ __global__ void na_init_kernel(const uint64_t* off, uint32_t n_queries, uint32_t
         matched[q] = 0;
     }
     for (uint64_t i = i0; i < (uint64_t)n_queries * n_colors; i += step) color_counts[i] = 0;
+}
+
+// Start offsets of the queries seq[0, n_bytes) (device memory), the counters
+// that the query adds to cleared, and query_kmers where wanted; block_nl holds
+// a word per NA_BLOCK_BYTES bytes, header 64 words.  Waits, and fails when the
+// bytes are not n_queries records.
+static int query_prepare(ggcat_gpu_ctx* ctx, const uint8_t* seq, uint64_t n_bytes, uint32_t n_queries, uint32_t* header,
+                         uint32_t* block_nl, uint64_t* off, uint64_t* query_kmers, uint64_t* matched,
+                         uint32_t* color_counts, uint32_t nc) {
+    const uint32_t nb = (uint32_t)((n_bytes + NA_BLOCK_BYTES - 1) / NA_BLOCK_BYTES);
+    hipLaunchKernelGGL(na_count_kernel, dim3(nb), dim3(256), 0, ctx->stream, seq, n_bytes, block_nl);
+    hipLaunchKernelGGL(na_scan_kernel, dim3(1), dim3(1024), 0, ctx->stream, block_nl, nb, header);
+    hipLaunchKernelGGL(na_fill_kernel, dim3(nb), dim3(256), 0, ctx->stream, seq, n_bytes, block_nl, off, n_queries,
+                       header);
+    hipLaunchKernelGGL(na_check_kernel, dim3(1), dim3(64), 0, ctx->stream, seq, n_bytes, n_queries, header);
+    HIPCHK(hipGetLastError());
+    HIPCHK(hipMemcpyAsync(ctx->seen, header, 8, hipMemcpyDeviceToHost, ctx->stream));
+    HIPCHK(hipStreamSynchronize(ctx->stream));
+    if (ctx->seen[0] >> 32) return fail(ctx, GGCAT_GPU_EINVAL, "queries must be n_queries records, each ending with '\\n'");
+    const uint32_t grid =
+        (uint32_t)std::min<uint64_t>(((uint64_t)n_queries * std::max(nc, 1u) + 255) / 256, (uint64_t)ctx->n_cu * 16);
+    hipLaunchKernelGGL(na_init_kernel, dim3(grid), dim3(256), 0, ctx->stream, off, n_queries, ctx->P.k, query_kmers,
+                       matched, color_counts, nc);
+    HIPCHK(hipGetLastError());
+    return GGCAT_GPU_OK;
+}
+
+// Whether a batch of host queries finds its offsets on the device: the host
+// takes about 0.13 ms per MB to look for the newlines, the device's five
+// launches and one more wait 0.06 ms in all.  The block counts' scan takes
+// NA_MAX_BLOCKS blocks.
+static bool query_offsets_on_device(uint64_t n_bytes, uint32_t n_queries) {
+    return n_queries && n_bytes >= (1u << 20) && n_bytes <= (uint64_t)NA_MAX_BLOCKS * NA_BLOCK_BYTES;
+}
+
+// Offsets, k-mer counts and cleared counters of the n_bytes uploaded to
+// ctx->q_seq; k-mer counts go to ctx->q_kmers.
+static int query_prepare_uploaded(ggcat_gpu_ctx* ctx, uint64_t n_bytes, uint32_t n_queries, uint32_t nc) {
+    ENSURE(ctx->q_kmers, (size_t)n_queries * 8);
+    ENSURE(ctx->q_blocks, 256 + (n_bytes / NA_BLOCK_BYTES + 1) * 4);
+    uint32_t* header = P_<uint32_t>(ctx->q_blocks);
+    hipLaunchKernelGGL(na_clear_kernel, dim3(1), dim3(64), 0, ctx->stream, header);
+    return query_prepare(ctx, P_<uint8_t>(ctx->q_seq), n_bytes, n_queries, header, header + 64, P_<uint64_t>(ctx->q_off),
+                         P_<uint64_t>(ctx->q_kmers), P_<uint64_t>(ctx->q_matched), P_<uint32_t>(ctx->q_counts), nc);
 }
 
 }  // namespace
@@ -190,21 +246,9 @@ extern "C" int ggcat_gpu_query_device_noalloc(ggcat_gpu_ctx* ctx, const uint8_t*
     hipLaunchKernelGGL(na_clear_kernel, dim3(1), dim3(64), 0, ctx->stream, header);
     HIPCHK(hipGetLastError());
     if (n_queries == 0 && n_bytes == 0) return GGCAT_GPU_OK;
-    const uint32_t nb = (uint32_t)((n_bytes + NA_BLOCK_BYTES - 1) / NA_BLOCK_BYTES);
-    hipLaunchKernelGGL(na_count_kernel, dim3(nb), dim3(256), 0, ctx->stream, d_queries, n_bytes, block_nl);
-    hipLaunchKernelGGL(na_scan_kernel, dim3(1), dim3(1024), 0, ctx->stream, block_nl, nb, header);
-    hipLaunchKernelGGL(na_fill_kernel, dim3(nb), dim3(256), 0, ctx->stream, d_queries, n_bytes, block_nl, off,
-                       n_queries, header);
-    hipLaunchKernelGGL(na_check_kernel, dim3(1), dim3(64), 0, ctx->stream, d_queries, n_bytes, n_queries, header);
-    HIPCHK(hipGetLastError());
-    uint32_t err = 0;
-    HIPCHK(hipMemcpyAsync(&err, header + 1, 4, hipMemcpyDeviceToHost, ctx->stream));
-    HIPCHK(hipStreamSynchronize(ctx->stream));
-    if (err) return fail(ctx, GGCAT_GPU_EINVAL, "queries must be n_queries records, each ending with '\\n'");
-    const uint32_t grid =
-        (uint32_t)std::min<uint64_t>(((uint64_t)n_queries * std::max(nc, 1u) + 255) / 256, (uint64_t)ctx->n_cu * 16);
-    hipLaunchKernelGGL(na_init_kernel, dim3(grid), dim3(256), 0, ctx->stream, off, n_queries, ctx->P.k, d_query_kmers,
-                       d_matched, d_color_counts, nc);
+    const int r = query_prepare(ctx, d_queries, n_bytes, n_queries, header, block_nl, off, d_query_kmers, d_matched,
+                                d_color_counts, nc);
+    if (r != GGCAT_GPU_OK) return r;
     QueryArgs Q = query_args(ctx);
     Q.seq = d_queries;
     Q.qoff = off;

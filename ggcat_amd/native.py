@@ -508,10 +508,19 @@ class GpuContext:
         self._check(self.lib.ggcat_gpu_index_colors(self.h, C.byref(n)), "ggcat_gpu_index_colors")
         return n.value
 
+    @staticmethod
+    def _count_records(q: np.ndarray) -> int:
+        """Newlines of a uint8 array, 256 KB at a time so that the comparison's
+        result stays in cache (15 MB: 1.8 ms, 3.5 in one piece)."""
+        step = 1 << 18
+        if q.size <= step:
+            return int(np.count_nonzero(q == 10))
+        return sum(int(np.count_nonzero(q[i:i + step] == 10)) for i in range(0, q.size, step))
+
     def query(self, queries: np.ndarray):
         """Joined queries -> (query_kmers, matched, color_counts (n, n_colors) or None)."""
         q = np.ascontiguousarray(queries, np.uint8)
-        nq = int(np.count_nonzero(q == 10))
+        nq = self._count_records(q)
         nc = self.index_colors()
         qk, mt = np.zeros(nq, np.uint64), np.zeros(nq, np.uint64)
         cc = np.zeros((nq, max(nc, 1)), np.uint32)
@@ -527,7 +536,7 @@ class GpuContext:
         q = np.ascontiguousarray(queries, np.uint8)
         t = C.c_uint64()
         self._check(self.lib.ggcat_gpu_serve_submit(self.h, q.ctypes.data_as(C.c_void_p), q.size,
-                                                    int(np.count_nonzero(q == 10)), C.byref(t)),
+                                                    self._count_records(q), C.byref(t)),
                     "ggcat_gpu_serve_submit")
         return t.value
 
