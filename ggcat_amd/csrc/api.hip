@@ -101,6 +101,7 @@ struct ggcat_gpu_ctx {
     uint32_t n_color_ids = 0;  // largest color id + 1 of the colored build
     // query index over the solid table
     DevBuf idx_slots, idx_count;
+    DevBuf idx_off;  // large tables: the partitions' starts
     bool have_index = false;
     gg::KmerTable idx{};
     DevBuf q_seq, q_off, q_matched, q_counts, q_kmers, q_blocks;
@@ -278,8 +279,37 @@ int table_build(ggcat_gpu_ctx* ctx, uint64_t n, DevBuf& slots, DevBuf& count, Km
     T.key_words = ctx->key_words;
     const uint64_t slot_words = (uint64_t)T.nb * TAB_BUCKET * T.key_words * 4;  // 32-bit
     ENSURE(slots, slot_words * 4);
-    ENSURE(count, (size_t)T.nb * 4);
     T.slots = P_<ulonglong2>(slots);
+    if (const uint32_t shift = part_shift(n, T.nb, T.key_words)) {
+        const uint32_t n_part = ((T.nb - 1) >> shift) + 1;
+        // per partition: entries, reserved entries; then the overflow's count and list
+        ENSURE(count, ((size_t)2 * n_part + 2) * 4);
+        ENSURE(ctx->idx_off, ((size_t)n_part + 1) * 8);
+        // gathered entries and overflow list: in the bucketing's unit regions,
+        // which nothing reads once the records are compacted
+        ENSURE(ctx->stage_slots, n * 20);
+        uint32_t* counts = P_<uint32_t>(count);
+        uint64_t* off = P_<uint64_t>(ctx->idx_off);
+        const uint64_t* key = P_<uint64_t>(ctx->out_key);
+        ulonglong2* part = P_<ulonglong2>(ctx->stage_slots);
+        uint32_t* rest = reinterpret_cast<uint32_t*>(part + n);
+        hipLaunchKernelGGL(fill32_kernel, dim3(16), dim3(256), 0, ctx->stream, counts, 0u, (uint64_t)2 * n_part + 2);
+        const uint64_t steps = (n + 1024 * PART_EACH - 1) / (1024 * PART_EACH);
+        const uint32_t grid = (uint32_t)std::min<uint64_t>(steps, (uint64_t)ctx->n_cu * 2);
+        hipLaunchKernelGGL(part_count_kernel, dim3(grid), dim3(1024), 0, ctx->stream, T, key, n, shift, n_part, counts);
+        const int r = device_scan(ctx, counts, off, n_part);
+        if (r != GGCAT_GPU_OK) return r;
+        hipLaunchKernelGGL(part_gather_kernel, dim3(grid), dim3(1024), 0, ctx->stream, T, key, n, shift, n_part, off,
+                           counts + n_part, part);
+        hipLaunchKernelGGL(part_insert_kernel, dim3(n_part), dim3(1024), (size_t)4 << shift, ctx->stream, T, shift, off,
+                           part, rest, counts + 2 * n_part);
+        hipLaunchKernelGGL(part_rest_kernel, dim3(64), dim3(256), 0, ctx->stream, T, shift, part,
+                           rest, counts + 2 * n_part);
+        HIPCHK(hipGetLastError());
+        *out = T;
+        return GGCAT_GPU_OK;
+    }
+    ENSURE(count, (size_t)T.nb * 4);
     T.count = P_<uint32_t>(count);
     const uint32_t wide = (uint32_t)ctx->n_cu * 16;
     hipLaunchKernelGGL(fill32_kernel, dim3((uint32_t)std::min<uint64_t>((slot_words + 255) / 256, wide)), dim3(256), 0,
@@ -575,7 +605,7 @@ void ggcat_gpu_destroy(ggcat_gpu_ctx* ctx) {
                       &ctx->parts, &ctx->redo, &ctx->out_key,
                       &ctx->out_val, &ctx->out_sub, &ctx->chunk_fill_dev, &ctx->chunk_off, &ctx->fix_key,
                       &ctx->fix_val, &ctx->fix_sub, &ctx->out_colors, &ctx->fix_colors,
-                      &ctx->idx_slots, &ctx->idx_count,
+                      &ctx->idx_slots, &ctx->idx_count, &ctx->idx_off,
                       &ctx->q_seq, &ctx->q_off, &ctx->q_matched, &ctx->q_counts, &ctx->q_kmers, &ctx->q_blocks,
                       &ctx->u_nb, &ctx->u_ext, &ctx->u_link, &ctx->u_seg, &ctx->u_head, &ctx->u_uhead,
                       &ctx->u_ubytes, &ctx->u_uoff, &ctx->u_totals, &ctx->u_seq, &ctx->u_sub, &ctx->u_flags, &ctx->u_visited, &ctx->u_rest,
