@@ -38,11 +38,11 @@ __global__ void fill32_kernel(uint32_t* p, uint32_t v, uint64_t n) {
 // each), cleared by one launch and read back by one copy into pinned memory:
 // single fills and copies cost 10 to 40 us apiece, most of a small build's time
 // (30 kbp genome with its table 0.94 -> 0.69 ms, 64 colors of 41 MB 2.42 -> 2.21).
-enum Cursor : uint32_t { CU_SPILL, CU_POOL, CU_KMERS, CU_DEFER, CU_ERROR, CU_ITEMS, CU_WORK, CU_REDO, CU_CHUNK, CU_FIX, CU_ADDED, CU_TOTAL, N_CURSORS };
-constexpr uint32_t CURSOR_STRIDE = 8;
+enum Cursor : uint32_t { CU_POOL, CU_KMERS, CU_DEFER, CU_ERROR, CU_ITEMS, CU_WORK, CU_REDO, CU_CHUNK, CU_FIX, CU_ADDED, CU_TOTAL, CU_SPILL, N_CURSORS = CU_SPILL + SPILL_STRIPES };
+constexpr uint32_t CURSOR_STRIDE = SPILL_STRIDE;
 constexpr size_t CURSOR_BYTES = (size_t)N_CURSORS * CURSOR_STRIDE * 8;
 __global__ void clear_cursors_kernel(unsigned long long* c, uint32_t which) {
-    if (threadIdx.x < N_CURSORS && ((which >> threadIdx.x) & 1u)) c[threadIdx.x * CURSOR_STRIDE] = 0;
+    if (threadIdx.x < CU_SPILL && ((which >> threadIdx.x) & 1u)) c[threadIdx.x * CURSOR_STRIDE] = 0;
 }
 
 namespace {
@@ -786,7 +786,7 @@ int ggcat_gpu_bucketing(ggcat_gpu_ctx* ctx, const uint8_t* data, uint64_t n_byte
         ctx->tune.unit_cap ? ctx->tune.unit_cap
                            : (uint32_t)std::max<uint64_t>(16, std::min<uint64_t>(1u << 16, ((est_records * 5 / 2) / n_units + 15) / 8 * 8));
     A.unit_cap = unit_cap;
-    uint64_t spill_cap = std::max<uint64_t>(n_bytes / 64 + 65536, ctx->stage_unit.cap / 4);
+    uint64_t spill_cap = std::max<uint64_t>(n_bytes / 64 + 65536, ctx->stage_unit.cap / 4 / SPILL_STRIPES * SPILL_STRIPES);
     uint64_t pool_cap = std::max<uint64_t>(ctx->pool.cap / 4, n_bytes / 64 + 65536);
     const uint32_t small_grid = (uint32_t)std::min<uint64_t>((std::max<uint64_t>(n_tiles, 1) + 255) / 256, 65535);
     auto pass_1 = [&]() {
@@ -859,11 +859,15 @@ int ggcat_gpu_bucketing(ggcat_gpu_ctx* ctx, const uint8_t* data, uint64_t n_byte
         HIPCHK(hipGetLastError());
         return GGCAT_GPU_OK;
     };
-    uint64_t staged = 0, pool_used = 0;
+    uint64_t staged = 0, longest = 0, pool_used = 0;  // spilled records in all and of the longest stripe
     uint32_t errf = 0;
     for (int attempt = 0;; attempt++) {
         const uint64_t region_slots = (uint64_t)n_units * unit_cap;
         ENSURE(ctx->stage_slots, region_slots * slot_words * 4);
+        // one stripe when a stripe was short: the sum is the same on every attempt
+        A.spill_stripes = attempt ? 1 : SPILL_STRIPES;
+        A.spill_cap = (spill_cap + A.spill_stripes - 1) / A.spill_stripes;
+        spill_cap = A.spill_cap * A.spill_stripes;
         ENSURE(ctx->spill_slots, spill_cap * slot_words * 4);
         ENSURE(ctx->stage_unit, spill_cap * 4);
         ENSURE(ctx->stage_rank, spill_cap * 4);
@@ -878,7 +882,6 @@ int ggcat_gpu_bucketing(ggcat_gpu_ctx* ctx, const uint8_t* data, uint64_t n_byte
         A.spill_unit = P_<uint32_t>(ctx->stage_unit);
         A.spill_rank = P_<uint32_t>(ctx->stage_rank);
         A.spill_color = n_colors ? P_<uint32_t>(ctx->spill_color) : nullptr;
-        A.spill_cap = spill_cap;
         A.pool = P_<uint32_t>(ctx->pool);
         A.pool_cap = pool_cap;
         HIPCHK(hipEventRecord(ctx->ev[0], ctx->stream));
@@ -914,13 +917,20 @@ int ggcat_gpu_bucketing(ggcat_gpu_ctx* ctx, const uint8_t* data, uint64_t n_byte
         HIPCHK(hipGetLastError());
         HIPCHK(hipEventRecord(ctx->ev[1], ctx->stream));
         FETCH(nullptr);
-        staged = seen<uint64_t>(ctx, CU_SPILL);
+        staged = longest = 0;
+        for (uint32_t q = 0; q < A.spill_stripes; q++) {
+            const uint64_t c = ctx->seen[(CU_SPILL + q) * CURSOR_STRIDE];
+            staged += c;
+            longest = std::max(longest, c);
+        }
         pool_used = seen<uint64_t>(ctx, CU_POOL);
         errf = seen<uint32_t>(ctx, CU_ERROR);
         if (errf & 8) return fail(ctx, GGCAT_GPU_ENOMEM, "a physical unit exceeds 2^32 k-mer occurrences");
         if (errf) return fail(ctx, GGCAT_GPU_EHIP, "bucketing: a group start was not found");
-        if (staged <= spill_cap && pool_used <= pool_cap) break;
-        if (attempt == 1) return fail(ctx, GGCAT_GPU_ENOMEM, "bucketing spill list overflow");
+        if (longest <= A.spill_cap && pool_used <= pool_cap) break;
+        // (records that found no spill entry did not count their pool words: a
+        // second retry may be for those)
+        if (attempt == 2) return fail(ctx, GGCAT_GPU_ENOMEM, "bucketing spill list overflow");
         spill_cap = std::max(spill_cap, staged + 1024);
         pool_cap = std::max(pool_cap, pool_used + 1024);
     }
@@ -984,8 +994,9 @@ int ggcat_gpu_bucketing(ggcat_gpu_ctx* ctx, const uint8_t* data, uint64_t n_byte
         hipLaunchKernelGGL(unit_compact_kernel, dim3(grid), dim3(256), 0, ctx->stream, A, n_units);
     }
     if (staged) {
-        const uint32_t grid = (uint32_t)std::min<uint64_t>((staged + 255) / 256, (uint64_t)ctx->n_cu * 64);
-        hipLaunchKernelGGL(spill_place_kernel, dim3(grid), dim3(256), 0, ctx->stream, A, staged);
+        const uint32_t grid =
+            (uint32_t)std::min<uint64_t>((longest * A.spill_stripes + 255) / 256, (uint64_t)ctx->n_cu * 64);
+        hipLaunchKernelGGL(spill_place_kernel, dim3(grid), dim3(256), 0, ctx->stream, A, longest);
     }
     HIPCHK(hipGetLastError());
     HIPCHK(hipEventRecord(ctx->ev[4], ctx->stream));

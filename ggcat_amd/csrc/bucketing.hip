@@ -39,6 +39,12 @@ namespace gg {
 // 64-bit words of the rolling-hash tables (BucketArgs::gtab).
 constexpr uint32_t GTAB_WORDS = 2 * (20 + 16);
 
+// Stripes of the spill list, their cursors a line apart: the updates of one
+// cursor wait for each other (0.23 Gbases with m = 11, whose frequent minimizers
+// overfill 3 % of the units: staging pass 2.4 ms with one, 1.4 to 1.8 with 64).
+constexpr uint32_t SPILL_STRIPES = 64;
+constexpr uint32_t SPILL_STRIDE = 8;
+
 // Records are scattered by physical unit: the sub-bucket (the semantic unit,
 // one kmers_transform job) refined by `xb` further bits of the minimizer hash
 // for unique minimizers.  Units of one sub-bucket are contiguous, so the merge
@@ -62,12 +68,15 @@ struct BucketArgs {
     uint32_t unit_cap;
     uint32_t* region;  // [n_units * unit_cap * slot_words]
     uint32_t* region_color;  // [n_units * unit_cap] (colored builds)
-    uint32_t* spill_slots;  // [spill_cap * slot_words]
-    uint32_t* spill_unit;  // [spill_cap]
-    uint32_t* spill_rank;  // [spill_cap]
-    uint32_t* spill_color;  // [spill_cap] (colored builds)
-    unsigned long long* spill_cursor;  // spilled records (may exceed spill_cap: the host retries)
+    // the list is cut into spill_stripes (a power of two, at most SPILL_STRIPES)
+    // of spill_cap entries, a workgroup appending to the one of its index
+    uint32_t* spill_slots;  // [spill_stripes * spill_cap * slot_words]
+    uint32_t* spill_unit;  // [spill_stripes * spill_cap]
+    uint32_t* spill_rank;  // [spill_stripes * spill_cap]
+    uint32_t* spill_color;  // [spill_stripes * spill_cap] (colored builds)
+    unsigned long long* spill_cursor;  // a stripe's records at SPILL_STRIDE * stripe (may exceed spill_cap: the host retries)
     uint64_t spill_cap;
+    uint32_t spill_stripes;
     uint64_t* defer;  // [n_tiles * 3] records whose group starts before the tile: end window, minimizer, last flag
     unsigned int* defer_count;
     unsigned long long* kmer_total;  // k-mer occurrences of all records
@@ -895,9 +904,11 @@ GG_DEV uint32_t* record_dest(const BucketArgs& A, uint32_t unit, uint32_t rank, 
         *color_at = A.region_color ? A.region_color + slot : nullptr;
         return A.region + slot * SW;
     }
-    const unsigned long long pos = atomicAdd(A.spill_cursor, 1ULL);
+    const uint32_t stripe = blockIdx.x & (A.spill_stripes - 1);
+    unsigned long long pos = atomicAdd(A.spill_cursor + stripe * SPILL_STRIDE, 1ULL);
     *color_at = nullptr;
     if (pos >= A.spill_cap) return nullptr;
+    pos += stripe * A.spill_cap;
     A.spill_unit[pos] = unit;
     A.spill_rank[pos] = rank;
     if (A.spill_color) *color_at = A.spill_color + pos;
@@ -1100,8 +1111,8 @@ __global__ void sub_totals_kernel(const uint32_t* unit_count, const uint32_t* un
 
 // Clears the cursors of pass 1 (a kernel, so the pass can be captured in a graph).
 __global__ void bucket_reset_kernel(BucketArgs A) {
+    if (threadIdx.x < SPILL_STRIPES) A.spill_cursor[threadIdx.x * SPILL_STRIDE] = 0;
     if (threadIdx.x == 0) {
-        *A.spill_cursor = 0;
         *A.pool_cursor = 0;
         A.kmer_total[0] = 0;
         A.kmer_total[1] = 0;
@@ -1325,11 +1336,14 @@ __global__ __launch_bounds__(256) void unit_compact_kernel(BucketArgs A, uint32_
 }
 
 // Pass 2c: spilled records (rank >= unit_cap) after their unit's stored
-// region records.
-__global__ void spill_place_kernel(BucketArgs A, uint64_t n_spill) {
+// region records.  longest: the longest stripe's records.
+__global__ void spill_place_kernel(BucketArgs A, uint64_t longest) {
     const uint32_t SW = A.slot_words;
-    for (uint64_t i = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; i < n_spill;
-         i += (uint64_t)gridDim.x * blockDim.x) {
+    for (uint64_t e = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; e < longest * A.spill_stripes;
+         e += (uint64_t)gridDim.x * blockDim.x) {
+        const uint32_t stripe = (uint32_t)(e / longest);
+        const uint64_t at = e - stripe * longest, i = stripe * A.spill_cap + at;
+        if (at >= A.spill_cursor[stripe * SPILL_STRIDE]) continue;
         const uint32_t unit = A.spill_unit[i];
         const uint64_t slot = A.sub_off[unit] + A.unit_dregion[unit] + (A.spill_rank[i] - A.unit_cap);
         if (slot >= A.sub_off[unit + 1]) {
