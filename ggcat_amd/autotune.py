@@ -46,17 +46,23 @@ class Schedule:
 def default_grid(k: int) -> list[Schedule]:
     """Unit size x record-table size x LDS table size: the knobs whose best
     value depends on the input (coverage, error rate, k); the others are
-    fixed at values that measured best on every configuration tried."""
+    fixed at values that measured best on every configuration tried.  A sample
+    has few enough units for their counters and open lines to stay in cache,
+    whatever their size; a full input does not (4 Gbases, k = 31: staging 33.1
+    ms with units of 1000 bytes, 22.7 with 2000), so smaller units are tried
+    for k > 32 only, whose records are fewer."""
     logs = (11,) if k <= 32 else (10,)
+    sizes = (2000, 3000) if k <= 32 else (1400, 2000, 3000)
     out = []
-    for ub, rc, lg in itertools.product((1400, 2000, 3000), (256, 512), logs):
+    for ub, rc, lg in itertools.product(sizes, (256, 512), logs):
         out.append(Schedule(unit_bytes=ub, table_pct=200, lds_table_log=lg, rec_cap=rc, use_graphs=1))
-    # smaller tables over smaller units, in workgroups of 128 and 256 threads
+    # smaller tables over small units, in workgroups of 128 and 256 threads
     # (more resident workgroups per CU)
-    out.append(Schedule(unit_bytes=1000, table_pct=200, lds_table_log=lg - 1, rec_cap=128, use_graphs=1,
+    small = sizes[0]
+    out.append(Schedule(unit_bytes=small, table_pct=200, lds_table_log=lg - 1, rec_cap=128, use_graphs=1,
                         merge_threads=128))
     for rc in (128, 256):
-        out.append(Schedule(unit_bytes=1000, table_pct=200, lds_table_log=lg - 1, rec_cap=rc, use_graphs=1,
+        out.append(Schedule(unit_bytes=small, table_pct=200, lds_table_log=lg - 1, rec_cap=rc, use_graphs=1,
                             merge_threads=256))
     return out
 
