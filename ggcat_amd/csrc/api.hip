@@ -1697,8 +1697,12 @@ int ggcat_gpu_kmers_merge(ggcat_gpu_ctx* ctx) {
                 if (w.item >= n_items) return fail(ctx, GGCAT_GPU_EHIP, "corrupt merge work list");
                 uint32_t L, base, stride;
                 if (w.log_parts == 0) {
-                    // about half a table of occurrences per part
-                    const uint64_t per = ctx->tune.part_occ ? ctx->tune.part_occ : M.lds_cap / 2;
+                    // up to three quarters of a table of occurrences per part: every
+                    // part reads all of the item's records, and even distinct
+                    // k-mers fit.  8.9 K items of 0.9 Gbases, k = 63: 1.57 ms
+                    // with half a table, 1.08; with 1.5 tables 0.70, but then
+                    // inputs without repeated k-mers are split twice
+                    const uint64_t per = ctx->tune.part_occ ? ctx->tune.part_occ : M.lds_cap / 4 * 3;
                     const uint64_t want = (w.occ + per - 1) / per;
                     L = 1;
                     while ((1ull << L) < want) L++;

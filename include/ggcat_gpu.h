@@ -198,7 +198,7 @@ int ggcat_gpu_solid_colors(ggcat_gpu_ctx* ctx, uint32_t* color_words, uint32_t* 
  *                     16x the LDS table
  *   merge_wgs_per_cu  persistent merge workgroups per CU; default 6
  *   part_occ          target occurrences per partition of an item that is
- *                     split into hash-partitioned passes; default half the
+ *                     split into hash-partitioned passes; default 3/4 of the
  *                     LDS table (a partition that still overflows is split
  *                     4 ways again)
  *   lds_table_log     log2 of the LDS table entries per workgroup (8..13;
