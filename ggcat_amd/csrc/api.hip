@@ -1572,7 +1572,14 @@ int ggcat_gpu_kmers_merge(ggcat_gpu_ctx* ctx) {
     M.color_words = W;
     M.slot_color = W ? P_<uint32_t>(ctx->slot_color) : nullptr;
     M.lds_try = ctx->tune.lds_max_occ ? ctx->tune.lds_max_occ : M.lds_cap * 16;
-    const uint32_t item_occ = ctx->tune.item_occ ? ctx->tune.item_occ : M.lds_cap / 2;
+    // Occurrences per work item: half a table, three quarters of one with
+    // two-word keys, whose tables are half as large, so that an item's fixed
+    // cost weighs more (merge of 551 M occurrences, k = 63, 9.8 ms with half,
+    // 9.4 with three quarters, 9.2 with a whole table, which all-distinct
+    // k-mers would overflow; one-word keys, 1.57 G: 8.6 with half, 9.1 with
+    // three eighths)
+    const uint32_t item_occ =
+        ctx->tune.item_occ ? ctx->tune.item_occ : mode != 0 && table_words == 2 ? M.lds_cap / 4 * 3 : M.lds_cap / 2;
     // work items whose units the compaction deduplicated skip the record hashing
     M.rec_direct = ctx->tune.no_dedup != 3 ? 1 : 0;
     // workgroup size of the merge (128 or 256 threads); a chunk of records

@@ -192,7 +192,8 @@ int ggcat_gpu_solid_colors(ggcat_gpu_ctx* ctx, uint32_t* color_words, uint32_t* 
  * handle a work item, never the result.  Zero selects the default.
  *   item_occ          target k-mer occurrences per work item (runs of
  *                     physical units of one sub-bucket); default: half the
- *                     LDS table (1024 for 64-bit keys, 512 for 128-bit)
+ *                     LDS table (1024) for 64-bit table keys, three quarters
+ *                     (768) for 128-bit ones
  *   lds_max_occ       items with more occurrences skip the whole-item pass
  *                     and go straight to hash-partitioned passes; default
  *                     16x the LDS table
