@@ -78,6 +78,7 @@ struct ggcat_gpu_ctx {
     // state
     ggcat_gpu_params P{};
     bool have_records = false, have_solid = false;
+    bool have_values = false;  // the table has multiplicities, flags and sub-buckets (a graph read from files has keys)
     uint32_t n_sub = 0, n_units = 0, xb = 0, slot_words = 0, key_words = 1;
     uint64_t n_records = 0, pool_words = 0, n_solid = 0, n_input = 0, kmer_occ = 0, n_big = 0, n_fix = 0;
     uint64_t n_stored = 0;  // arena slots: records with identical copies stored once
@@ -1828,7 +1829,7 @@ int ggcat_gpu_kmers_merge(ggcat_gpu_ctx* ctx) {
         HIPCHK(hipEventSynchronize(ctx->ev[10]));
         HIPCHK(hipEventElapsedTime(&t, ctx->ev[5], ctx->ev[10]));
         ctx->ms[6] = t;
-        ctx->have_solid = true;
+        ctx->have_solid = ctx->have_values = true;
         return GGCAT_GPU_OK;
     }
     return fail(ctx, GGCAT_GPU_ENOMEM, "solid output overflow");
@@ -1848,9 +1849,8 @@ int ggcat_gpu_solid_copy(ggcat_gpu_ctx* ctx, uint64_t* keys, uint32_t* multiplic
     HIPCHK(hipSetDevice(ctx->device));
     const uint32_t kw = ctx->key_words;
     const uint64_t n = ctx->n_solid;
-    // a graph read from files has keys only
-    if (((multiplicity || flags) && ctx->out_val.cap < n * 4) || (sub && ctx->out_sub.cap < n * 4))
-        return fail(ctx, GGCAT_GPU_EHIP, "the table holds keys only");
+    if ((multiplicity || flags || sub) && !ctx->have_values)
+        return fail(ctx, GGCAT_GPU_ESTATE, "the table of a graph read from files holds keys only");
     if (n && keys) HIPCHK(hipMemcpy(keys, ctx->out_key.p, n * 8 * kw, hipMemcpyDeviceToHost));
     if (n && sub) HIPCHK(hipMemcpy(sub, ctx->out_sub.p, n * 4, hipMemcpyDeviceToHost));
     if (multiplicity || flags) {
@@ -2513,6 +2513,8 @@ namespace {
 // or over the whole table, joined across sub-buckets (joined == true).
 static int build_unitigs(ggcat_gpu_ctx* ctx, bool joined, uint64_t* n_unitigs, uint64_t* n_bytes) {
     if (!ctx->have_solid) return fail(ctx, GGCAT_GPU_ESTATE, "no merge result");
+    if (!ctx->have_values)
+        return fail(ctx, GGCAT_GPU_ESTATE, "the table of a graph read from files holds keys only");
     if (ctx->P.hash_kind != GGCAT_GPU_HASH_SEQ)
         return fail(ctx, GGCAT_GPU_EINVAL, "unitig extension needs seq-hash keys (the k-mer is the key)");
     HIPCHK(hipSetDevice(ctx->device));

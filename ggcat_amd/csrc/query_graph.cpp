@@ -334,6 +334,7 @@ extern "C" int ggcat_gpu_query_graph(ggcat_gpu_ctx* ctx, const char* input_graph
     ctx->P.k = k;
     ctx->P.hash_kind = hash_kind;
     ctx->have_solid = true;
+    ctx->have_values = false;
     int r = ggcat_gpu_index_build(ctx);
     if (r != GGCAT_GPU_OK) return r;
     gg_host::ReadResult Q;
