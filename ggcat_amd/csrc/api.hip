@@ -566,6 +566,7 @@ extern "C" {
 namespace {
 static int noalloc_scratch_setup(int device);
 static bool query_offsets_on_device(uint64_t n_bytes, uint32_t n_queries);
+static int query_check_uploaded(ggcat_gpu_ctx* ctx, uint64_t n_bytes, uint32_t n_queries);
 static int query_prepare_uploaded(ggcat_gpu_ctx* ctx, uint64_t n_bytes, uint32_t n_queries, uint32_t nc);
 }  // namespace
 
@@ -2330,10 +2331,14 @@ int ggcat_gpu_query(ggcat_gpu_ctx* ctx, const uint8_t* queries, uint64_t n_bytes
     HIPCHK(hipSetDevice(ctx->device));
     const uint32_t nc = ctx->colored ? ctx->n_color_ids : 0;
     ENSURE(ctx->q_seq, n_bytes + 16);
+    if (n_bytes) HIPCHK(hipMemcpy(ctx->q_seq.p, queries, n_bytes, hipMemcpyHostToDevice));
+    if (on_device) {
+        const int r = query_check_uploaded(ctx, n_bytes, n_queries);
+        if (r != GGCAT_GPU_OK) return r;
+    }
     ENSURE(ctx->q_off, ((size_t)n_queries + 1) * 8);
     ENSURE(ctx->q_matched, (size_t)n_queries * 8 + 8);
     ENSURE(ctx->q_counts, (size_t)n_queries * nc * 4 + 4);
-    if (n_bytes) HIPCHK(hipMemcpy(ctx->q_seq.p, queries, n_bytes, hipMemcpyHostToDevice));
     if (on_device) {
         const int r = query_prepare_uploaded(ctx, n_bytes, n_queries, nc);
         if (r != GGCAT_GPU_OK) return r;

@@ -178,23 +178,30 @@ __global__ void na_init_kernel(const uint64_t* off, uint32_t n_queries, uint32_t
     for (uint64_t i = i0; i < (uint64_t)n_queries * n_colors; i += step) color_counts[i] = 0;
 }
 
-// Start offsets of the queries seq[0, n_bytes) (device memory), the counters
-// that the query adds to cleared, and query_kmers where wanted; block_nl holds
-// a word per NA_BLOCK_BYTES bytes, header 64 words.  Waits, and fails when the
-// bytes are not n_queries records.
-static int query_prepare(ggcat_gpu_ctx* ctx, const uint8_t* seq, uint64_t n_bytes, uint32_t n_queries, uint32_t* header,
-                         uint32_t* block_nl, uint64_t* off, uint64_t* query_kmers, uint64_t* matched,
-                         uint32_t* color_counts, uint32_t nc) {
+// Newlines before each NA_BLOCK_BYTES bytes of seq[0, n_bytes) (device memory)
+// in block_nl, a word per block; header holds 64 words.  Waits, and fails when
+// the bytes are not n_queries records.
+static int query_check(ggcat_gpu_ctx* ctx, const uint8_t* seq, uint64_t n_bytes, uint32_t n_queries, uint32_t* header,
+                       uint32_t* block_nl) {
     const uint32_t nb = (uint32_t)((n_bytes + NA_BLOCK_BYTES - 1) / NA_BLOCK_BYTES);
     hipLaunchKernelGGL(na_count_kernel, dim3(nb), dim3(256), 0, ctx->stream, seq, n_bytes, block_nl);
     hipLaunchKernelGGL(na_scan_kernel, dim3(1), dim3(1024), 0, ctx->stream, block_nl, nb, header);
-    hipLaunchKernelGGL(na_fill_kernel, dim3(nb), dim3(256), 0, ctx->stream, seq, n_bytes, block_nl, off, n_queries,
-                       header);
     hipLaunchKernelGGL(na_check_kernel, dim3(1), dim3(64), 0, ctx->stream, seq, n_bytes, n_queries, header);
     HIPCHK(hipGetLastError());
     HIPCHK(hipMemcpyAsync(ctx->seen, header, 8, hipMemcpyDeviceToHost, ctx->stream));
     HIPCHK(hipStreamSynchronize(ctx->stream));
     if (ctx->seen[0] >> 32) return fail(ctx, GGCAT_GPU_EINVAL, "queries must be n_queries records, each ending with '\\n'");
+    return GGCAT_GPU_OK;
+}
+
+// After query_check: the queries' start offsets, the counters that the query
+// adds to cleared, and query_kmers where wanted.
+static int query_prepare(ggcat_gpu_ctx* ctx, const uint8_t* seq, uint64_t n_bytes, uint32_t n_queries, uint32_t* header,
+                         const uint32_t* block_nl, uint64_t* off, uint64_t* query_kmers, uint64_t* matched,
+                         uint32_t* color_counts, uint32_t nc) {
+    const uint32_t nb = (uint32_t)((n_bytes + NA_BLOCK_BYTES - 1) / NA_BLOCK_BYTES);
+    hipLaunchKernelGGL(na_fill_kernel, dim3(nb), dim3(256), 0, ctx->stream, seq, n_bytes, block_nl, off, n_queries,
+                       header);
     const uint32_t grid =
         (uint32_t)std::min<uint64_t>(((uint64_t)n_queries * std::max(nc, 1u) + 255) / 256, (uint64_t)ctx->n_cu * 16);
     hipLaunchKernelGGL(na_init_kernel, dim3(grid), dim3(256), 0, ctx->stream, off, n_queries, ctx->P.k, query_kmers,
@@ -211,13 +218,19 @@ static bool query_offsets_on_device(uint64_t n_bytes, uint32_t n_queries) {
     return n_queries && n_bytes >= (1u << 20) && n_bytes <= (uint64_t)NA_MAX_BLOCKS * NA_BLOCK_BYTES;
 }
 
-// Offsets, k-mer counts and cleared counters of the n_bytes uploaded to
-// ctx->q_seq; k-mer counts go to ctx->q_kmers.
-static int query_prepare_uploaded(ggcat_gpu_ctx* ctx, uint64_t n_bytes, uint32_t n_queries, uint32_t nc) {
-    ENSURE(ctx->q_kmers, (size_t)n_queries * 8);
+// The two steps for the n_bytes uploaded to ctx->q_seq; k-mer counts go to
+// ctx->q_kmers.  Room for the results is made between them: a count that the
+// bytes do not hold is refused before anything of its size is allocated.
+static int query_check_uploaded(ggcat_gpu_ctx* ctx, uint64_t n_bytes, uint32_t n_queries) {
     ENSURE(ctx->q_blocks, 256 + (n_bytes / NA_BLOCK_BYTES + 1) * 4);
     uint32_t* header = P_<uint32_t>(ctx->q_blocks);
     hipLaunchKernelGGL(na_clear_kernel, dim3(1), dim3(64), 0, ctx->stream, header);
+    return query_check(ctx, P_<uint8_t>(ctx->q_seq), n_bytes, n_queries, header, header + 64);
+}
+
+static int query_prepare_uploaded(ggcat_gpu_ctx* ctx, uint64_t n_bytes, uint32_t n_queries, uint32_t nc) {
+    ENSURE(ctx->q_kmers, (size_t)n_queries * 8);
+    uint32_t* header = P_<uint32_t>(ctx->q_blocks);
     return query_prepare(ctx, P_<uint8_t>(ctx->q_seq), n_bytes, n_queries, header, header + 64, P_<uint64_t>(ctx->q_off),
                          P_<uint64_t>(ctx->q_kmers), P_<uint64_t>(ctx->q_matched), P_<uint32_t>(ctx->q_counts), nc);
 }
@@ -246,8 +259,10 @@ extern "C" int ggcat_gpu_query_device_noalloc(ggcat_gpu_ctx* ctx, const uint8_t*
     hipLaunchKernelGGL(na_clear_kernel, dim3(1), dim3(64), 0, ctx->stream, header);
     HIPCHK(hipGetLastError());
     if (n_queries == 0 && n_bytes == 0) return GGCAT_GPU_OK;
-    const int r = query_prepare(ctx, d_queries, n_bytes, n_queries, header, block_nl, off, d_query_kmers, d_matched,
-                                d_color_counts, nc);
+    int r = query_check(ctx, d_queries, n_bytes, n_queries, header, block_nl);
+    if (r == GGCAT_GPU_OK)
+        r = query_prepare(ctx, d_queries, n_bytes, n_queries, header, block_nl, off, d_query_kmers, d_matched,
+                          d_color_counts, nc);
     if (r != GGCAT_GPU_OK) return r;
     QueryArgs Q = query_args(ctx);
     Q.seq = d_queries;
