@@ -239,6 +239,7 @@ u128_t mk128(uint64_t hi, uint64_t lo) { return ((u128_t)hi << 64) | lo; }
 
 // Colored merges keep one bit per color in each table entry.
 const uint32_t MAX_COLORS = 1024;
+static_assert(MAX_COLORS / 32 <= 64, "a lane of fix_join_kernel per color word");
 
 // Device-wide exclusive scan counts[0..n) -> off[0..n].
 int device_scan(ggcat_gpu_ctx* ctx, const uint32_t* counts, uint64_t* off, uint32_t n) {
@@ -1762,7 +1763,7 @@ int ggcat_gpu_kmers_merge(ggcat_gpu_ctx* ctx) {
                                P_<uint64_t>(ctx->chunk_off), used_chunks, M.out_key, key_words, M.out_val, M.out_sub,
                                M.out_colors, W);
             if (join)
-                hipLaunchKernelGGL(fix_join_kernel, dim3(((uint32_t)n_fix + 255) / 256), dim3(256), 0, ctx->stream,
+                hipLaunchKernelGGL(fix_join_kernel, dim3(((uint32_t)n_fix + 3) / 4), dim3(256), 0, ctx->stream,
                                    M.fix_key, M.fix_val, M.fix_sub, M.fix_colors, (uint32_t)n_fix, key_words, W,
                                    P_<uint64_t>(ctx->chunk_off) + used_chunks, out_cap, M.out_key, M.out_val, M.out_sub,
                                    M.out_colors, cursor<unsigned long long>(ctx, CU_ADDED));
