@@ -769,6 +769,7 @@ int ggcat_gpu_bucketing(ggcat_gpu_ctx* ctx, const uint8_t* data, uint64_t n_byte
     A.error_flag = cursor<uint32_t>(ctx, CU_ERROR);
     nthash_tables(p.m, A.gtab);
     const TileGeom G = tile_geom(T, w, p.k, p.m);
+    const uint32_t stage_lds = regs16 ? std::max(G.bytes, STAGE_W16_LDS) : G.bytes;
     ENSURE(ctx->defer, std::max<uint64_t>(n_tiles, 1) * 24);
     A.spill_cursor = cursor<unsigned long long>(ctx, CU_SPILL);
     A.defer = P_<uint64_t>(ctx->defer);
@@ -798,7 +799,7 @@ int ggcat_gpu_bucketing(ggcat_gpu_ctx* ctx, const uint8_t* data, uint64_t n_byte
         hipLaunchKernelGGL(fill32_kernel, dim3(256), dim3(256), 0, ctx->stream, A.seg_bits, 0u, (uint64_t)seg_words);
         hipLaunchKernelGGL(bucket_reset_kernel, dim3(1), dim3(64), 0, ctx->stream, A);
         if (n_tiles) {
-            hipLaunchKernelGGL(stage_kernel, dim3((uint32_t)n_tiles), dim3(64), G.bytes, ctx->stream, A);
+            hipLaunchKernelGGL(stage_kernel, dim3((uint32_t)n_tiles), dim3(64), stage_lds, ctx->stream, A);
             hipLaunchKernelGGL(bucket_defer_kernel, dim3(small_grid), dim3(256), 0, ctx->stream, A);
         }
         hipLaunchKernelGGL(unit_split_kernel, dim3(std::min<uint32_t>((n_units + 255) / 256, 4096)), dim3(256), 0,
@@ -850,7 +851,7 @@ int ggcat_gpu_bucketing(ggcat_gpu_ctx* ctx, const uint8_t* data, uint64_t n_byte
             if (safe > tiles_done) {
                 A.tile0 = tiles_done;
                 const dim3 grid((uint32_t)(safe - tiles_done));
-                hipLaunchKernelGGL(stage_kernel, grid, dim3(64), G.bytes, ctx->stream, A);
+                hipLaunchKernelGGL(stage_kernel, grid, dim3(64), stage_lds, ctx->stream, A);
                 HIPCHK(hipGetLastError());
                 tiles_done = safe;
             }

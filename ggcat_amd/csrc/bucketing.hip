@@ -123,6 +123,16 @@ __host__ __device__ inline uint32_t tile_block(uint32_t w) { return w >= 16 ? 16
 // a lane for k <= 47.
 __host__ __device__ inline bool tile_w16(uint32_t w, uint32_t k) { return w == 16 && k <= 47; }
 
+// LDS of a workgroup of that variant, with the kernel's own 2064 bytes 9
+// allocation units of 1280: a CU holds 14 wavefronts where its tile would allow
+// 16.  Where buffers lie in memory decides how many wavefronts may wait in the
+// record part before its rate drops, and it changes with what was allocated
+// before: staging pass of 1 Gbase, in a fresh process and after larger builds,
+// with 16 wavefronts 5.5 and 9.0 ms, with 14 5.5 and 5.5 to 8.4, with 12 6.0 and
+// 5.5; of 4 Gbases 22.3 and 35, 22.4 and 22 to 28, 24.6 and 22.2.
+constexpr uint32_t STAGE_W16_LDS = 9 * 1280 - 2064;
+static_assert(160 * 1024 / (STAGE_W16_LDS + 2064) == 14, "workgroups per CU");
+
 // LDS layout of one tile (host and device agree through this struct).
 struct TileGeom {
     uint32_t NW, NB;
@@ -289,10 +299,11 @@ GG_DEV uint64_t bits64(const uint32_t* a, int64_t r) {
 // combination of the two (van Herk / Gil-Werman in registers).  The window
 // flags of phase 3 are formed in the same pass from a 64-bit slice of the
 // invalid-base bitmap and written as 16-bit pieces.
-// Bound by the record part's atomics and 16-byte stores (17 G/s each), which
-// get slower the more wavefronts wait in them at once.  With the hashes, minima
-// and flags of tile_minima (28 % fewer VALU instructions) a wavefront reaches
-// them sooner and the pass of 1.6 Gbases takes 10.2 ms instead of 9.0.
+// Bound by the record part's atomics and 16-byte stores, one of each per record
+// and all at random addresses: 20 G/s of each as long as few enough wavefronts
+// wait in them, 12 G/s once too many do, where the launch then stays
+// (see STAGE_W16_LDS).  The hashes, minima and flags of tile_minima are 28 %
+// fewer VALU instructions; with them wavefronts come sooner and more wait.
 GG_DEV void tile_minima_w16(Tile& t) {
     const TileGeom& G = t.G;
     const uint32_t lane = threadIdx.x;
