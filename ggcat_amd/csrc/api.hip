@@ -657,13 +657,28 @@ int ggcat_gpu_bucketing(ggcat_gpu_ctx* ctx, const uint8_t* data, uint64_t n_byte
     ctx->P = p;
     const uint32_t w = p.k - p.m;
     const uint32_t n_sub = ((1u << p.buckets_log) + 1) << p.second_buckets_log;
-    // physical units: about `unit_bytes` input bytes per unit (default 2000),
-    // at most 2^25 units (unit sizes then stay near unit_bytes up to ~30 GB
-    // of input, so a schedule tuned on a sample holds at full size)
+    ctx->colored = n_colors > 0;
+    ctx->color_words = 0;
+    ctx->n_color_ids = 0;
+    if (n_colors) {
+        uint32_t max_color = 0;
+        for (uint32_t i = 0; i < n_colors; i++) max_color = std::max(max_color, colors[i]);
+        if (max_color >= MAX_COLORS)
+            return fail(ctx, GGCAT_GPU_EINVAL, "color ids must be < " + std::to_string(MAX_COLORS));
+        ctx->color_words = max_color / 32 + 1;
+        ctx->n_color_ids = max_color + 1;
+    }
+    // physical units: about `unit_bytes` input bytes per unit, at most 2^25 units
+    // (unit sizes then stay near unit_bytes up to ~30 GB of input).  Default
+    // 2000, half of that for colored builds whose merge tables have fewer than
+    // 2048 entries: two-word keys, or more than two color words in an entry.
+    // Bucketing and merge with units of 2000 and 1000 bytes: 64 colors of 70 MB
+    // 3.04 and 3.14 ms; 224 of 58 MB 4.75 and 3.20; 16 of 49 MB with k = 45 4.95
+    // and 2.53, k = 63 rabin-karp128 15.4 and 11.1
+    const bool two_words = p.hash_kind == GGCAT_GPU_HASH_RK128 || p.k > 32;
     uint32_t xb = 0;
-    // (colored builds with the same units, although their LDS tables are
-    // smaller: 64 colors of 41 MB 2.54 ms against 2.74 ms with units of 1000)
-    const uint64_t unit_bytes = ctx->tune.unit_bytes ? ctx->tune.unit_bytes : 2000;
+    const uint64_t unit_bytes =
+        ctx->tune.unit_bytes ? ctx->tune.unit_bytes : n_colors && (two_words || ctx->color_words > 2) ? 1000 : 2000;
     while (xb < 10 && (n_bytes >> xb) / n_sub > unit_bytes && ((uint64_t)n_sub << (xb + 1)) <= (1u << 25)) xb++;
     const uint32_t n_units = n_sub << xb;
     // slot: meta word + inline bases for the longest unique-minimizer record (2k - m)
@@ -677,17 +692,6 @@ int ggcat_gpu_bucketing(ggcat_gpu_ctx* ctx, const uint8_t* data, uint64_t n_byte
     ctx->n_units = n_units;
     ctx->slot_words = slot_words;
     ctx->n_input = n_bytes;
-    ctx->colored = n_colors > 0;
-    ctx->color_words = 0;
-    ctx->n_color_ids = 0;
-    if (n_colors) {
-        uint32_t max_color = 0;
-        for (uint32_t i = 0; i < n_colors; i++) max_color = std::max(max_color, colors[i]);
-        if (max_color >= MAX_COLORS)
-            return fail(ctx, GGCAT_GPU_EINVAL, "color ids must be < " + std::to_string(MAX_COLORS));
-        ctx->color_words = max_color / 32 + 1;
-        ctx->n_color_ids = max_color + 1;
-    }
 
     const uint8_t* d_in = data;
     // Host input of at least two upload chunks goes through the pinned

@@ -220,7 +220,8 @@ int ggcat_gpu_solid_colors(ggcat_gpu_ctx* ctx, uint32_t* color_words, uint32_t* 
  *                     which otherwise take their records by position
  *                     (no mode changes a result)
  *   unit_bytes        bucketing: input bytes per physical unit (sub-bucket
- *                     refinement); default 2000
+ *                     refinement); default 2000, 1000 for colored builds
+ *                     with 128-bit table keys or more than 64 colors
  *   use_graphs        1: capture the bucketing staging pass (clears, stage
  *                     and deferred-record kernels) in a HIP graph per
  *                     argument set and replay it on later calls
