@@ -1566,7 +1566,7 @@ int ggcat_gpu_kmers_merge(ggcat_gpu_ctx* ctx) {
     // not, among it the schedules without spread k-mers
     const bool rk = p.hash_kind == GGCAT_GPU_HASH_RK128;
     int mode = 0;
-    if (M.dedup && ctx->tune.no_dedup != 2 && p.k < 64 && !(rk && W))
+    if (M.dedup && (ctx->tune.no_dedup != 2 || rk) && p.k < 64 && !(rk && W))
         mode = W    ? (p.k <= 32 ? 6 : 7)
                : rk ? (p.k <= 32 ? 3 : 5)
                     : (p.k > 32 ? 4 : ctx->slot_words == 4 ? 1 : 2);

@@ -210,11 +210,10 @@ int ggcat_gpu_solid_colors(ggcat_gpu_ctx* ctx, uint32_t* color_words, uint32_t* 
  *                     every k-mer is distinct; lower values trade overflow
  *                     redos for smaller tables)
  *   no_dedup          1: insert every record's k-mers even when identical
- *                     records could be counted once; 2: count identical
- *                     records once but let one thread roll each distinct
- *                     record's k-mers (the mode of 128-bit keys) instead of
- *                     spreading single k-mer positions over the threads;
- *                     3: hash the records of every work item, also of those
+ *                     records could be counted once; 2: seq-hash: count
+ *                     identical records once but let one thread roll each
+ *                     distinct record's k-mers instead of spreading them
+ *                     over the threads; 3: hash the records of every work item, also of those
  *                     whose units the bucketing already deduplicated (no
  *                     unit above the deduplication's 1024-record limit),
  *                     which otherwise take their records by position
