@@ -294,11 +294,14 @@ def serve_measurement(ctx, rate_hz: float, n_requests: int) -> dict:
 
 
 def shape_sample(config: int, scale: float, full_bytes: int, cap: int) -> tuple[np.ndarray, str]:
-    """A read set of the same configuration with its genome scaled so that it
-    holds about `cap` bytes: coverage, read length, error rate and repeat
-    content as at full size, so work items (and the items that need
-    partitioned passes) look like the full-size ones."""
-    f = min(1.0, cap / max(full_bytes, 1))
+    """A read set of the same configuration with its genome scaled to at most
+    `cap` bytes, by a power of two so that its units are as large as the
+    full input's: coverage, read length, error rate and repeat content as at
+    full size, so work items (and the items that need partitioned passes) look
+    like the full-size ones."""
+    from ggcat_amd.autotune import sample_fraction
+
+    f = sample_fraction(full_bytes, cap)
     s = make_workload(config, scale * f)
     return s.data, s.name
 
@@ -365,7 +368,7 @@ def measure(ctx, wl, steps: int, warmup: int, tune: bool, check: bool, threads: 
         from ggcat_amd.autotune import autotune
 
         t = time.perf_counter()
-        tuning = autotune(ctx, sample, params, colored=False)
+        tuning = autotune(ctx, sample, params, colored=False, full_bytes=nbytes)
         tuning["sample"] = sample_name
         log(f"[bench] autotune: {tuning['tried']} schedules on {cut} bytes in {time.perf_counter() - t:.1f} s -> "
             f"{tuning['schedule']}")
@@ -476,7 +479,7 @@ def main() -> None:
         log("[bench] calibration copy (copy16_kernel): 1073741824 bytes read, 1073741824 bytes written")
     threads = min(os.cpu_count() or 1, 64)
     # the schedule is tuned and gated on the same configuration with its genome
-    # scaled to a 256 MiB read set (same coverage)
+    # scaled to a read set of at most 256 MiB (same coverage)
     sample, sample_name = shape_sample(a.config, a.scale, wl.data.size, 256 << 20)
     out = measure(ctx, wl, a.steps, a.warmup, not a.no_autotune, not a.no_check, threads, a.scale,
                   sample=sample, sample_name=sample_name, schedule=json.loads(a.schedule) if a.schedule else None,

@@ -43,14 +43,39 @@ class Schedule:
                        rec_cap=self.rec_cap, unit_cap=self.unit_cap, merge_threads=self.merge_threads)
 
 
+def unit_size(n_bytes: int, n_sub: int, unit_bytes: int) -> int:
+    """Bytes of a physical unit of an input: the sub-buckets' share of it,
+    halved until it is at most unit_bytes (ggcat_gpu_bucketing's rule), so that
+    many values of unit_bytes come to the same units."""
+    xb = 0
+    while xb < 10 and (n_bytes >> xb) // n_sub > unit_bytes and n_sub << (xb + 1) <= 1 << 25:
+        xb += 1
+    return (n_bytes >> xb) // n_sub
+
+
+def sample_fraction(full_bytes: int, cap: int) -> float:
+    """The share of an input of full_bytes that a sample of at most cap bytes
+    should hold: a power of two, which gives the same unit sizes."""
+    j = 0
+    while full_bytes / 2**j > cap:
+        j += 1
+    return 1 / 2**j
+
+
+def default_item_occ(k: int, lds: int) -> int:
+    """Occurrences per work item that the merge takes by default with a table of
+    lds entries: half of it, three quarters with two-word keys."""
+    return lds // 4 * 3 if 32 < k < 64 else lds // 2
+
+
 def default_grid(k: int) -> list[Schedule]:
     """Unit size x record-table size x LDS table size: the knobs whose best
     value depends on the input (coverage, error rate, k); the others are
-    fixed at values that measured best on every configuration tried.  A sample
-    has few enough units for their counters and open lines to stay in cache,
-    whatever their size; a full input does not (4 Gbases, k = 31: staging 33.1
-    ms with units of 1000 bytes, 22.7 with 2000), so smaller units are tried
-    for k > 32 only, whose records are fewer."""
+    fixed at values that measured best on every configuration tried.  Units
+    below 2000 bytes are tried for k > 32 only: their counters and open lines
+    stay in cache on a sample and do not on a large input (4 Gbases, k = 31:
+    staging 33.1 ms with units of 956 bytes, 22.7 with 1913), and it is k <= 32
+    whose records are many."""
     logs = (11,) if k <= 32 else (10,)
     sizes = (2000, 3000) if k <= 32 else (1400, 2000, 3000)
     out = []
@@ -78,7 +103,7 @@ def load_grid(best: Schedule, k: int) -> list[Schedule]:
         s.no_dedup = 2
         out.append(s)
     for pct, occ in itertools.product((100, 200, 400), (lds // 2, lds, 2 * lds)):
-        if (pct, occ) == (best.table_pct or 200, best.item_occ or lds // 2):
+        if (pct, occ) == (best.table_pct or 200, best.item_occ or default_item_occ(k, lds)):
             continue
         s = Schedule(**asdict(best))
         s.table_pct, s.item_occ = pct, occ
@@ -102,8 +127,12 @@ def _digest(ctx) -> tuple:
 
 def autotune(ctx, sample: np.ndarray, params: Params, grid: list[Schedule] | None = None, repeats: int = 3,
              cache_path: str | None = None, colored: bool = False, bucket_logs: tuple[int, ...] = (),
-             min_gain: float = 0.01) -> dict:
-    """Returns {"schedule": Schedule fields, "ms": best bucketing+merge ms on
+             min_gain: float = 0.01, full_bytes: int | None = None) -> dict:
+    """Times schedules on `sample`, for inputs of full_bytes (the sample's own
+    size when not given): each runs with the unit size nearest to the one it
+    comes to on the full input, since a table that suits units of 1000 bytes
+    may split most items of units of 2000; schedules that come to the same
+    units there are tried once.  Returns {"schedule": Schedule fields, "ms": best bucketing+merge ms on
     the sample, "tried": n, "buckets_log": recommended b}; applies the best
     schedule to ctx.  A schedule is timed by the device (the bucketing's
     kernels and the merge call between its stream events, the lowest of
@@ -119,6 +148,28 @@ def autotune(ctx, sample: np.ndarray, params: Params, grid: list[Schedule] | Non
     two_stage = grid is None
     grid = grid or default_grid(params.k)
     sample = np.ascontiguousarray(sample, np.uint8)
+    full = full_bytes or sample.size
+
+    def n_sub(b):
+        return ((1 << b) + 1) << params.second_buckets_log
+
+    def distinct(schedules):
+        """The first of the schedules that differ in unit_bytes only and come to
+        the same units on the full input."""
+        out = {}
+        for s in schedules:
+            unit = unit_size(full, n_sub(params.buckets_log), s.unit_bytes) if s.unit_bytes else 0
+            out.setdefault((unit, *(v for f, v in asdict(s).items() if f != "unit_bytes")), s)
+        return list(out.values())
+
+    def on_sample(s, b=params.buckets_log):
+        """The schedule with the sample's unit size nearest to the full input's."""
+        sizes = {(sample.size >> x) // n_sub(b) for x in range(11)} - {0}
+        if not s.unit_bytes or not sizes:
+            return s
+        want = max(unit_size(full, n_sub(b), s.unit_bytes), 1)
+        return Schedule(**dict(asdict(s), unit_bytes=min(sizes, key=lambda u: abs(np.log(u / want)))))
+
     ptr, n = ctx.upload(sample)
     ref = None
     best = None
@@ -126,7 +177,7 @@ def autotune(ctx, sample: np.ndarray, params: Params, grid: list[Schedule] | Non
 
     def run(sch):
         nonlocal ref, best, tried
-        sch.apply(ctx)
+        on_sample(sch).apply(ctx)
         ts = []
         for _ in range(repeats):
             ctx.bucketing(None, params, device_ptr=ptr, n_bytes=n)
@@ -148,7 +199,7 @@ def autotune(ctx, sample: np.ndarray, params: Params, grid: list[Schedule] | Non
             best = (ms, sch)
 
     try:
-        for sch in grid:
+        for sch in distinct(grid):
             run(sch)
         if two_stage:
             for sch in load_grid(best[1], params.k):
@@ -157,7 +208,7 @@ def autotune(ctx, sample: np.ndarray, params: Params, grid: list[Schedule] | Non
         for b in bucket_logs:
             p2 = Params(params.k, params.m, b, params.second_buckets_log, params.forward_only, params.hash_kind,
                         params.min_multiplicity)
-            best[1].apply(ctx)
+            on_sample(best[1], b).apply(ctx)
             ctx.bucketing(None, p2, device_ptr=ptr, n_bytes=n)
             ctx.kmers_merge()
             tm = ctx.timings()
