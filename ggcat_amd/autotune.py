@@ -13,7 +13,7 @@ from __future__ import annotations
 import itertools
 import json
 import os
-from dataclasses import asdict, dataclass
+from dataclasses import asdict, dataclass, replace
 
 import numpy as np
 
@@ -43,14 +43,35 @@ class Schedule:
                        rec_cap=self.rec_cap, unit_cap=self.unit_cap, merge_threads=self.merge_threads)
 
 
-def unit_size(n_bytes: int, n_sub: int, unit_bytes: int) -> int:
-    """Bytes of a physical unit of an input: the sub-buckets' share of it,
-    halved until it is at most unit_bytes (ggcat_gpu_bucketing's rule), so that
-    many values of unit_bytes come to the same units."""
+def unit_log(n_bytes: int, n_sub: int, unit_bytes: int) -> int:
+    """log2 of the physical units per sub-bucket: the sub-bucket's share of the
+    input is halved until it is at most unit_bytes (ggcat_gpu_bucketing's rule)."""
     xb = 0
     while xb < 10 and (n_bytes >> xb) // n_sub > unit_bytes and n_sub << (xb + 1) <= 1 << 25:
         xb += 1
-    return (n_bytes >> xb) // n_sub
+    return xb
+
+
+def unit_size(n_bytes: int, n_sub: int, unit_bytes: int) -> int:
+    """Bytes of a physical unit of an input; many values of unit_bytes come to
+    the same units."""
+    return (n_bytes >> unit_log(n_bytes, n_sub, unit_bytes)) // n_sub
+
+
+def n_sub(params: Params) -> int:
+    return ((1 << params.buckets_log) + 1) << params.second_buckets_log
+
+
+def sample_params(params: Params, full_bytes: int, sample_bytes: int) -> Params:
+    """The parameters with fewer sub-buckets, as the sample is smaller, so that
+    its sub-buckets have as many units of the same size as the full input's: a
+    work item is a run of units of one sub-bucket, and with too few of them
+    large items would not fill up on the sample as they do on the full input."""
+    less = max(0, round(np.log2(full_bytes / max(sample_bytes, 1))))
+    s = min(less, params.second_buckets_log)
+    b = min(less - s, params.buckets_log - 1)
+    return Params(params.k, params.m, params.buckets_log - b, params.second_buckets_log - s, params.forward_only,
+                  params.hash_kind, params.min_multiplicity)
 
 
 def sample_fraction(full_bytes: int, cap: int) -> float:
@@ -127,18 +148,20 @@ def _digest(ctx) -> tuple:
 
 def autotune(ctx, sample: np.ndarray, params: Params, grid: list[Schedule] | None = None, repeats: int = 3,
              cache_path: str | None = None, colored: bool = False, bucket_logs: tuple[int, ...] = (),
-             min_gain: float = 0.01, full_bytes: int | None = None) -> dict:
+             min_gain: float = 0.02, full_bytes: int | None = None) -> dict:
     """Times schedules on `sample`, for inputs of full_bytes (the sample's own
-    size when not given): each runs with the unit size nearest to the one it
-    comes to on the full input, since a table that suits units of 1000 bytes
-    may split most items of units of 2000; schedules that come to the same
-    units there are tried once.  Returns {"schedule": Schedule fields, "ms": best bucketing+merge ms on
-    the sample, "tried": n, "buckets_log": recommended b}; applies the best
-    schedule to ctx.  A schedule is timed by the device (the bucketing's
+    size when not given): each runs with the units and sub-buckets that it
+    comes to on the full input (sample_params, and the nearest unit size), since
+    a table that suits units of 1000 bytes may split most items of units of
+    2000; schedules that come to the same units there are tried once.  Returns
+    {"schedule": Schedule fields, "ms": best bucketing+merge ms on the sample,
+    "tried": n, "buckets_log": recommended b}; applies the best schedule to
+    ctx.  A schedule is timed by the device (the bucketing's
     kernels and the merge call between its stream events, the lowest of
     `repeats` runs), so host-side call overheads, which do not grow with the
     input, do not decide between schedules on a small sample; a schedule
-    must be at least `min_gain` faster than the best so far to replace it."""
+    must be at least `min_gain` faster than the best so far to replace it (a
+    schedule's time on a 250 MB sample differs by 2 % between runs)."""
     key = f"k{params.k}-m{params.m}-h{params.hash_kind}-c{int(colored)}"
     if cache_path and os.path.exists(cache_path):
         cached = json.load(open(cache_path)).get(key)
@@ -150,25 +173,28 @@ def autotune(ctx, sample: np.ndarray, params: Params, grid: list[Schedule] | Non
     sample = np.ascontiguousarray(sample, np.uint8)
     full = full_bytes or sample.size
 
-    def n_sub(b):
-        return ((1 << b) + 1) << params.second_buckets_log
-
     def distinct(schedules):
         """The first of the schedules that differ in unit_bytes only and come to
         the same units on the full input."""
         out = {}
         for s in schedules:
-            unit = unit_size(full, n_sub(params.buckets_log), s.unit_bytes) if s.unit_bytes else 0
+            unit = unit_size(full, n_sub(params), s.unit_bytes) if s.unit_bytes else 0
             out.setdefault((unit, *(v for f, v in asdict(s).items() if f != "unit_bytes")), s)
         return list(out.values())
 
-    def on_sample(s, b=params.buckets_log):
-        """The schedule with the sample's unit size nearest to the full input's."""
-        sizes = {(sample.size >> x) // n_sub(b) for x in range(11)} - {0}
-        if not s.unit_bytes or not sizes:
-            return s
-        want = max(unit_size(full, n_sub(b), s.unit_bytes), 1)
-        return Schedule(**dict(asdict(s), unit_bytes=min(sizes, key=lambda u: abs(np.log(u / want)))))
+    def time_on_sample(sch, p):
+        """Device milliseconds of bucketing and merge with the schedule for p,
+        with the sample's unit size nearest to the full input's."""
+        q = sample_params(p, full, sample.size)
+        sizes = {(sample.size >> x) // n_sub(q) for x in range(11)} - {0}
+        if sch.unit_bytes and sizes:
+            want = max(unit_size(full, n_sub(p), sch.unit_bytes), 1)
+            sch = replace(sch, unit_bytes=min(sizes, key=lambda u: abs(np.log(u / want))))
+        sch.apply(ctx)
+        ctx.bucketing(None, q, device_ptr=ptr, n_bytes=n)
+        ctx.kmers_merge()
+        tm = ctx.timings()
+        return float(tm[5] + tm[6])
 
     ptr, n = ctx.upload(sample)
     ref = None
@@ -177,13 +203,7 @@ def autotune(ctx, sample: np.ndarray, params: Params, grid: list[Schedule] | Non
 
     def run(sch):
         nonlocal ref, best, tried
-        on_sample(sch).apply(ctx)
-        ts = []
-        for _ in range(repeats):
-            ctx.bucketing(None, params, device_ptr=ptr, n_bytes=n)
-            ctx.kmers_merge()
-            tm = ctx.timings()
-            ts.append(float(tm[5] + tm[6]))
+        ts = [time_on_sample(sch, params) for _ in range(repeats)]
         d = _digest(ctx)
         if ref is None:
             ref = d
@@ -208,11 +228,7 @@ def autotune(ctx, sample: np.ndarray, params: Params, grid: list[Schedule] | Non
         for b in bucket_logs:
             p2 = Params(params.k, params.m, b, params.second_buckets_log, params.forward_only, params.hash_kind,
                         params.min_multiplicity)
-            on_sample(best[1], b).apply(ctx)
-            ctx.bucketing(None, p2, device_ptr=ptr, n_bytes=n)
-            ctx.kmers_merge()
-            tm = ctx.timings()
-            ms = float(tm[5] + tm[6])
+            ms = time_on_sample(best[1], p2)
             if ms < best[0]:
                 rec_b = b
     finally:
