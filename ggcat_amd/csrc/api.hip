@@ -282,14 +282,16 @@ int table_build(ggcat_gpu_ctx* ctx, uint64_t n, DevBuf& slots, DevBuf& count, Km
     const uint64_t slot_words = (uint64_t)T.nb * TAB_BUCKET * T.key_words * 4;  // 32-bit
     ENSURE(slots, slot_words * 4);
     T.slots = P_<ulonglong2>(slots);
-    if (const uint32_t shift = part_shift(n, T.nb, T.key_words)) {
+    uint32_t shift = part_shift(n, T.nb, T.key_words);
+    // gathered entries and overflow list: in the bucketing's unit regions, which
+    // nothing reads once the records are compacted; where those are too small
+    // and there is no room for more, the general build does without
+    if (shift && ensure(ctx, ctx->stage_slots, n * 20) != GGCAT_GPU_OK) shift = 0;
+    if (shift) {
         const uint32_t n_part = ((T.nb - 1) >> shift) + 1;
         // per partition: entries, reserved entries; then the overflow's count and list
         ENSURE(count, ((size_t)2 * n_part + 2) * 4);
         ENSURE(ctx->idx_off, ((size_t)n_part + 1) * 8);
-        // gathered entries and overflow list: in the bucketing's unit regions,
-        // which nothing reads once the records are compacted
-        ENSURE(ctx->stage_slots, n * 20);
         uint32_t* counts = P_<uint32_t>(count);
         uint64_t* off = P_<uint64_t>(ctx->idx_off);
         const uint64_t* key = P_<uint64_t>(ctx->out_key);

@@ -335,8 +335,11 @@ extern "C" int ggcat_gpu_query_graph(ggcat_gpu_ctx* ctx, const char* input_graph
     ctx->P.hash_kind = hash_kind;
     ctx->have_solid = true;
     ctx->have_values = false;
+    const size_t regions = ctx->stage_slots.cap;
     int r = ggcat_gpu_index_build(ctx);
     if (r != GGCAT_GPU_OK) return r;
+    // room that the index build gathered its entries in and no bucketing asked for
+    if (ctx->stage_slots.cap > regions) free_buf(ctx->stage_slots);
     gg_host::ReadResult Q;
     if (!gg_host::read_files({std::string(input_query)}, k, false, Q)) return fail(ctx, GGCAT_GPU_EINVAL, Q.error);
     const uint32_t nq = (uint32_t)Q.records;

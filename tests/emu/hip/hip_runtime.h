@@ -8,6 +8,7 @@
 #include <barrier>
 #include <chrono>
 #include <cstdint>
+#include <cstdio>
 #include <cstdlib>
 #include <cstring>
 #include <functional>
@@ -199,7 +200,16 @@ inline hipError_t hipEventElapsedTime(float* ms, hipEvent_t a, hipEvent_t b) {
     *ms = std::chrono::duration<float, std::milli>(b->t - a->t).count();
     return hipSuccess;
 }
-inline hipError_t hipMalloc(void** p, size_t n) { *p = std::calloc(1, n + 64); return *p ? hipSuccess : 1; }
+// allocations of lo to hi - 1 bytes fail while GGCAT_EMU_FAIL_BYTES is "lo-hi"
+inline bool emu_alloc_fails(size_t n) {
+    const char* e = std::getenv("GGCAT_EMU_FAIL_BYTES");
+    unsigned long long lo, hi;
+    return e && std::sscanf(e, "%llu-%llu", &lo, &hi) == 2 && n >= lo && n < hi;
+}
+inline hipError_t hipMalloc(void** p, size_t n) {
+    *p = emu_alloc_fails(n) ? nullptr : std::calloc(1, n + 64);
+    return *p ? hipSuccess : 1;
+}
 template <class T>
 inline hipError_t hipMalloc(T** p, size_t n) { return hipMalloc(reinterpret_cast<void**>(p), n); }
 constexpr unsigned hipHostMallocDefault = 0;
