@@ -108,7 +108,7 @@ struct ggcat_gpu_ctx {
     DevBuf q_seq, q_off, q_matched, q_counts, q_kmers, q_blocks;
     struct Server* server = nullptr;
     // unitig chains
-    DevBuf u_nb, u_ext, u_link, u_seg, u_head, u_uhead, u_ubytes, u_uoff, u_seq, u_sub, u_flags, u_visited, u_rest,
+    DevBuf u_nb, u_ext, u_link, u_seg, u_head, u_ubytes, u_uoff, u_seq, u_sub, u_flags, u_visited, u_rest,
         u_rest_n, u_totals, u_rep, u_tab;
     bool have_unitigs = false;
     bool u_joined = false;
@@ -612,7 +612,7 @@ void ggcat_gpu_destroy(ggcat_gpu_ctx* ctx) {
                       &ctx->fix_val, &ctx->fix_sub, &ctx->out_colors, &ctx->fix_colors,
                       &ctx->idx_slots, &ctx->idx_count, &ctx->idx_off,
                       &ctx->q_seq, &ctx->q_off, &ctx->q_matched, &ctx->q_counts, &ctx->q_kmers, &ctx->q_blocks,
-                      &ctx->u_nb, &ctx->u_ext, &ctx->u_link, &ctx->u_seg, &ctx->u_head, &ctx->u_uhead,
+                      &ctx->u_nb, &ctx->u_ext, &ctx->u_link, &ctx->u_seg, &ctx->u_head,
                       &ctx->u_ubytes, &ctx->u_uoff, &ctx->u_totals, &ctx->u_seq, &ctx->u_sub, &ctx->u_flags, &ctx->u_visited, &ctx->u_rest,
                       &ctx->u_rest_n, &ctx->u_rep, &ctx->u_tab, &ctx->u_path, &ctx->stage_slots, &ctx->stage_unit,
                       &ctx->stage_rank, &ctx->stage_color, &ctx->defer, &ctx->spill_slots, &ctx->spill_color, &ctx->raw, &ctx->p_stats,
@@ -2540,7 +2540,6 @@ static int build_unitigs(ggcat_gpu_ctx* ctx, bool joined, uint64_t* n_unitigs, u
     const uint64_t n_seg = 2 * ((n_pos + SPLIT - 1) / SPLIT);
     ENSURE(ctx->u_seg, n_seg * 8 + 8);
     ENSURE(ctx->u_head, ne * 8 + 8);
-    ENSURE(ctx->u_uhead, n_pos * 4 + 8);
     ENSURE(ctx->u_ubytes, n_pos * 4 + 8);
     ENSURE(ctx->u_totals, 24);
     ENSURE(ctx->u_visited, n_pos + 8);
@@ -2564,7 +2563,6 @@ static int build_unitigs(ggcat_gpu_ctx* ctx, bool joined, uint64_t* n_unitigs, u
     U.seg = P_<uint64_t>(ctx->u_seg);
     U.head = P_<uint64_t>(ctx->u_head);
     U.uni_of = U.nb;  // the neighbours are not read once the links are made
-    U.uni_head = P_<uint32_t>(ctx->u_uhead);
     U.uni_bytes = P_<uint32_t>(ctx->u_ubytes);
     U.totals = P_<unsigned long long>(ctx->u_totals);
     U.visited = P_<uint8_t>(ctx->u_visited);

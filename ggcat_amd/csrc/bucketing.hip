@@ -1445,29 +1445,4 @@ __global__ __launch_bounds__(1024) void scan_apply_kernel(const uint32_t* counts
     if (blockIdx.x == nb - 1 && threadIdx.x == 0) off[n] = partial[nb];
 }
 
-// Exclusive prefix sum of counts -> offsets (n+1 entries), one workgroup.
-__global__ __launch_bounds__(1024) void scan_kernel(const uint32_t* counts, uint64_t* off, uint32_t n) {
-    __shared__ uint64_t part[1024];
-    const uint32_t tid = threadIdx.x;
-    const uint32_t per = (n + 1023) / 1024;
-    uint32_t s0 = tid * per, s1 = s0 + per;
-    if (s1 > n) s1 = n;
-    uint64_t sum = 0;
-    for (uint32_t i = s0; i < s1; i++) sum += counts[i];
-    part[tid] = sum;
-    __syncthreads();
-    for (uint32_t d = 1; d < 1024; d <<= 1) {
-        uint64_t v = (tid >= d) ? part[tid - d] : 0;
-        __syncthreads();
-        part[tid] += v;
-        __syncthreads();
-    }
-    uint64_t run = (tid == 0) ? 0 : part[tid - 1];
-    for (uint32_t i = s0; i < s1; i++) {
-        off[i] = run;
-        run += counts[i];
-    }
-    if (tid == 1023) off[n] = part[1023];
-}
-
 }  // namespace gg

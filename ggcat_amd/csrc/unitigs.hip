@@ -46,7 +46,6 @@ struct UnitigArgs {
     uint64_t* seg;  // [2 groups of SPLIT positions] rest of the path behind each splitter, see seg_pair
     uint64_t* head;  // [2 n_pos] the same for path ends (other entries unused)
     uint32_t* uni_of;  // [2 n_pos] unitig written from this end, NO_LINK when written from its other end
-    uint32_t* uni_head;  // [unitigs] the end it is written from
     uint32_t* uni_bytes;  // [unitigs]
     const uint64_t* uni_off;  // [unitigs + 1] exclusive scan of uni_bytes
     unsigned long long* totals;  // unitigs, bytes, duplicate entries (joined mode)
@@ -341,7 +340,6 @@ __global__ __launch_bounds__(256) void head_kernel(UnitigArgs A, uint64_t n_pos)
         for (uint32_t j = 0; j < 4; j++) {
             if (!len[j]) continue;
             const uint64_t e = e0 + 4 * threadIdx.x + j;
-            A.uni_head[i] = (uint32_t)e;
             A.uni_bytes[i] = len[j];
             A.uni_of[e] = i++;
         }
