@@ -59,35 +59,51 @@ def kernel_bytes(cnt: np.ndarray, key_words: int) -> dict:
     }
 
 
-# rocprofv3 FETCH_SIZE / WRITE_SIZE of one launch per kernel at full size,
-# scaled by the counters' reading for a 1 GiB copy (profiles/ holds the
-# commands and the per-kernel table)
+# rocprofv3 FETCH_SIZE / WRITE_SIZE of one pass per kernel at full size, scaled
+# by the counters' reading for a 1 GiB copy, and the schedule they were read
+# under (profiles/ holds the commands and the per-kernel table)
 TRAFFIC_FILE = os.path.join(ROOT, "profiles", "hbm_traffic_config2.json")
-TRAFFIC_KERNELS = {"bucket_stage": ("gg::bucket_stage_kernel<16>",),
+TRAFFIC_KERNELS = {"bucket_stage": ("gg::bucket_stage_kernel<0>",),
                    "unit_compact": ("gg::unit_dedup_kernel", "gg::unit_dedup_wide_kernel", "gg::unit_compact_kernel"),
-                   "merge": ("gg::merge_lds_seq64_kernel",)}
+                   "merge": ("gg::merge_lds_seq64_kernel", "gg::out_close_holes_kernel")}
 
 
-def measured_traffic(workload: str, scale: float, kernel: str):
-    """HBM bytes (GB, read + write) of one launch of `kernel` as measured by
-    the committed counter runs of the same workload, else (None, None)."""
-    if not workload.startswith("config2") or scale != 1.0 or not os.path.exists(TRAFFIC_FILE):
+def measured_traffic(wl, scale: float, kernel: str, schedule: dict | None):
+    """HBM bytes (GB, read + write) of one pass of `kernel` as measured by the
+    committed counter runs of the same workload under a schedule that launches
+    it the same way, else (None, None)."""
+    from ggcat_amd.autotune import default_item_occ, unit_size
+
+    if not wl.name.startswith("config2") or scale != 1.0 or not os.path.exists(TRAFFIC_FILE):
         return None, None
     table = json.load(open(TRAFFIC_FILE))
-    parts = [table.get(name) for name in TRAFFIC_KERNELS.get(kernel, ())]
+    n_sub = ((1 << wl.buckets_log) + 1) << wl.second_buckets_log
+
+    def launched(s: dict) -> tuple:
+        bucketing = (unit_size(wl.data.size, n_sub, s.get("unit_bytes") or 2000), s.get("unit_cap", 0))
+        if kernel != "merge":
+            return bucketing
+        lds = s.get("lds_table_log") or 11
+        # an item of at most half a table asks for more slots than a table has from 200 % on
+        return (*bucketing, lds, min(s.get("table_pct") or 200, 200), s.get("item_occ") or default_item_occ(wl.k, 1 << lds),
+                s.get("no_dedup", 0), s.get("merge_wgs_per_cu", 0), s.get("rec_cap") or 256, s.get("merge_threads") or 256)
+
+    if launched(schedule or {}) != launched(table["schedule"]):
+        return None, None
+    parts = [table["kernels"].get(name) for name in TRAFFIC_KERNELS.get(kernel, ())]
     if not parts or not all(parts):
         return None, None
     gb = sum(t["read_gb"] + t["write_gb"] for t in parts)
-    return round(gb, 3), "profiles/hbm_traffic_config2.md (rocprofv3 --pmc, GB per launch)"
+    return round(gb, 3), "profiles/hbm_traffic_config2.md (rocprofv3 --pmc, GB per pass)"
 
 
-def kernel_rooflines(kb: dict, kern_ms: dict, workload: str, scale: float) -> dict:
+def kernel_rooflines(kb: dict, kern_ms: dict, wl, scale: float, schedule: dict | None) -> dict:
     """Every timed kernel against the HBM peak: algorithmic bytes over its
     HIP-event time, and the counter-measured bytes over the same time."""
     out = {}
     for name, ms in kern_ms.items():
         alg = kb[name] / (ms * 1e-3) / 1e9
-        traffic, _ = measured_traffic(workload, scale, name)
+        traffic, _ = measured_traffic(wl, scale, name, schedule)
         out[name] = {"ms": round(float(ms), 3), "algorithmic_gb": round(kb[name] / 1e9, 3),
                      "achieved_gbs": round(alg, 1), "frac": round(alg / HBM_PEAK_GBS, 4),
                      "traffic_gb": traffic,
@@ -401,7 +417,8 @@ def measure(ctx, wl, steps: int, warmup: int, tune: bool, check: bool, threads: 
     kern_ms = {"bucket_stage": ms[0], "unit_compact": ms[2], "merge": ms[3] + ms[4]}
     dom = max(kern_ms, key=lambda x: kern_ms[x])
     achieved = kb[dom] / (kern_ms[dom] * 1e-3) / 1e9
-    traffic, traffic_src = measured_traffic(wl.name, scale, dom)
+    timed = (tuning or {}).get("schedule")
+    traffic, traffic_src = measured_traffic(wl, scale, dom, timed)
     ms_step = dt / steps * 1e3
     value = wl.bases / (dt / steps) / 1e9
     return {
@@ -425,7 +442,7 @@ def measure(ctx, wl, steps: int, warmup: int, tune: bool, check: bool, threads: 
                      "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": traffic,
                      "algorithmic_gb": round(kb[dom] / 1e9, 3), "traffic_source": traffic_src},
         "kernels_ms": {k: round(float(v), 3) for k, v in kern_ms.items()},
-        "kernels_roofline": kernel_rooflines(kb, kern_ms, wl.name, scale),
+        "kernels_roofline": kernel_rooflines(kb, kern_ms, wl, scale, timed),
         "counters": {"records": int(cnt[1]), "stored_records": int(cnt[10]), "record_bases": int(cnt[2]),
                      "kmer_occurrences": int(cnt[3]), "split_items": int(cnt[4]), "solid_entries": int(n),
                      "merge_passes": int(cnt[7])},
