@@ -125,11 +125,17 @@ __host__ __device__ inline bool tile_w16(uint32_t w, uint32_t k) { return w == 1
 
 // LDS of a workgroup of that variant, with the kernel's own 2064 bytes 9
 // allocation units of 1280: a CU holds 14 wavefronts where its tile would allow
-// 16.  Where buffers lie in memory decides how many wavefronts may wait in the
-// record part before its rate drops, and it changes with what was allocated
-// before: staging pass of 1 Gbase, in a fresh process and after larger builds,
-// with 16 wavefronts 5.5 and 9.0 ms, with 14 5.5 and 5.5 to 8.4, with 12 6.0 and
-// 5.5; of 4 Gbases 22.3 and 35, 22.4 and 22 to 28, 24.6 and 22.2.
+// 16.  The records' atomics and stores run at 20 G/s each while few enough
+// wavefronts wait in them and at 12 G/s once too many do (the L2s' write requests
+// to memory then stall, 69 M stall cycles against 1 M), and how many that is
+// depends on where the buffers lie in memory, which changes with what was
+// allocated before.  Cheaper hashes or input bytes bring wavefronts there sooner,
+// so neither helps.  Staging pass where few are enough and where many are:
+//   bytes four at a time, 16 wavefronts: 1 Gbase 9.0 and 5.5 ms, 4 Gbases 35 and 22.2
+//   bytes four at a time, 14             5.4 to 8.5 and 5.55     22 to 29 and 22.4
+//   byte by byte, 16                     6.3 to 8.8 and 5.4      23 to 30 and 22.0
+//   byte by byte, 14 (taken)             5.3 to 5.6 and 5.75     21.9 to 22.6 and 23.3
+//   bytes four at a time, 12             5.5 and 6.0             22.3 and 24.6
 constexpr uint32_t STAGE_W16_LDS = 9 * 1280 - 2064;
 static_assert(160 * 1024 / (STAGE_W16_LDS + 2064) == 14, "workgroups per CU");
 
@@ -264,8 +270,19 @@ GG_DEV void tile_compute(Tile& t) {
         uint32_t packed = 0, invm = 0;
         if (a >= 0 && a + 16 <= (int64_t)A.n) {
             uint4 v = *reinterpret_cast<const uint4*>(A.seq + a);
-            packed = codes4(v.x) | codes4(v.y) << 8 | codes4(v.z) << 16 | codes4(v.w) << 24;
-            invm = not_acgt4(v.x) | not_acgt4(v.y) << 4 | not_acgt4(v.z) << 8 | not_acgt4(v.w) << 12;
+            if constexpr (B == 0) {
+                // byte by byte: its VALU work is what this variant can spare (see STAGE_W16_LDS)
+                const uint32_t wds[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+                for (uint32_t idx = 0; idx < 16; idx++) {
+                    const uint8_t ch = (uint8_t)(wds[idx >> 2] >> (8 * (idx & 3)));
+                    packed |= (uint32_t)((ch >> 1) & 3) << (2 * idx);
+                    invm |= (is_acgt(ch) ? 0u : 1u) << idx;
+                }
+            } else {
+                packed = codes4(v.x) | codes4(v.y) << 8 | codes4(v.z) << 16 | codes4(v.w) << 24;
+                invm = not_acgt4(v.x) | not_acgt4(v.y) << 4 | not_acgt4(v.z) << 8 | not_acgt4(v.w) << 12;
+            }
         } else {
             for (uint32_t idx = 0; idx < 16; idx++) {
                 int64_t p = a + idx;
@@ -300,10 +317,9 @@ GG_DEV uint64_t bits64(const uint32_t* a, int64_t r) {
 // flags of phase 3 are formed in the same pass from a 64-bit slice of the
 // invalid-base bitmap and written as 16-bit pieces.
 // Bound by the record part's atomics and 16-byte stores, one of each per record
-// and all at random addresses: 20 G/s of each as long as few enough wavefronts
-// wait in them, 12 G/s once too many do, where the launch then stays
-// (see STAGE_W16_LDS).  The hashes, minima and flags of tile_minima are 28 %
-// fewer VALU instructions; with them wavefronts come sooner and more wait.
+// and all at random addresses: 20 G/s of each, as long as wavefronts do not come
+// to them sooner (see STAGE_W16_LDS).  The hashes, minima and flags of tile_minima
+// are 28 % fewer VALU instructions and would bring them sooner.
 GG_DEV void tile_minima_w16(Tile& t) {
     const TileGeom& G = t.G;
     const uint32_t lane = threadIdx.x;
