@@ -86,6 +86,8 @@ struct ggcat_gpu_ctx {
     uint32_t dd_max = 0;  // the compaction deduplicated the units of up to this many records
     bool resplit_done = false;  // the arena holds resplit buckets (ggcat_gpu_resplit_outliers)
     uint64_t n_spill = 0;  // records of the last bucketing past their unit's region
+    bool stage_sparse = false;  // staging pass, w = 16: 14 wavefronts per CU (see STAGE_W16_LDS)
+    const void* stage_at = nullptr;  // the unit regions for which that was found
     uint32_t n_passes = 0;  // kernel passes of the last merge
     DevBuf copy_mult, copy_flags;  // multiplicities and flags on their way to the host
     bool colored = false;
@@ -98,6 +100,7 @@ struct ggcat_gpu_ctx {
         gg::BucketArgs args;  // every kernel argument of the captured launches
         uint64_t seg_words;
         uint32_t n_units;
+        uint32_t stage_lds;
     } graph_a_key{};
     uint32_t n_color_ids = 0;  // largest color id + 1 of the colored build
     // query index over the solid table
@@ -775,7 +778,8 @@ int ggcat_gpu_bucketing(ggcat_gpu_ctx* ctx, const uint8_t* data, uint64_t n_byte
     A.error_flag = cursor<uint32_t>(ctx, CU_ERROR);
     nthash_tables(p.m, A.gtab);
     const TileGeom G = tile_geom(T, w, p.k, p.m);
-    const uint32_t stage_lds = regs16 ? std::max(G.bytes, STAGE_W16_LDS) : G.bytes;
+    uint32_t stage_lds = G.bytes;
+    bool judge_stage = false;  // the pass's rate says how many wavefronts per CU the next one takes
     ENSURE(ctx->defer, std::max<uint64_t>(n_tiles, 1) * 24);
     A.spill_cursor = cursor<unsigned long long>(ctx, CU_SPILL);
     A.defer = P_<uint64_t>(ctx->defer);
@@ -894,6 +898,13 @@ int ggcat_gpu_bucketing(ggcat_gpu_ctx* ctx, const uint8_t* data, uint64_t n_byte
         A.spill_color = n_colors ? P_<uint32_t>(ctx->spill_color) : nullptr;
         A.pool = P_<uint32_t>(ctx->pool);
         A.pool_cap = pool_cap;
+        // (a pass over new regions is not judged: it may be their first use)
+        judge_stage = regs16 && !chunked && ctx->stage_at == ctx->stage_slots.p;
+        if (ctx->stage_at != ctx->stage_slots.p) {
+            ctx->stage_at = ctx->stage_slots.p;
+            ctx->stage_sparse = false;
+        }
+        stage_lds = regs16 && ctx->stage_sparse ? std::max(G.bytes, STAGE_W16_LDS) : G.bytes;
         HIPCHK(hipEventRecord(ctx->ev[0], ctx->stream));
         if (attempt == 0 && chunked) {
             const int r = pass_1_chunked();
@@ -904,6 +915,7 @@ int ggcat_gpu_bucketing(ggcat_gpu_ctx* ctx, const uint8_t* data, uint64_t n_byte
             key.args = A;
             key.seg_words = seg_words;
             key.n_units = n_units;
+            key.stage_lds = stage_lds;
             if (!ctx->graph_a || memcmp(&key, &ctx->graph_a_key, sizeof key) != 0) {
                 if (ctx->graph_a) (void)hipGraphExecDestroy(ctx->graph_a);
                 ctx->graph_a = nullptr;
@@ -919,6 +931,7 @@ int ggcat_gpu_bucketing(ggcat_gpu_ctx* ctx, const uint8_t* data, uint64_t n_byte
                     return fail(ctx, GGCAT_GPU_EHIP, std::string("graph instantiate: ") + hipGetErrorString(e));
                 }
                 ctx->graph_a_key = key;
+                HIPCHK(hipEventRecord(ctx->ev[0], ctx->stream));  // the pass's time is without the capture
             }
             HIPCHK(hipGraphLaunch(ctx->graph_a, ctx->stream));
         } else {
@@ -1015,6 +1028,10 @@ int ggcat_gpu_bucketing(ggcat_gpu_ctx* ctx, const uint8_t* data, uint64_t n_byte
     float t;
     HIPCHK(hipEventElapsedTime(&t, ctx->ev[0], ctx->ev[1]));
     ctx->ms[0] = t;
+    // 17.5 G records/s lie between the rates of the two cases of STAGE_W16_LDS;
+    // short passes and inputs of few records per byte say nothing
+    if (judge_stage && ctx->n_records >= 1u << 24 && ctx->n_records > n_bytes / 12 && (double)ctx->n_records < t * 17.5e6)
+        ctx->stage_sparse = true;
     HIPCHK(hipEventElapsedTime(&t, ctx->ev[15], ctx->ev[2]));
     ctx->ms[1] = t;
     float t_dedup;

@@ -124,18 +124,20 @@ __host__ __device__ inline uint32_t tile_block(uint32_t w) { return w >= 16 ? 16
 __host__ __device__ inline bool tile_w16(uint32_t w, uint32_t k) { return w == 16 && k <= 47; }
 
 // LDS of a workgroup of that variant, with the kernel's own 2064 bytes 9
-// allocation units of 1280: a CU holds 14 wavefronts where its tile would allow
+// allocation units of 1280: a CU holds 14 wavefronts where its tile alone allows
 // 16.  The records' atomics and stores run at 20 G/s each while few enough
 // wavefronts wait in them and at 12 G/s once too many do (the L2s' write requests
 // to memory then stall, 69 M stall cycles against 1 M), and how many that is
 // depends on where the buffers lie in memory, which changes with what was
 // allocated before.  Cheaper hashes or input bytes bring wavefronts there sooner,
-// so neither helps.  Staging pass where few are enough and where many are:
+// so neither helps.  Staging pass where few are too many and where 16 are not:
 //   bytes four at a time, 16 wavefronts: 1 Gbase 9.0 and 5.5 ms, 4 Gbases 35 and 22.2
 //   bytes four at a time, 14             5.4 to 8.5 and 5.55     22 to 29 and 22.4
 //   byte by byte, 16                     6.3 to 8.8 and 5.4      23 to 30 and 22.0
-//   byte by byte, 14 (taken)             5.3 to 5.6 and 5.75     21.9 to 22.6 and 23.3
+//   byte by byte, 14                     5.3 to 5.6 and 5.75     21.9 to 22.6 and 23.5
 //   bytes four at a time, 12             5.5 and 6.0             22.3 and 24.6
+// So bytes are taken one by one, and 16 wavefronts until a pass over regions used
+// before shows too low a rate, then 14 for as long as the regions stay.
 constexpr uint32_t STAGE_W16_LDS = 9 * 1280 - 2064;
 static_assert(160 * 1024 / (STAGE_W16_LDS + 2064) == 14, "workgroups per CU");
 
