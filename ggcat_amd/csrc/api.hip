@@ -1603,8 +1603,9 @@ int ggcat_gpu_kmers_merge(ggcat_gpu_ctx* ctx) {
     // two-word keys, whose tables are half as large, so that an item's fixed
     // cost weighs more (merge of 551 M occurrences, k = 63, 9.8 ms with half,
     // 9.4 with three quarters, 9.2 with a whole table, which all-distinct
-    // k-mers would overflow; one-word keys, 1.57 G: 8.6 with half, 9.1 with
-    // three eighths)
+    // k-mers would overflow; of three quarters of one they need more than the 96
+    // probes in 1 % of the items, which are then redone in parts; one-word keys,
+    // 1.57 G: 8.6 with half, 9.1 with three eighths)
     const uint32_t item_occ =
         ctx->tune.item_occ ? ctx->tune.item_occ : mode != 0 && table_words == 2 ? M.lds_cap / 4 * 3 : M.lds_cap / 2;
     // work items whose units the compaction deduplicated skip the record hashing
@@ -1732,8 +1733,10 @@ int ggcat_gpu_kmers_merge(ggcat_gpu_ctx* ctx) {
                 uint32_t L, base, stride;
                 if (w.log_parts == 0) {
                     // up to three quarters of a table of occurrences per part: every
-                    // part reads all of the item's records, and even distinct
-                    // k-mers fit.  8.9 K items of 0.9 Gbases, k = 63: 1.57 ms
+                    // part reads all of the item's records, and distinct k-mers
+                    // fit too (but for 1 % of the parts of 1024 slots and 3 % of
+                    // those of 2048, which need more than 96 probes and are split
+                    // again).  8.9 K items of 0.9 Gbases, k = 63: 1.57 ms
                     // with half a table, 1.08; with 1.5 tables 0.70, but then
                     // inputs without repeated k-mers are split twice
                     const uint64_t per = ctx->tune.part_occ ? ctx->tune.part_occ : M.lds_cap / 4 * 3;

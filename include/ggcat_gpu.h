@@ -175,7 +175,9 @@ int ggcat_gpu_kmers_merge(ggcat_gpu_ctx* ctx);
 int ggcat_gpu_solid_info(ggcat_gpu_ctx* ctx, uint64_t* n_solid, uint32_t* key_words);
 
 /* Copy of the solid entries: keys (key_words uint64 per entry, low word
- * first), multiplicity, flags and sub-bucket.  Order is unspecified. */
+ * first), multiplicity, flags and sub-bucket (each may be NULL).  Order is
+ * unspecified.  After ggcat_gpu_query_graph the table is that graph's and has
+ * keys only: anything else, and unitigs, give GGCAT_GPU_ESTATE. */
 int ggcat_gpu_solid_copy(ggcat_gpu_ctx* ctx, uint64_t* keys, uint32_t* multiplicity, uint8_t* flags,
                          uint32_t* sub);
 
@@ -206,9 +208,11 @@ int ggcat_gpu_solid_colors(ggcat_gpu_ctx* ctx, uint32_t* color_words, uint32_t* 
  *                     default 11 for 64-bit keys, 10 for 128-bit; reduced
  *                     to fit 48 KiB with colors)
  *   table_pct         table slots per 100 occurrences of an item, rounded up
- *                     to a power of two (default 200: never overflows when
- *                     every k-mer is distinct; lower values trade overflow
- *                     redos for smaller tables)
+ *                     to a power of two, at most the LDS table (default 200;
+ *                     lower values trade overflow redos for smaller tables.
+ *                     Items of half a table of distinct k-mers do not
+ *                     overflow; 1 % of those of three quarters do and are
+ *                     redone in parts)
  *   no_dedup          1: insert every record's k-mers even when identical
  *                     records could be counted once; 2: seq-hash: count
  *                     identical records once but let one thread roll each
